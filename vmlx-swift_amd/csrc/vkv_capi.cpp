@@ -199,7 +199,7 @@ void run_attention(int dtype, int bits, int group, bool qsem, AttnArgs& a, int64
     d.kv.vc = d.kv.kc;
     // a stand-in base with the copy's alignment decides support first
     d.kv.kc.ptr = d.kv.vc.ptr = reinterpret_cast<const uint8_t*>(uintptr_t{256});
-    if (a.D == a.Dv && prefill_supported(dtype, 0, d)) {
+    if (a.D == a.Dv && prefill_supported(dtype, 0, d) && prefill_mask_fits(d, batch)) {
       d.n_parts = prefill_parts(batch, a.Hkv, a.L, a.Hq / a.Hkv, T, a.D, &d.part_tokens);
       // key windows of whole parts, each gathered to a copy of at most
       // kGatherCopyBytes (or the gather_tokens option) before its parts run
@@ -211,12 +211,14 @@ void run_attention(int dtype, int bits, int group, bool qsem, AttnArgs& a, int64
         d.part_tokens = static_cast<int32_t>(win);
         d.n_parts = static_cast<int32_t>((T + win - 1) / win);
       }
+      prefill_mask_parts(d, T, &d.part_tokens, &d.n_parts);
       const int ppw = static_cast<int>(std::max<int64_t>(1, win / d.part_tokens));
       const int64_t wtok = std::min<int64_t>(T, static_cast<int64_t>(ppw) * d.part_tokens);
       const int64_t wbytes = batch * a.Hkv * wtok * a.D * es;  // one matrix of a window
       const size_t copy_floats = static_cast<size_t>((2 * wbytes + 255) / 256 * 64);
       const size_t per = static_cast<size_t>(rows) * a.Hq * d.n_parts;
-      float* ws = workspace(st, copy_floats + (d.n_parts > 1 ? per * (a.Dv + 2) : 0), noalloc);
+      const size_t part_floats = d.n_parts > 1 ? (per * (a.Dv + 2) + 63) / 64 * 64 : 0;
+      float* ws = workspace(st, copy_floats + part_floats + prefill_mask_floats(d, batch), noalloc);
       uint8_t* kd = reinterpret_cast<uint8_t*>(ws);
       uint8_t* vd = kd + wbytes;
       const int64_t wph = wtok * a.D * es;  // copy bytes per (row, kv head)
@@ -226,6 +228,7 @@ void run_attention(int dtype, int bits, int group, bool qsem, AttnArgs& a, int64
         d.ws_o = ws + copy_floats;
         d.ws_ml = d.ws_o + per * a.Dv;
       }
+      launch_prefill_mask(d, batch, ws + copy_floats + part_floats, st);
       for (int p0 = 0; p0 < d.n_parts; p0 += ppw) {
         GatherArgs g{};
         g.kv = a.kv;
@@ -251,14 +254,19 @@ void run_attention(int dtype, int bits, int group, bool qsem, AttnArgs& a, int64
       return;
     }
   }
-  if (prefill_supported(dtype, bits, a) && !option(VKV_OPTION_GENERIC_ATTENTION)) {
+  if (prefill_supported(dtype, bits, a) && !option(VKV_OPTION_GENERIC_ATTENTION) &&
+      prefill_mask_fits(a, rows / a.L)) {
     const int64_t batch = rows / a.L;
     a.n_parts = prefill_parts(batch, a.Hkv, a.L, a.Hq / a.Hkv, a.kv.T, a.D, &a.part_tokens);
-    if (a.n_parts > 1) {
-      const size_t per = static_cast<size_t>(rows) * a.Hq * a.n_parts;
-      float* ws = workspace(st, per * (a.Dv + 2), noalloc);
+    prefill_mask_parts(a, a.kv.T, &a.part_tokens, &a.n_parts);
+    const size_t per = static_cast<size_t>(rows) * a.Hq * a.n_parts;
+    const size_t part_floats = a.n_parts > 1 ? (per * (a.Dv + 2) + 63) / 64 * 64 : 0;
+    const size_t mask_floats = prefill_mask_floats(a, batch);
+    if (part_floats + mask_floats) {
+      float* ws = workspace(st, part_floats + mask_floats, noalloc);
       a.ws_o = ws;
       a.ws_ml = ws + per * a.Dv;
+      launch_prefill_mask(a, batch, ws + part_floats, st);
     }
     launch_prefill(dtype, qsem, a, batch, st);
     return;

@@ -119,6 +119,14 @@ struct AttnArgs {
   // group); non-null merges the split partials inside the decode launch
   // (the last part of a row merges, then zeroes its counter again)
   uint32_t* counters;
+  // matrix-core prefill under a bool array mask: the mask as bits (row
+  // b * mw_b + h * mw_h + l, mw_words words each), per (row, 256 keys) whether
+  // any key is seen, and per (row block, 32-key tile) its class
+  // (launch_prefill_mask)
+  uint32_t* mw;
+  uint8_t* mrow;
+  uint8_t* mcls;
+  int64_t mw_words, mw_b, mw_h;
   // float decode only: > 0 = the launch is one workgroup of wg_parts waves
   // per (row, kv head, head group) (n_parts == wg_parts), merged in LDS
   int32_t wg_parts;
@@ -201,13 +209,19 @@ void launch_attn_combine(int dtype, const AttnArgs& a, int64_t rows, hipStream_t
 // qualifies (float, L = 1, dense, D = Dv in {64, 128, 256}, 16-byte aligned
 // rows), its token split (about 2048 waves, 64-token steps), and the launch
 // (with the merge when a.n_parts > 1).
-// Multi-query attention (L >= 2) over dense bf16 / f16 K/V, D = 128, no or
-// causal mask, on matrix cores (vkv_prefill.hip).
+// Multi-query attention (L >= 2) over dense bf16 / f16 K/V, D = 64, 128 or
+// 256, no, causal or bool array mask, on matrix cores (vkv_prefill.hip).  A
+// bool array is packed first (launch_prefill_mask, into prefill_mask_floats
+// of workspace); prefill_mask_parts bounds its parts to the kernel's tile list.
 bool prefill_supported(int dtype, int bits, const AttnArgs& a);
 int prefill_parts(int64_t batch, int Hkv, int64_t L, int rep, int64_t T, int D, int32_t* part_tokens);
 // combine = false leaves the split merge to the caller (a window of parts)
 void launch_prefill(int dtype, bool qsem, const AttnArgs& a, int64_t batch, hipStream_t st,
                     bool combine = true);
+bool prefill_mask_fits(const AttnArgs& a, int64_t batch);
+size_t prefill_mask_floats(const AttnArgs& a, int64_t batch);
+void prefill_mask_parts(const AttnArgs& a, int64_t T, int32_t* part_tokens, int32_t* n_parts);
+void launch_prefill_mask(AttnArgs& a, int64_t batch, float* ws, hipStream_t st);
 bool fdecode_supported(int dtype, int bits, bool qsem, const AttnArgs& a);
 int fdecode_parts(int64_t rows_x_heads, int64_t T, int32_t* part_tokens, int waves);
 void launch_fdecode(int dtype, const AttnArgs& a, int64_t rows, hipStream_t st);

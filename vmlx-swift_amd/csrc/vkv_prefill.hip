@@ -1,8 +1,8 @@
 // vkv_prefill.hip -- multi-query attention (L >= 2 query tokens per row:
 // chunked prefill) over dense float K/V on gfx950 matrix cores.
 //
-// Semantics: MLXFast.scaledDotProductAttention with a causal or no mask
-// (MLXFast.swift:173-218; causal = query l of L sees keys 0 .. T - L + l,
+// Semantics: MLXFast.scaledDotProductAttention with no mask, a causal or a
+// bool array mask (MLXFast.swift:173-218; causal = query l of L sees keys 0 .. T - L + l,
 // with T each row's own length when the rows are ragged: the chunk of a
 // continuous batch over a paged pool),
 // and quantizedScaledDotProductAttention (KVCache.swift:1909-1997) of the
@@ -72,6 +72,8 @@ constexpr int kStages = 4;    // K+V tiles in LDS; the open-tile loop is unrolle
 constexpr int kWaves = 8;     // two per SIMD, one workgroup per CU
 constexpr int kThreads = 64 * kWaves;
 constexpr float kTau = 8.0f;  // rescale threshold (log2)
+constexpr int kMaskChunk = 256;     // tokens a mask-packing workgroup takes
+constexpr int kMaxMaskTiles = 2048; // key tiles of one part under an array mask
 constexpr float kLog2e = 1.4426950408889634f;
 
 // Layout for head dim D (keys and values).  Every wave owns 32 query rows.
@@ -187,16 +189,108 @@ __device__ __forceinline__ float halves_max(float v) {
   return fmaxf(lo, hi);
 }
 
+// 4 bytes per lane from base + voff to LDS lds + 4 * lane, as dma16.
+__device__ __forceinline__ void dma4(const void* base, uint32_t voff, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dword %0, %2" ::"v"(voff), "s"(lds), "s"(base)
+               : "memory", "m0");
+}
+
+// 16 mask bytes (any non-zero value is true) as 16 bits, byte i in bit i.
+__device__ __forceinline__ uint32_t mask_bits16(const u32x4_t& x) {
+  uint32_t b = 0;
+#pragma unroll
+  for (int w = 0; w < 4; w++) {
+    // bit 7 of every non-zero byte, then the four gathered by one product
+    // (byte k's bit lands at 24 + k; no two partial products share a bit)
+    const uint32_t t = ((((x[w] & 0x7f7f7f7fu) + 0x7f7f7f7fu) | x[w]) >> 7) & 0x01010101u;
+    b |= (t * 0x01020408u >> 24 & 15u) << (4 * w);
+  }
+  return b;
+}
+
+// A bool array mask as one bit per (query row, key), before the attention:
+// words[row][T / 32] with the bits past the row's length clear, the class of
+// every (row block of the attention kernel, 32-key tile) -- 0: no row sees
+// any of it, 2: every row sees all of it, 1: else -- and per (row, 256 keys)
+// whether any key is seen.  The attention kernel then skips class-0 tiles,
+// runs class-2 tiles without mask work and reads one word per row and tile
+// of the others, where the bytes would be 16 loads a lane in the softmax
+// phase.  A workgroup takes the rows of one row block x 256 keys, 16 lanes a
+// row, 16 bytes a lane.  Latency bound: a [512, 1535] mask (0.8 MB) is 64
+// workgroups of two loads a wave and takes 4.7 us; one row a wave with byte
+// loads unrolled eight deep (1800 instructions, each fetched once) took 14 us.
+__global__ void __launch_bounds__(512) mask_pack_kernel(const AttnArgs a, int rep, int rows_per_wg) {
+  __shared__ uint32_t s_or[8], s_and[8];
+  const int c = blockIdx.x, rblk = blockIdx.y;
+  const int lane = threadIdx.x & 63, sub = threadIdx.x & 15;
+  const int nh = a.m_sh ? a.Hkv : 1;
+  const int zb = blockIdx.z / nh, zh = blockIdx.z - zb * nh;
+  const int T = a.kv.seq_lens ? min(a.kv.seq_lens[zb], a.kv.T) : a.kv.T;
+  // the block's positions (rows are position-major), and the heads of each
+  const int row0 = rblk * rows_per_wg, row1 = min(a.L * rep, row0 + rows_per_wg) - 1;
+  const int p0 = row0 / rep, heads = a.m_sh ? rep : 1;
+  const int items = (row1 / rep - p0 + 1) * heads;
+  if (threadIdx.x < 8) {
+    s_or[threadIdx.x] = 0;
+    s_and[threadIdx.x] = ~0u;
+  }
+  __syncthreads();
+  const int t0 = c * kMaskChunk + 16 * sub;  // this lane's 16 keys
+  const int left = T - t0;                   // keys of them that exist
+  const uint8_t* mz = static_cast<const uint8_t*>(a.mask) + zb * a.m_sb;
+#pragma unroll 2
+  for (int it = threadIdx.x >> 4; it < items; it += 32) {
+    const int dl = heads == 1 ? it : it / heads;
+    const int h = zh * rep + it - dl * heads, l = p0 + dl;
+    const uint8_t* m = mz + h * a.m_sh + l * a.m_sl;
+    uint32_t w = 0;
+    if (a.m_st == 1 && T >= 16) {
+      // a lane at the row's end reads its last 16 bytes and shifts
+      u32x4_t x;
+      __builtin_memcpy(&x, m + min(t0, T - 16), 16);
+      w = left > 0 ? mask_bits16(x) >> max(16 - left, 0) : 0;
+    } else if (left > 0) {
+      for (int k = 0; k < min(left, 16); k++) w |= (m[(t0 + k) * a.m_st] ? 1u : 0u) << k;
+    }
+    // even lanes hold 32 keys: their own 16 and the next lane's
+    w |= static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(w, 0xB1, 0xF, 0xF, false)) << 16;
+    const int64_t row = zb * a.mw_b + h * a.mw_h + l;
+    const uint64_t any = __builtin_amdgcn_ballot_w64(w != 0) >> (lane & 48) & 0xFFFF;
+    if (sub == 0) a.mrow[row * (a.mw_words / 8) + c] = any != 0;
+    if (!(sub & 1)) {
+      a.mw[row * a.mw_words + 8 * c + sub / 2] = w;
+      atomicOr(&s_or[sub / 2], w);
+      atomicAnd(&s_and[sub / 2], w);
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x < 8)
+    a.mcls[(static_cast<int64_t>(blockIdx.z) * gridDim.y + rblk) * a.mw_words + 8 * c + threadIdx.x] =
+        s_or[threadIdx.x] == 0 ? 0 : s_and[threadIdx.x] == ~0u ? 2 : 1;
+}
+
 // QSEM: the quantized-SDPA arithmetic (KVCache.swift:1909-1997): queries
 // times the scale rounded to the dtype, rounded again, instead of fp32 scores
 // times the scale; scores rounded to the dtype before the softmax.
-template <int DT, bool QSEM, int D>
+// ARR: a bool array mask, packed by mask_pack_kernel: the workgroup runs the
+// tiles some row of it sees, the wholly visible ones first (the order of the
+// keys does not matter to the online softmax), and each wave loads its rows'
+// words of a tile beside the tile.  Measured (512-token chunk on a 1024-token
+// window, 16/8 heads x 256, 1535 keys): 55 us and 4.7 us for the packing, where
+// the generic kernel took 1780 us.
+template <int DT, bool QSEM, int D, bool ARR>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 prefill_kernel(const AttnArgs a, int rep) {
   using Cfg = PfCfg<D>;
   constexpr int kChunks = Cfg::kChunks, kDBw = Cfg::kDBw, kRows = Cfg::kRows;
-  constexpr int kRowB = Cfg::kRowB, kTileB = Cfg::kTileB, kLoads = Cfg::kLoads;
+  constexpr int kRowB = Cfg::kRowB, kTileB = Cfg::kTileB;
+  constexpr int kLoads = Cfg::kLoads + (ARR ? 1 : 0);  // loads per wave per tile
+  constexpr bool HL = QSEM || ARR;  // P as hi + lo
   __shared__ __attribute__((aligned(16))) uint8_t kv[kStages][2][kTileB];  // [stage][K/V]
+  // ARR: the mask words of each wave's rows per stage, and the tiles to run
+  __shared__ uint32_t mwords[ARR ? kStages : 1][ARR ? kWaves : 1][ARR ? 64 : 1];
+  __shared__ uint16_t tlist[ARR ? kMaxMaskTiles : 1];
+  __shared__ int tcount[2];
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -233,10 +327,10 @@ prefill_kernel(const AttnArgs a, int rep) {
   // has every score at T's lowest value in the reference (where(mask, s,
   // finfo.min)), i.e. uniform weights over all of the row's keys; a
   // workgroup holding such a query scans them all
-  const bool some_none = QSEM && a.mask_mode == 1 && T - L + row0 / rep < 0;
+  bool some_none = QSEM && a.mask_mode == 1 && T - L + row0 / rep < 0;
   if (a.mask_mode == 1 && !some_none) k_end = min<int64_t>(k_end, T - L + rlast / rep + 1);
   const int64_t k_begin = static_cast<int64_t>(part) * a.part_tokens;
-  const int ntiles = k_end > k_begin ? static_cast<int>((k_end - k_begin + kTok - 1) / kTok) : 0;
+  int ntiles = k_end > k_begin ? static_cast<int>((k_end - k_begin + kTok - 1) / kTok) : 0;
   // tiles that every row of the workgroup sees whole (no mask work)
   int n_open = 0;
   if (!some_none) {
@@ -249,6 +343,54 @@ prefill_kernel(const AttnArgs a, int rep) {
   // = dims 16c + 8 kg .. +8
   using E = Elem<DT>;
   const int64_t qrow = row0 + 32 * rb + l32;
+  bool none = false;   // ARR: the row sees no key at all (QSEM averages V then)
+  uint32_t mrow_off = 0;  // ARR: byte offset of the row's mask words
+  if constexpr (ARR) {
+    const int64_t qr = min<int64_t>(qrow, nrows - 1);
+    const int64_t mr = b * a.mw_b + (hk * rep + qr % rep) * a.mw_h + qr / rep;
+    mrow_off = static_cast<uint32_t>(4 * mr * a.mw_words);
+    if constexpr (QSEM) {
+      // (whole 32-bit words: the row's bytes are padded to 4)
+      const int nc = a.mw_words / 8;
+      const uint32_t* ra = reinterpret_cast<const uint32_t*>(a.mrow + mr * nc);
+      uint32_t any = 0;
+      for (int c = 0; c < nc / 4; c++) any |= ra[c];
+      none = any == 0;
+      some_none = __syncthreads_or(none);
+    }
+    // the tiles some row sees, the wholly visible ones first
+    const int nh = a.m_sh ? a.Hkv : 1;
+    const int64_t z = (a.mw_b ? b : 0) * nh + (a.m_sh ? hk : 0);
+    const uint8_t* cls = a.mcls + (z * rblocks + rblk) * a.mw_words + k_begin / kTok;
+    if (wave == 0) {
+      auto cls_at = [&](int t) -> int {
+        if (t >= ntiles) return 0;
+        const int x = cls[t];
+        return QSEM && some_none ? 1 : x;
+      };
+      int open = 0;
+      for (int t0 = 0; t0 < ntiles; t0 += 64)
+        open += __popcll(__builtin_amdgcn_ballot_w64(cls_at(t0 + lane) == 2));
+      int io = 0, ip = open;
+      for (int t0 = 0; t0 < ntiles; t0 += 64) {
+        const int x = cls_at(t0 + lane);
+        const uint64_t bo = __builtin_amdgcn_ballot_w64(x == 2);
+        const uint64_t bp = __builtin_amdgcn_ballot_w64(x == 1);
+        const uint64_t below = (uint64_t{1} << lane) - 1;
+        if (x == 2) tlist[io + __popcll(bo & below)] = static_cast<uint16_t>(t0 + lane);
+        if (x == 1) tlist[ip + __popcll(bp & below)] = static_cast<uint16_t>(t0 + lane);
+        io += __popcll(bo);
+        ip += __popcll(bp);
+      }
+      if (lane == 0) {
+        tcount[0] = ip;
+        tcount[1] = open;
+      }
+    }
+    __syncthreads();
+    ntiles = __builtin_amdgcn_readfirstlane(tcount[0]);
+    n_open = __builtin_amdgcn_readfirstlane(tcount[1]);
+  }
   int64_t kmax;  // last key the row may see
   u32x4_t qf[kChunks];
   {
@@ -309,17 +451,22 @@ prefill_kernel(const AttnArgs a, int rep) {
       const int slot = lane % Cfg::kSlots, r = lrow(x);
       return wave + kWaves * x >= Cfg::kKLoads ? slot ^ vswz<D>(r & 3) : slot ^ kswz<D>(r);
     };
-    uint32_t loff[kLoads];  // offsets within a whole tile (T * stride < 2^31, host-checked)
+    uint32_t loff[Cfg::kLoads];  // offsets within a whole tile (T * stride < 2^31, host-checked)
 #pragma unroll
-    for (int x = 0; x < kLoads; x++) {
+    for (int x = 0; x < Cfg::kLoads; x++) {
       const bool is_v = wave + kWaves * x >= Cfg::kKLoads;  // wave-uniform
       loff[x] = static_cast<uint32_t>(lrow(x) * (is_v ? vst : kst)) + 16 * lpiece(x);
     }
     auto load_tile = [&](int i, int s) __attribute__((always_inline)) {
       const int ti = min(i, ntiles - 1);  // clamped: every wave issues the same loads
-      const int64_t t0 = k_begin + static_cast<int64_t>(kTok) * ti;
+      const int64_t t0 =
+          k_begin + static_cast<int64_t>(kTok) *
+                        (ARR ? __builtin_amdgcn_readfirstlane(tlist[ti]) : ti);
+      if constexpr (ARR)
+        dma4(a.mw, mrow_off + static_cast<uint32_t>(4 * (t0 / kTok)),
+             __builtin_amdgcn_readfirstlane(lds_addr(&mwords[s][wave][0])));
 #pragma unroll
-      for (int x = 0; x < kLoads; x++) {
+      for (int x = 0; x < Cfg::kLoads; x++) {
         const int n = wave + kWaves * x, pn = n % Cfg::kKLoads;
         const bool is_v = n >= Cfg::kKLoads;
         const int64_t st = is_v ? vst : kst;
@@ -347,9 +494,12 @@ prefill_kernel(const AttnArgs a, int rep) {
     const int vpc = 2 * (a4 & 1) + (jj >> 1);  // piece within the 4-piece group
     const int vx = vswz<D>(e4);                // swizzle of rows 4 (a4 / 2) + e (+ 8 hf + 16 ks)
 
-    // QSEM: P carried as hi + lo (two operands of the dtype, ~16
-    // significant bits), so the weighted sum keeps fp32-like accuracy on
-    // large value channels; otherwise one operand
+    // HL: P carried as hi + lo (two operands of the dtype, ~16
+    // significant bits), so the weighted sum keeps fp32-like accuracy (on
+    // large value channels of quantized caches; under array masks, whose
+    // calls held the probabilities in fp32 on the generic kernel: error
+    // against 64 bits 1.7e-3 with it, 2.3e-3 with one bf16 operand);
+    // otherwise one operand
     u32x4_t pb[2], pl[2];
     f32x16_t x;
     // the matrix phase: scores of the tile at LDS base kb (K rows) into x
@@ -383,7 +533,7 @@ prefill_kernel(const AttnArgs a, int rep) {
       if constexpr (PV) {
         // the score chain (8 dependent MFMAs) interleaved with the P.V
         // MFMAs (one chain per 32-dim block)
-        constexpr int kPv = (QSEM ? 4 : 2) * kDBw;  // P.V MFMAs
+        constexpr int kPv = (HL ? 4 : 2) * kDBw;  // P.V MFMAs
         sfor<kChunks>([&](auto C) {
           constexpr int c = decltype(C)::value;
           x = mfma<DT>(kf[c], qf[c], x);
@@ -392,9 +542,9 @@ prefill_kernel(const AttnArgs a, int rep) {
             constexpr int n = decltype(J)::value;  // n-th P.V MFMA
             if constexpr (n >= c * kPv / kChunks && n < (c + 1) * kPv / kChunks) {
               constexpr int db = n % kDBw;
-              constexpr int q = n / kDBw;  // QSEM: ks hi, ks lo; else ks
-              constexpr int ks = QSEM ? q / 2 : q;
-              if constexpr (QSEM && q % 2 == 1)
+              constexpr int q = n / kDBw;  // HL: ks hi, ks lo; else ks
+              constexpr int ks = HL ? q / 2 : q;
+              if constexpr (HL && q % 2 == 1)
                 o[db] = mfma<DT>(vf[db][ks], pl[ks], o[db]);
               else
                 o[db] = mfma<DT>(vf[db][ks], pb[ks], o[db]);
@@ -432,6 +582,7 @@ prefill_kernel(const AttnArgs a, int rep) {
     // softmax of the row over tile i's scores x: the running max and sum,
     // the rescale of o, and the P operands.  EDGE: keys past the range or
     // the causal limit of some row are masked
+    // (ARR: the mask words of the tile, in its stage)
     auto softmax = [&](int i, auto EDGE_) __attribute__((always_inline)) {
       constexpr bool EDGE = decltype(EDGE_)::value;
       const int64_t t0 = k_begin + static_cast<int64_t>(kTok) * i;
@@ -446,7 +597,25 @@ prefill_kernel(const AttnArgs a, int rep) {
           x[j + 1] = E::to_f32(static_cast<typename E::T>(w >> 16));
         }
       }
-      if constexpr (EDGE) {
+      if constexpr (EDGE && ARR) {
+        uint32_t w = mwords[i % kStages][wave][lane];
+        if (QSEM && some_none) {
+          // rows that see no key: equal scores (0) on the row's keys
+          const int64_t left =
+              k_end - k_begin - kTok * static_cast<int64_t>(tlist[i]);  // >= 1
+          const uint32_t all = left >= kTok ? ~0u : (1u << left) - 1;
+          w = none ? all : w;
+#pragma unroll
+          for (int j = 0; j < 16; j++) x[j] = none ? 0.0f : x[j];
+        }
+        w >>= 4 * kg;
+#pragma unroll
+        for (int j = 0; j < 16; j++) {
+          const uint32_t m =
+              static_cast<uint32_t>(__builtin_amdgcn_sbfe(w, 8 * (j >> 2) + (j & 3), 1));
+          x[j] = __uint_as_float((__float_as_uint(x[j]) & m) | (0xff800000u & ~m));
+        }
+      } else if constexpr (EDGE) {
         if (QSEM && some_none && __builtin_amdgcn_ballot_w64(kmax < 0)) {
           // rows that see no key: equal scores (0) on the row's keys
           const bool none = kmax < 0;
@@ -484,7 +653,7 @@ prefill_kernel(const AttnArgs a, int rep) {
         l_run += ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
         pb[ks] = u32x4_t{pack2<DT>(p[0], p[1]), pack2<DT>(p[2], p[3]), pack2<DT>(p[4], p[5]),
                          pack2<DT>(p[6], p[7])};
-        if constexpr (QSEM) {
+        if constexpr (HL) {
           float r[8];
 #pragma unroll
           for (int w = 0; w < 4; w++) {
@@ -595,7 +764,11 @@ bool prefill_supported(int dtype, int bits, const AttnArgs& a) {
   if (dtype != kBF16 && dtype != kF16) return false;
   if (a.L < 2 || a.Dv != a.D || a.Hq % a.Hkv) return false;
   if (a.D != 64 && a.D != 128 && a.D != 256) return false;
-  if (a.mask_mode != 0 && a.mask_mode != 1) return false;
+  // none, causal, or a bool array (additive arrays are the generic kernel's);
+  // an array's scores are compared before the scale, so scale > 0, and its
+  // word offsets are 32-bit
+  if (a.mask_mode != 0 && a.mask_mode != 1 && a.mask_mode != 2) return false;
+  if (a.mask_mode == 2 && (!(a.scale > 0.0f) || !a.mask)) return false;
   // uniform rows: a causal chunk longer than the keys is the generic
   // kernel's; ragged rows (seq_lens) shorter than the chunk see no keys for
   // their first queries, as there
@@ -635,17 +808,71 @@ int prefill_parts(int64_t rows, int Hkv, int64_t L, int rep, int64_t T, int D, i
   return static_cast<int>((T + *part_tokens - 1) / *part_tokens);
 }
 
-template <int D>
+namespace {
+// Extents of a packed mask: batch rows and heads it distinguishes.
+struct MaskPlan {
+  int64_t nb, nz, rows, words, rblocks;
+};
+MaskPlan mask_plan(const AttnArgs& a, int64_t batch) {
+  MaskPlan p;
+  // (rows of unequal length differ even under one mask)
+  p.nb = a.m_sb || a.kv.seq_lens ? batch : 1;
+  p.nz = p.nb * (a.m_sh ? a.Hkv : 1);
+  p.rows = p.nb * (a.m_sh ? a.Hq : 1) * a.L;
+  // whole 1024-key groups, so that a row's per-256-key bytes fill 32-bit words
+  p.words = (static_cast<int64_t>(a.kv.T) + 1023) / 1024 * 32;
+  const int64_t rpw = prefill_rows_per_wg(a.D);
+  p.rblocks = (static_cast<int64_t>(a.L) * (a.Hq / a.Hkv) + rpw - 1) / rpw;
+  return p;
+}
+}  // namespace
+
+bool prefill_mask_fits(const AttnArgs& a, int64_t batch) {
+  if (a.mask_mode != 2) return true;
+  const MaskPlan p = mask_plan(a, batch);
+  return 4 * p.rows * p.words < (int64_t{1} << 32) && p.rblocks < 65536 && p.nz < 65536;
+}
+
+size_t prefill_mask_floats(const AttnArgs& a, int64_t batch) {
+  if (a.mask_mode != 2) return 0;
+  const MaskPlan p = mask_plan(a, batch);
+  const int64_t bytes = 4 * p.rows * p.words + p.rows * p.words / 8 + p.nz * p.rblocks * p.words;
+  return static_cast<size_t>((bytes + 255) / 256 * 64);
+}
+
+void prefill_mask_parts(const AttnArgs& a, int64_t T, int32_t* part_tokens, int32_t* n_parts) {
+  if (a.mask_mode != 2 || *part_tokens <= kMaxMaskTiles * kTok) return;
+  *part_tokens = kMaxMaskTiles * kTok;
+  *n_parts = static_cast<int32_t>((T + *part_tokens - 1) / *part_tokens);
+}
+
+void launch_prefill_mask(AttnArgs& a, int64_t batch, float* ws, hipStream_t st) {
+  if (a.mask_mode != 2 || batch <= 0 || a.L <= 0) return;
+  const MaskPlan p = mask_plan(a, batch);
+  a.mw = reinterpret_cast<uint32_t*>(ws);
+  a.mrow = reinterpret_cast<uint8_t*>(a.mw + p.rows * p.words);
+  a.mcls = a.mrow + p.rows * p.words / 8;
+  a.mw_words = p.words;
+  a.mw_h = a.m_sh ? a.L : 0;
+  a.mw_b = p.nb > 1 ? (a.m_sh ? static_cast<int64_t>(a.Hq) : 1) * a.L : 0;
+  const dim3 grid(static_cast<unsigned>(p.words / 8), static_cast<unsigned>(p.rblocks),
+                  static_cast<unsigned>(p.nz));
+  hipLaunchKernelGGL(mask_pack_kernel, grid, dim3(512), 0, st, a, a.Hq / a.Hkv,
+                     static_cast<int>(prefill_rows_per_wg(a.D)));
+  VKV_HIP(hipGetLastError());
+}
+
+template <int D, bool ARR>
 static void launch_prefill_d(int dtype, bool qsem, const AttnArgs& a, const dim3& grid, int rep,
                              hipStream_t st) {
   if (dtype == kBF16 && qsem)
-    hipLaunchKernelGGL((prefill_kernel<kBF16, true, D>), grid, dim3(kThreads), 0, st, a, rep);
+    hipLaunchKernelGGL((prefill_kernel<kBF16, true, D, ARR>), grid, dim3(kThreads), 0, st, a, rep);
   else if (dtype == kBF16)
-    hipLaunchKernelGGL((prefill_kernel<kBF16, false, D>), grid, dim3(kThreads), 0, st, a, rep);
+    hipLaunchKernelGGL((prefill_kernel<kBF16, false, D, ARR>), grid, dim3(kThreads), 0, st, a, rep);
   else if (qsem)
-    hipLaunchKernelGGL((prefill_kernel<kF16, true, D>), grid, dim3(kThreads), 0, st, a, rep);
+    hipLaunchKernelGGL((prefill_kernel<kF16, true, D, ARR>), grid, dim3(kThreads), 0, st, a, rep);
   else
-    hipLaunchKernelGGL((prefill_kernel<kF16, false, D>), grid, dim3(kThreads), 0, st, a, rep);
+    hipLaunchKernelGGL((prefill_kernel<kF16, false, D, ARR>), grid, dim3(kThreads), 0, st, a, rep);
 }
 
 void launch_prefill(int dtype, bool qsem, const AttnArgs& a, int64_t batch, hipStream_t st,
@@ -660,12 +887,21 @@ void launch_prefill(int dtype, bool qsem, const AttnArgs& a, int64_t batch, hipS
   const int64_t wgs = rblocks * prun * a.Hkv * batch;
   VKV_CHECK(wgs < (int64_t{1} << 31), "too many prefill workgroups for one launch");
   const dim3 grid(static_cast<unsigned>(wgs));
+  VKV_CHECK(a.mask_mode != 2 || (a.mw && a.part_tokens <= kMaxMaskTiles * kTok),
+            "prefill mask not packed");
+  auto run = [&](auto D_) {
+    constexpr int D = decltype(D_)::value;
+    if (a.mask_mode == 2)
+      launch_prefill_d<D, true>(dtype, qsem, a, grid, rep, st);
+    else
+      launch_prefill_d<D, false>(dtype, qsem, a, grid, rep, st);
+  };
   if (a.D == 64)
-    launch_prefill_d<64>(dtype, qsem, a, grid, rep, st);
+    run(std::integral_constant<int, 64>{});
   else if (a.D == 128)
-    launch_prefill_d<128>(dtype, qsem, a, grid, rep, st);
+    run(std::integral_constant<int, 128>{});
   else
-    launch_prefill_d<256>(dtype, qsem, a, grid, rep, st);
+    run(std::integral_constant<int, 256>{});
   VKV_HIP(hipGetLastError());
   if (combine && a.n_parts > 1) launch_attn_combine(dtype, a, batch * a.L, st);
 }

@@ -512,43 +512,49 @@ __global__ void __launch_bounds__(256) scatter_codes_kernel(ScatterCodesArgs a) 
 
 // ------------------------------------------------------------ copy4d
 
-template <typename U>
-__global__ void __launch_bounds__(256) copy4d_kernel(const U* src, U* dst, int64_t n0, int64_t n1,
-                                                     int64_t n2, int64_t n3, int64_t s0, int64_t s1,
-                                                     int64_t s2, int64_t s3, int64_t d0, int64_t d1,
-                                                     int64_t d2, int64_t d3) {
-  const int64_t total = n0 * n1 * n2 * n3;
-  for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < total;
-       i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-    int64_t i3 = i % n3;
-    int64_t r = i / n3;
-    int64_t i2 = r % n2;
-    r /= n2;
-    int64_t i1 = r % n1;
-    int64_t i0 = r / n1;
-    dst[i0 * d0 + i1 * d1 + i2 * d2 + i3 * d3] = src[i0 * s0 + i1 * s1 + i2 * s2 + i3 * s3];
-  }
+// A strided 4-D copy in units of the widest aligned run (1 to 16 bytes):
+// extents and unit strides, outermost first, and the divisors that turn a
+// unit's index into its coordinates (index < 2^31: mul = 2^(31 + sh) / n + 1
+// with 2^sh >= n, so mulhi >> (sh - 1) is the exact quotient).
+struct CopyPlan {
+  const void* src;
+  void* dst;
+  uint32_t total, n[4];
+  int64_t s[4], d[4];
+  uint32_t mul[4], sh[4];
+};
+
+__device__ __forceinline__ uint32_t plan_div(const CopyPlan& p, int k, uint32_t x) {
+  return p.n[k] == 1 ? x : __umulhi(x, p.mul[k]) >> (p.sh[k] - 1);
 }
 
-// Two strided 4-D copies of one element size in one launch (blockIdx.y
-// picks the copy): a cache update writes its K and V tokens with one launch.
-template <typename U>
-__global__ void __launch_bounds__(256) copy4d_pair_kernel(Copy4D c0, Copy4D c1) {
-  const Copy4D& c = blockIdx.y ? c1 : c0;
-  const int64_t total = c.n[0] * c.n[1] * c.n[2] * c.n[3];
-  const U* src = static_cast<const U*>(c.src);
-  U* dst = static_cast<U*>(c.dst);
-  for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < total;
-       i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-    int64_t i3 = i % c.n[3];
-    int64_t r = i / c.n[3];
-    int64_t i2 = r % c.n[2];
-    r /= c.n[2];
-    int64_t i1 = r % c.n[1];
-    int64_t i0 = r / c.n[1];
-    dst[i0 * c.d[0] + i1 * c.d[1] + i2 * c.d[2] + i3 * c.d[3]] =
-        src[i0 * c.s[0] + i1 * c.s[1] + i2 * c.s[2] + i3 * c.s[3]];
+// Up to two copies in one launch (blockIdx.y picks one: a cache update
+// writes its K and V tokens with one launch), N units a thread, all loaded
+// before any is stored.  HBM bound: the copy moves whole 16-byte units where
+// runs and strides allow it, with 32-bit index arithmetic, and keeps N loads
+// in flight a thread.  Measured against one element a thread with 64-bit
+// divisions: 134 MB of f32 rows 126 -> 58 us, 8 x 1023 bf16 rows of 256 dims
+// (8.4 MB moved) 9.3 -> 3.7 us.
+template <typename U, int N>
+__global__ void __launch_bounds__(256) copy_units_kernel(CopyPlan p0, CopyPlan p1) {
+  const CopyPlan& p = blockIdx.y ? p1 : p0;
+  const U* src = static_cast<const U*>(p.src);
+  U* dst = static_cast<U*>(p.dst);
+  const uint32_t i0 = blockIdx.x * (256u * N) + threadIdx.x;
+  if (i0 >= p.total) return;
+  U v[N];
+  int64_t to[N];
+#pragma unroll
+  for (int j = 0; j < N; j++) {
+    const uint32_t i = min(i0 + 256u * j, p.total - 1);  // (clamped copies are not stored)
+    const uint32_t r3 = plan_div(p, 3, i), r2 = plan_div(p, 2, r3), r1 = plan_div(p, 1, r2);
+    const int64_t c3 = i - r3 * p.n[3], c2 = r3 - r2 * p.n[2], c1 = r2 - r1 * p.n[1], c0 = r1;
+    to[j] = c0 * p.d[0] + c1 * p.d[1] + c2 * p.d[2] + c3 * p.d[3];
+    v[j] = src[c0 * p.s[0] + c1 * p.s[1] + c2 * p.s[2] + c3 * p.s[3]];
   }
+#pragma unroll
+  for (int j = 0; j < N; j++)
+    if (i0 + 256u * j < p.total) dst[to[j]] = v[j];
 }
 
 // Whole-block copy across all layers (copy-on-write, prefix store).  The
@@ -1103,44 +1109,140 @@ void launch_scatter_codes(const ScatterCodesArgs& a, hipStream_t st) {
   VKV_HIP(hipGetLastError());
 }
 
-void launch_copy4d(int esize, const void* src, const int64_t* n, const int64_t* s, void* dst,
-                   const int64_t* d, hipStream_t st) {
-  const int64_t total = n[0] * n[1] * n[2] * n[3];
-  if (total <= 0) return;
-  const unsigned nb = static_cast<unsigned>(std::min<int64_t>((total + 255) / 256, 65536));
-  if (esize == 2) {
-    hipLaunchKernelGGL((copy4d_kernel<uint16_t>), dim3(nb), dim3(256), 0, st,
-                       static_cast<const uint16_t*>(src), static_cast<uint16_t*>(dst), n[0], n[1],
-                       n[2], n[3], s[0], s[1], s[2], s[3], d[0], d[1], d[2], d[3]);
-  } else if (esize == 4) {
-    hipLaunchKernelGGL((copy4d_kernel<uint32_t>), dim3(nb), dim3(256), 0, st,
-                       static_cast<const uint32_t*>(src), static_cast<uint32_t*>(dst), n[0], n[1],
-                       n[2], n[3], s[0], s[1], s[2], s[3], d[0], d[1], d[2], d[3]);
-  } else if (esize == 1) {
-    hipLaunchKernelGGL((copy4d_kernel<uint8_t>), dim3(nb), dim3(256), 0, st,
-                       static_cast<const uint8_t*>(src), static_cast<uint8_t*>(dst), n[0], n[1],
-                       n[2], n[3], s[0], s[1], s[2], s[3], d[0], d[1], d[2], d[3]);
-  } else {
-    throw Error("copy4d: element size must be 1, 2 or 4");
+namespace {
+// The copy with its unit dims dropped and dims that are contiguous on both
+// sides joined.
+Copy4D collapse(const Copy4D& c) {
+  Copy4D r = c;
+  int m = 0;  // dims kept, innermost first
+  int64_t n[4], s[4], d[4];
+  for (int i = 3; i >= 0; i--) {
+    if (c.n[i] == 1) continue;
+    if (m > 0 && c.s[i] == s[m - 1] * n[m - 1] && c.d[i] == d[m - 1] * n[m - 1]) {
+      n[m - 1] *= c.n[i];
+    } else {
+      n[m] = c.n[i];
+      s[m] = c.s[i];
+      d[m] = c.d[i];
+      m++;
+    }
+  }
+  for (int k = 0; k < 4; k++) {
+    r.n[3 - k] = k < m ? n[k] : 1;
+    r.s[3 - k] = k < m ? s[k] : k == 0;
+    r.d[3 - k] = k < m ? d[k] : k == 0;
+  }
+  return r;
+}
+
+// The widest unit (bytes) both sides of a collapsed copy are whole in.
+int copy_unit(int es, const Copy4D& c) {
+  if (c.s[3] != 1 || c.d[3] != 1) return es;
+  int u = 16;
+  auto whole = [&](int64_t x) { return x % u == 0; };
+  for (; u > es; u /= 2) {
+    bool ok = whole(c.n[3] * es) && whole(static_cast<int64_t>(reinterpret_cast<uintptr_t>(c.src))) &&
+              whole(static_cast<int64_t>(reinterpret_cast<uintptr_t>(c.dst)));
+    for (int i = 0; ok && i < 3; i++) ok = whole(c.s[i] * es) && whole(c.d[i] * es);
+    if (ok) break;
+  }
+  return u;
+}
+
+CopyPlan copy_plan(const Copy4D& c, int es, int unit) {
+  CopyPlan p{};
+  p.src = c.src;
+  p.dst = c.dst;
+  const int64_t k = unit / es;
+  int64_t total = 1;
+  for (int i = 0; i < 4; i++) {
+    const bool inner = i == 3;
+    const int64_t n = inner ? c.n[i] / k : c.n[i];
+    p.n[i] = static_cast<uint32_t>(n);
+    p.s[i] = inner ? c.s[i] : c.s[i] / k;
+    p.d[i] = inner ? c.d[i] : c.d[i] / k;
+    while ((uint64_t{1} << p.sh[i]) < static_cast<uint64_t>(n)) p.sh[i]++;
+    p.mul[i] = static_cast<uint32_t>((uint64_t{1} << (31 + p.sh[i])) / static_cast<uint64_t>(n) + 1);
+    total *= n;
+  }
+  p.total = static_cast<uint32_t>(total);
+  return p;
+}
+
+template <int N>
+void launch_copy_units(int unit, const CopyPlan& p0, const CopyPlan& p1, const dim3& grid,
+                       hipStream_t st) {
+  switch (unit) {
+    case 1: hipLaunchKernelGGL((copy_units_kernel<uint8_t, N>), grid, dim3(256), 0, st, p0, p1); break;
+    case 2: hipLaunchKernelGGL((copy_units_kernel<uint16_t, N>), grid, dim3(256), 0, st, p0, p1); break;
+    case 4: hipLaunchKernelGGL((copy_units_kernel<uint32_t, N>), grid, dim3(256), 0, st, p0, p1); break;
+    case 8: hipLaunchKernelGGL((copy_units_kernel<uint64_t, N>), grid, dim3(256), 0, st, p0, p1); break;
+    default: hipLaunchKernelGGL((copy_units_kernel<uint4, N>), grid, dim3(256), 0, st, p0, p1);
   }
   VKV_HIP(hipGetLastError());
 }
 
-void launch_copy4d_pair(int esize, const Copy4D& c0, const Copy4D& c1, hipStream_t st) {
-  const int64_t t0 = c0.n[0] * c0.n[1] * c0.n[2] * c0.n[3];
-  const int64_t t1 = c1.n[0] * c1.n[1] * c1.n[2] * c1.n[3];
-  const int64_t total = std::max(t0, t1);
-  if (total <= 0) return;
-  const dim3 grid(static_cast<unsigned>(std::min<int64_t>((total + 255) / 256, 65536)), 2);
-  if (esize == 2)
-    hipLaunchKernelGGL((copy4d_pair_kernel<uint16_t>), grid, dim3(256), 0, st, c0, c1);
-  else if (esize == 4)
-    hipLaunchKernelGGL((copy4d_pair_kernel<uint32_t>), grid, dim3(256), 0, st, c0, c1);
-  else if (esize == 1)
-    hipLaunchKernelGGL((copy4d_pair_kernel<uint8_t>), grid, dim3(256), 0, st, c0, c1);
+// n copies (1 or 2); copies of 2^31 units or more go in halves of their
+// longest dim.
+void launch_copies(int es, const Copy4D* c, int n, hipStream_t st) {
+  if (es != 1 && es != 2 && es != 4) throw Error("copy4d: element size must be 1, 2 or 4");
+  Copy4D r[2];
+  CopyPlan p[2];
+  int unit = 16, m = 0;
+  for (int i = 0; i < n; i++) {
+    int64_t total = 1;
+    for (int k = 0; k < 4; k++) total *= std::max<int64_t>(0, c[i].n[k]);
+    if (total == 0) continue;
+    if (total >= int64_t{1} << 31) {
+      int big = 0;
+      for (int k = 1; k < 4; k++)
+        if (c[i].n[k] > c[i].n[big]) big = k;
+      Copy4D h = c[i];
+      const int64_t half = h.n[big] / 2;
+      h.n[big] = half;
+      launch_copies(es, &h, 1, st);
+      h.n[big] = c[i].n[big] - half;
+      h.src = static_cast<const uint8_t*>(h.src) + half * h.s[big] * es;
+      h.dst = static_cast<uint8_t*>(h.dst) + half * h.d[big] * es;
+      launch_copies(es, &h, 1, st);
+      continue;
+    }
+    r[m] = collapse(c[i]);
+    unit = std::min(unit, copy_unit(es, r[m]));
+    m++;
+  }
+  if (m == 0) return;
+  uint32_t most = 0;
+  for (int i = 0; i < m; i++) {
+    p[i] = copy_plan(r[i], es, unit);
+    most = std::max(most, p[i].total);
+  }
+  if (m == 1) p[1] = p[0];
+  // four units a thread once that leaves every CU eight workgroups
+  constexpr int kN = 4;
+  if (most >= 256u * kN * 2048u)
+    launch_copy_units<kN>(unit, p[0], p[1], dim3((most + 256u * kN - 1) / (256u * kN), m), st);
   else
-    throw Error("copy4d: element size must be 1, 2 or 4");
-  VKV_HIP(hipGetLastError());
+    launch_copy_units<1>(unit, p[0], p[1], dim3((most + 255u) / 256u, m), st);
+}
+}  // namespace
+
+void launch_copy4d(int esize, const void* src, const int64_t* n, const int64_t* s, void* dst,
+                   const int64_t* d, hipStream_t st) {
+  Copy4D c;
+  c.src = src;
+  c.dst = dst;
+  for (int i = 0; i < 4; i++) {
+    c.n[i] = n[i];
+    c.s[i] = s[i];
+    c.d[i] = d[i];
+  }
+  launch_copies(esize, &c, 1, st);
+}
+
+void launch_copy4d_pair(int esize, const Copy4D& c0, const Copy4D& c1, hipStream_t st) {
+  const Copy4D c[2] = {c0, c1};
+  launch_copies(esize, c, 2, st);
 }
 
 void launch_copy_blocks(const uint8_t* base, int64_t layer_bytes, int n_layers, int64_t block_bytes,

@@ -151,31 +151,25 @@ void run_attention(int dtype, int bits, int group, bool qsem, AttnArgs& a, int64
     return;
   }
   if (fdecode_supported(dtype, bits, qsem, a) && !option(VKV_OPTION_GENERIC_ATTENTION)) {
-    // a small launch: one workgroup per (row, head group), merged in LDS
-    // (the fdecode_waves option, a tuning override, keeps the split launch)
-    a.wg_parts = option(VKV_OPTION_FDECODE_WAVES)
-                     ? 0
-                     : fdecode_wg_parts(rows, a.Hq, a.Hkv, max_len, a.D, dtype, &a.part_tokens);
-    if (a.wg_parts > 0) {
-      a.n_parts = a.wg_parts;
-      launch_fdecode(dtype, a, rows, st);
-      return;
-    }
-    a.n_parts = fdecode_parts(rows * a.Hkv, max_len, &a.part_tokens,
-                              static_cast<int>(option(VKV_OPTION_FDECODE_WAVES)));
-    if (a.n_parts > 1) {
-      const size_t per = static_cast<size_t>(rows) * a.Hq * a.n_parts;
+    const int waves = static_cast<int>(option(VKV_OPTION_FDECODE_WAVES));
+    a.n_parts = fdecode_parts(dtype, rows, a.Hq, a.Hkv, max_len, a.D, &a.part_tokens, waves);
+    const size_t per = static_cast<size_t>(rows) * a.Hq * a.n_parts;
+    const size_t counts = static_cast<size_t>(rows) * fdecode_counter_count(a.Hq, a.Hkv);
+    // merged inside the launch where that is the faster merge; the
+    // no-allocation path has no counters
+    const bool inside =
+        !noalloc && a.n_parts > 1 && fdecode_merge_here(dtype, a.n_parts, a.Dv, a.Hq, a.Hkv);
+    if (a.n_parts > 1 && dtype != VKV_F32 && !noalloc &&
+        !attention_scratch_ready(st, per * (a.Dv + 2), counts)) {
+      // a capture that may not allocate: one workgroup a row and head group,
+      // merged in LDS
+      a.n_parts = 1;
+      a.part_tokens = static_cast<int32_t>((max_len + 15) / 16 * 16);
+    } else if (a.n_parts > 1) {
       float* ws = workspace(st, per * (a.Dv + 2), noalloc);
       a.ws_o = ws;
       a.ws_ml = ws + per * a.Dv;
-      // the merge inside the decode launch where the last part's merge is
-      // small (18 parts x 128 dims x 4 heads, one f16 row: step 19.4 -> 17.8
-      // us); larger ones keep the separate merge (config 4's window layer,
-      // 32 parts x 256 dims x 2 heads: 19.9 us with it, 25.1 inside), as
-      // does the no-allocation path, which has no counters
-      if (!noalloc && fdecode_merge_here(a.n_parts, a.Dv, a.Hq, a.Hkv))
-        a.counters = attention_counters(st, static_cast<size_t>(rows) *
-                                                fdecode_counter_count(a.Hq, a.Hkv));
+      if (inside) a.counters = attention_counters(st, counts);
     }
     launch_fdecode(dtype, a, rows, st);
     return;
@@ -218,7 +212,10 @@ void run_attention(int dtype, int bits, int group, bool qsem, AttnArgs& a, int64
       const size_t copy_floats = static_cast<size_t>((2 * wbytes + 255) / 256 * 64);
       const size_t per = static_cast<size_t>(rows) * a.Hq * d.n_parts;
       const size_t part_floats = d.n_parts > 1 ? (per * (a.Dv + 2) + 63) / 64 * 64 : 0;
-      float* ws = workspace(st, copy_floats + part_floats + prefill_mask_floats(d, batch), noalloc);
+      const size_t floats = copy_floats + part_floats + prefill_mask_floats(d, batch);
+      // (an array mask under a capture that may not allocate: the generic kernel)
+      if (d.mask_mode != 2 || attention_scratch_ready(st, floats, 0)) {
+      float* ws = workspace(st, floats, noalloc);
       uint8_t* kd = reinterpret_cast<uint8_t*>(ws);
       uint8_t* vd = kd + wbytes;
       const int64_t wph = wtok * a.D * es;  // copy bytes per (row, kv head)
@@ -252,6 +249,7 @@ void run_attention(int dtype, int bits, int group, bool qsem, AttnArgs& a, int64
       }
       if (d.n_parts > 1) launch_attn_combine(dtype, d, rows, st);
       return;
+      }
     }
   }
   if (prefill_supported(dtype, bits, a) && !option(VKV_OPTION_GENERIC_ATTENTION) &&
@@ -262,14 +260,16 @@ void run_attention(int dtype, int bits, int group, bool qsem, AttnArgs& a, int64
     const size_t per = static_cast<size_t>(rows) * a.Hq * a.n_parts;
     const size_t part_floats = a.n_parts > 1 ? (per * (a.Dv + 2) + 63) / 64 * 64 : 0;
     const size_t mask_floats = prefill_mask_floats(a, batch);
-    if (part_floats + mask_floats) {
-      float* ws = workspace(st, part_floats + mask_floats, noalloc);
-      a.ws_o = ws;
-      a.ws_ml = ws + per * a.Dv;
-      launch_prefill_mask(a, batch, ws + part_floats, st);
+    if (a.mask_mode != 2 || attention_scratch_ready(st, part_floats + mask_floats, 0)) {
+      if (part_floats + mask_floats) {
+        float* ws = workspace(st, part_floats + mask_floats, noalloc);
+        a.ws_o = ws;
+        a.ws_ml = ws + per * a.Dv;
+        launch_prefill_mask(a, batch, ws + part_floats, st);
+      }
+      launch_prefill(dtype, qsem, a, batch, st);
+      return;
     }
-    launch_prefill(dtype, qsem, a, batch, st);
-    return;
   }
   a.n_parts = choose_parts(rows * a.Hkv, max_len, &a.part_tokens);
   if (a.n_parts > 1) {

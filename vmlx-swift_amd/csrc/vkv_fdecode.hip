@@ -8,43 +8,55 @@
 // yields zeros; split partials are merged by attn_combine_kernel as
 // sdpa_vector_2pass_2 merges them (sdpa_vector.h:320-394).
 //
-// Layout.  One wave per workgroup owns a (row, kv head, head group, token
-// range) and walks it 32 tokens at a time:
-//   * scores, bf16 / f16 K/V: on matrix cores, S^T (16 tokens x 16 columns,
-//     the group's REP <= 8 heads) = K (A operands: lane (m, g) loads dims
-//     32 s + 8 g .. + 7 of token m of a 16-token tile, 16 bytes straight
-//     from memory) . Q^T (B operands: the raw queries in registers), one
-//     16x16x32 MFMA per tile and 32 dims; the fp32 scores are then scaled
-//     (the reference scales the queries first: the same fp32 arithmetic up
-//     to summation order).  The max and sum of a head reduce over the four
-//     lanes that hold it and reach every lane through readlane (config 4's
-//     window layer: 16.0 -> 12.1 us; config 1's step 17.8 -> 16.1 us);
-//   * scores, f32 K/V: lanes t and t + 32 own token t, each taking half of
-//     its key row with 16-byte loads (every byte of a row used), against the
-//     queries of the group's REP heads in LDS; one lane swap adds the
-//     halves.  Two lanes per token give a launch twice the waves of one
-//     lane per token for the same bytes (a 33.6 MB D = 256 decode: 14.9 ->
-//     12.3 us).
-//   * online softmax per head over the 32 scores (DPP reductions within
-//     each half-wave), the probabilities into LDS;
-//   * values: lanes own 16-byte runs of a value row, D/8 (bf16/f16) or D/4
-//     (f32) lanes per row, so every load instruction reads whole rows;
-//     the lanes that share a run sum their tokens at the end.
-// The value contraction stays on the vector ALUs (at REP <= 8 query heads
-// per kv head about one FMA per KV byte); on matrix cores its value rows
-// would have to be transposed through LDS.
+// bf16 / f16 K/V (fdecode16_kernel).  A workgroup of 8 waves owns a (row, kv
+// head, head group, token part) and deals its part to the waves in steps of
+// 16 tokens:
+//   * scores on matrix cores, S^T (16 tokens x 16 columns, the group's REP <=
+//     8 heads) = K (A operands: lane (m, g) loads dims 32 s + 8 g .. + 7 of
+//     token m, 16 bytes straight from memory) . Q^T (B operands: the raw
+//     queries in registers), one 16x16x32 MFMA per 32 dims; the fp32 scores
+//     are then scaled (the reference scales the queries first: the same fp32
+//     arithmetic up to summation order);
+//   * online softmax in the lanes that hold a head's scores, the running max
+//     refreshed only when a score exceeds it by kTau (one ballot a step), the
+//     sum kept per lane until the end, the probabilities through LDS;
+//   * values on the vector ALUs (at REP <= 8 heads about one FMA a byte):
+//     lanes own 16-byte runs of a value row, D / 8 lanes a row, so every load
+//     instruction reads whole rows; the lanes that share a run sum their
+//     tokens at the end.
+// A step's keys are loaded while the step before is in its softmax and
+// values, its values while it is in its scores: the operand registers are
+// reloaded as soon as they are used, so a wave always has loads in flight
+// and still fits 128 registers (four waves a SIMD).  Loads are buffer loads
+// with the step's base in scalar registers and the rows that exist as the
+// bound: rows past the end read as zeros without traffic, and a lane's
+// addresses are two 32-bit offsets.  K/V may be dense (strided slices of a
+// cache) or float pages behind a block table, rows of unequal length.
 //
-// Split merge.  With counters (one per (row, kv head, head group)) the
-// parts merge inside the launch: each part stores its (o, max, sum)
-// partial with device-coherent stores (relaxed agent-scope atomics, which
-// write through to the level every XCD reads), waits for them to complete,
-// and counts itself in; the part that counts last reads every partial back
-// with device-coherent loads, merges them as sdpa_vector_2pass_2 does and
-// writes the output, then zeroes the counter for the next launch.  No
-// fence writes back or invalidates an L2, and a part has no loads in
-// flight when it waits for its stores.  Without counters the partials go
-// to attn_combine_kernel (a launch of its own).
+// Bound: HBM on large launches, the chain launch -> queries and first rows ->
+// merge on small ones.  Measured against one-wave workgroups that loaded a
+// 32-token step and then computed on it, with a merge launch behind (us a
+// call): 8 x 6001 tokens, 8/32 heads x 128 (197 MB) 52.1 -> 37.7 (5.2 TB/s);
+// 4 x 1024 tokens, 8/16 heads x 256 (34 MB) 15.8 -> 11.8; one row of 512 tokens
+// 10.0 -> 9.3; pages of 16 rows of 128-4096 tokens (159 MB, the generic kernel
+// before) 214 -> 39.
+//
+// Split merge.  The waves merge in LDS (sdpa_vector.h:320-394).  Parts
+// merge inside the launch: the workgroup stores its (o, max, sum) with
+// device-coherent stores (relaxed agent-scope atomics, which write through to
+// the level every XCD reads), waits for them and counts itself in on a
+// per-(row, kv head, head group) counter; the workgroup that counts last
+// reads the parts back with device-coherent loads, merges them, writes the
+// output and zeroes the counter for the next launch.  No fence writes back
+// or invalidates an L2.  Without counters (the no-allocation entry point) the
+// partials go to attn_combine_kernel.
+//
+// f32 K/V (fdecode_kernel): one wave per workgroup and token part, steps of
+// 32 tokens, lanes t and t + 32 on token t, each scoring half of its row
+// against the queries in LDS; parts merge as above or in
+// attn_combine_kernel.
 #include <algorithm>
+#include <type_traits>
 
 #include "vkv_device.h"
 #include <hip/hip_ext.h>
@@ -142,23 +154,6 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
 }
 
-// Waves of a workgroup that owns a whole (row, kv head, head group) and
-// merges its parts in LDS: up to 8 (two per SIMD: the kernel needs ~240
-// registers a wave, and 16 waves would leave it 128, spilling), with the
-// partials (REP x D floats a wave) within 48 KB.
-template <int D, int REP>
-constexpr int fd_wg_waves() {
-  constexpr int n = 49152 / (REP * D * 4);
-  return n > 8 ? 8 : (n < 2 ? 2 : n);
-}
-// The shapes whose 8-wave workgroup fits its registers without spilling:
-// bf16 / f16 (matrix-core scores) at 64 dims, or 128 dims and at most 4
-// heads per group.
-template <int DT, int D, int REP>
-constexpr bool fd_wg_ok() {
-  return DT != kF32 && (D == 64 || (D == 128 && REP <= 4));
-}
-
 // The in-launch merge of a (row, kv head, head group)'s parts
 // (sdpa_vector.h:320-394), by the part that counted in last: the partials
 // come back through device-coherent loads; all 64 lanes take D / 64 dims of
@@ -225,8 +220,9 @@ __device__ __forceinline__ void fdecode_merge_rows(const AttnArgs& a, int64_t b,
   }
 }
 
-template <int DT, int D, int REP, int NW = 1>
-__global__ void __launch_bounds__(64 * NW) fdecode_kernel(AttnArgs a, int rep_total) {
+template <int DT, int D, int REP>
+__global__ void __launch_bounds__(64) fdecode_kernel(AttnArgs a, int rep_total) {
+  static_assert(DT == kF32, "16-bit K/V take fdecode16_kernel");
   using E = Elem<DT>;
   constexpr int VEC = 16 / E::kBytes;  // elements per 16-byte load
   constexpr int KL = D / VEC;          // loads per key row
@@ -234,26 +230,10 @@ __global__ void __launch_bounds__(64 * NW) fdecode_kernel(AttnArgs a, int rep_to
   constexpr int RPI = 64 / LPR;        // value rows per load instruction
   static_assert(LPR <= 64 && 64 % LPR == 0, "value rows must tile a wave");
   static_assert(KL % 2 == 0 && kStep % RPI == 0, "key rows split in two halves, value rows tile a step");
-  // bf16 / f16 K/V: the scores on matrix cores (S^T = K . Q^T, 16 tokens x
-  // 16 columns of heads per MFMA, the raw queries as B operands, the scale
-  // applied to the fp32 scores); f32 K/V: on the vector ALUs
-  constexpr bool MF = DT != kF32;
-  constexpr int KS = D / 32;  // 32-dim K steps of a key row
-  static_assert(!MF || 2 * KS == KL / 2, "the key operands reuse the key-load registers");
-  // (NW > 1: a workgroup of NW waves owns the whole row, wave w its part
-  // w, and merges the parts in LDS at the end; each wave's LDS is its own)
-  __shared__ float qs_g[NW][MF ? 1 : REP][MF ? 1 : D];
-  __shared__ float ps_g[NW][REP][kStep];
-  const int wv = NW > 1 ? static_cast<int>(threadIdx.x >> 6) : 0;
-  float(*qs)[MF ? 1 : D] = qs_g[wv];
-  float(*ps)[kStep] = ps_g[wv];
-  auto step_sync = [&]() __attribute__((always_inline)) {
-    if constexpr (NW > 1) wave_lds_sync();
-    else __syncthreads();
-  };
-
+  __shared__ float qs[REP][D];
+  __shared__ float ps[REP][kStep];
   const int lane = threadIdx.x & 63;
-  const int part = static_cast<int>(blockIdx.x) * NW + wv;
+  const int part = static_cast<int>(blockIdx.x);
   const int n_hg = (rep_total + REP - 1) / REP;
   const int hk = blockIdx.y / n_hg, hg = blockIdx.y % n_hg;
   const int64_t b = blockIdx.z;
@@ -286,25 +266,11 @@ __global__ void __launch_bounds__(64 * NW) fdecode_kernel(AttnArgs a, int rep_to
   const bool writes_new = new_t >= t_begin && new_t < t_end && hg == 0;
   const uint8_t* nkrow = a.has_new ? a.nk_ptr + b * a.nk_sb + hk * a.nk_sh : kbase;
   const uint8_t* nvrow = a.has_new ? a.nv_ptr + b * a.nv_sb + hk * a.nv_sh : vbase;
-  // matrix-core layout: lane (mrow, kgrp) loads dims 32 s + 8 kgrp .. + 7 of
-  // token t0 + 16 T + mrow into kw[T KS + s] (the A operand of step s, tile T)
-  const int mrow = lane & 15, kgrp = lane >> 4;
   auto load_k = [&](int64_t t0) __attribute__((always_inline)) {
-    if constexpr (MF) {
+    const int64_t t = t0 + tok < t_end ? t0 + tok : t_begin;
+    const uint8_t* krow = (t == new_t ? nkrow : kbase + t * kst) + 16 * (KL / 2) * half;
 #pragma unroll
-      for (int T = 0; T < 2; T++) {
-        const int64_t tt = t0 + 16 * T + mrow;
-        const int64_t t = tt < t_end ? tt : t_begin;
-        const uint8_t* krow = (t == new_t ? nkrow : kbase + t * kst) + 16 * kgrp;
-#pragma unroll
-        for (int st = 0; st < KS; st++) kw[T * KS + st] = *(g_u32x4_t*)(krow + 64 * st);
-      }
-    } else {
-      const int64_t t = t0 + tok < t_end ? t0 + tok : t_begin;
-      const uint8_t* krow = (t == new_t ? nkrow : kbase + t * kst) + 16 * (KL / 2) * half;
-#pragma unroll
-      for (int c = 0; c < KL / 2; c++) kw[c] = *(g_u32x4_t*)(krow + 16 * c);
-    }
+    for (int c = 0; c < KL / 2; c++) kw[c] = *(g_u32x4_t*)(krow + 16 * c);
   };
   auto load_v = [&](int64_t t0) __attribute__((always_inline)) {
 #pragma unroll
@@ -316,40 +282,24 @@ __global__ void __launch_bounds__(64 * NW) fdecode_kernel(AttnArgs a, int rep_to
 
   // the queries (times the scale) go to LDS; their loads go out first,
   // then the first step's key and value loads, so both latencies overlap
-  constexpr int NQ = MF ? 1 : REP * D / 64;
+  constexpr int NQ = REP * D / 64;
   float qv[NQ];
-  u32x4_t qb[MF ? KS : 1];  // matrix-core B operands: head mrow, dims 32 s + 8 kgrp .. + 7
-  if constexpr (MF) {
-    const uint16_t* qp = static_cast<const uint16_t*>(a.q) + b * a.q_sb +
-                         static_cast<int64_t>(h0 + min(mrow, nh - 1)) * a.q_sh + 8 * kgrp;
 #pragma unroll
-    for (int st = 0; st < KS; st++) {
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        const uint32_t lo = qp[32 * st + 2 * e], hi = qp[32 * st + 2 * e + 1];
-        qb[st][e] = mrow < nh ? (lo | (hi << 16)) : 0u;
-      }
-    }
-  } else {
-#pragma unroll
-    for (int j = 0; j < NQ; j++) {
-      const int i = lane + 64 * j, r = i / D, d = i % D;
-      qv[j] = r < nh ? E::load(static_cast<const typename E::T*>(a.q) + b * a.q_sb + (h0 + r) * a.q_sh + d)
-                     : 0.0f;
-    }
+  for (int j = 0; j < NQ; j++) {
+    const int i = lane + 64 * j, r = i / D, d = i % D;
+    qv[j] = r < nh ? E::load(static_cast<const typename E::T*>(a.q) + b * a.q_sb + (h0 + r) * a.q_sh + d)
+                   : 0.0f;
   }
   if (t_begin < t_end) {
     load_k(t_begin);
     if constexpr (kVEarly) load_v(t_begin);
   }
-  if constexpr (!MF) {
 #pragma unroll
-    for (int j = 0; j < NQ; j++) {
-      const int i = lane + 64 * j;
-      qs[i / D][i % D] = qv[j] * a.scale;
-    }
-    step_sync();
+  for (int j = 0; j < NQ; j++) {
+    const int i = lane + 64 * j;
+    qs[i / D][i % D] = qv[j] * a.scale;
   }
+  __syncthreads();
   float m[REP], l[REP], o[REP][VEC];
 #pragma unroll
   for (int r = 0; r < REP; r++) {
@@ -375,83 +325,6 @@ __global__ void __launch_bounds__(64 * NW) fdecode_kernel(AttnArgs a, int rep_to
       load_k(t0);
       if constexpr (kVEarly) load_v(t0);
     }
-    if constexpr (MF) {
-      // ---- scores on matrix cores: lane (mrow, kgrp) ends with head mrow
-      // of tokens t0 + 16 T + 4 kgrp + i
-      f32x4_t acc[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
-#pragma unroll
-      for (int st = 0; st < KS; st++)
-#pragma unroll
-        for (int T = 0; T < 2; T++) acc[T] = mfma16<DT>(kw[T * KS + st], qb[st], acc[T]);
-      if constexpr (!kVEarly) load_v(t0);
-      if (writes_new) {  // the new token's key row into the cache
-#pragma unroll
-        for (int T = 0; T < 2; T++) {
-          if (t0 + 16 * T + mrow == new_t) {
-            uint8_t* dst = const_cast<uint8_t*>(kbase) + new_t * kst + 16 * kgrp;
-#pragma unroll
-            for (int st = 0; st < KS; st++) *reinterpret_cast<u32x4_t*>(dst + 64 * st) = kw[T * KS + st];
-          }
-        }
-      }
-      float sc[2][4];
-      float mx = -INFINITY;
-#pragma unroll
-      for (int T = 0; T < 2; T++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-          const int64_t t = t0 + 16 * T + 4 * kgrp + i;
-          float x = acc[T][i] * a.scale;
-          bool vis = t < t_end && mrow < nh;
-          if (vis && a.mask_mode >= 2) {
-            const int64_t mo = b * a.m_sb + (h0 + mrow) * a.m_sh + t * a.m_st;
-            if (a.mask_mode == 2) {
-              vis = static_cast<const uint8_t*>(a.mask)[mo] != 0;
-            } else {
-              // the mask in the query dtype; keys below its lowest finite
-              // value are skipped (sdpa_vector.h:105-121)
-              const float add = load_as<DT>(a.mask, a.mask_dtype, mo);
-              vis = add >= -E::kMax;
-              x += add;
-            }
-          }
-          sc[T][i] = vis ? x : -INFINITY;
-          mx = fmaxf(mx, sc[T][i]);
-        }
-      // the step's max of head mrow over its four lanes, then the new
-      // running max (this lane's head)
-      mx = fmaxf(mx, __shfl_xor(mx, 16));
-      mx = fmaxf(mx, __shfl_xor(mx, 32));
-      float m_own = m[0];
-#pragma unroll
-      for (int r = 1; r < REP; r++) m_own = mrow == r ? m[r] : m_own;
-      const float mn_own = fmaxf(m_own, mx);
-      float psum = 0.0f;
-#pragma unroll
-      for (int T = 0; T < 2; T++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-          const float pr = (mn_own == -INFINITY || sc[T][i] == -INFINITY) ? 0.0f
-                                                                         : __expf(sc[T][i] - mn_own);
-          psum += pr;
-          if (mrow < REP) ps[mrow][16 * T + 4 * kgrp + i] = pr;
-        }
-      psum += __shfl_xor(psum, 16);
-      psum += __shfl_xor(psum, 32);
-      // ---- online softmax per head (sdpa_vector.h:116-131): lane r holds
-      // head r's new max and step sum
-#pragma unroll
-      for (int r = 0; r < REP; r++) {
-        const float mn = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, mn_own), r));
-        const float ls = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, psum), r));
-        float alpha = 1.0f;
-        if (mn != -INFINITY) alpha = m[r] == -INFINITY ? 0.0f : __expf(m[r] - mn);
-        l[r] = l[r] * alpha + ls;
-        m[r] = mn;
-#pragma unroll
-        for (int e = 0; e < VEC; e++) o[r][e] *= alpha;
-      }
-    } else {
     float s[REP];
 #pragma unroll
     for (int r = 0; r < REP; r++) s[r] = 0.0f;
@@ -506,8 +379,7 @@ __global__ void __launch_bounds__(64 * NW) fdecode_kernel(AttnArgs a, int rep_to
 #pragma unroll
       for (int e = 0; e < VEC; e++) o[r][e] *= alpha;
     }
-    }
-    step_sync();
+    __syncthreads();
 #pragma unroll
     for (int k = 0; k < NV; k++) {
       const int tt = rs + RPI * k;
@@ -522,7 +394,7 @@ __global__ void __launch_bounds__(64 * NW) fdecode_kernel(AttnArgs a, int rep_to
         for (int e = 0; e < VEC; e++) o[r][e] = fmaf(p, vv[e], o[r][e]);
       }
     }
-    step_sync();
+    __syncthreads();
   }
 
   // the row slots of a run hold disjoint tokens: sum them
@@ -534,40 +406,6 @@ __global__ void __launch_bounds__(64 * NW) fdecode_kernel(AttnArgs a, int rep_to
       if constexpr (LPR <= 16) o[r][e] += swz_xor<16>(o[r][e]);
       if constexpr (LPR <= 32) o[r][e] = add_xor32(o[r][e]);
     }
-  if constexpr (NW > 1) {
-    // ---- the workgroup's parts merge in LDS (sdpa_vector.h:320-394): each
-    // wave's (o, max, sum) per head, then every thread one (head, dim)
-    __shared__ float mo_g[NW][REP][D];
-    __shared__ float ml_g[NW][REP][2];
-    if (rs == 0) {
-#pragma unroll
-      for (int r = 0; r < REP; r++) {
-#pragma unroll
-        for (int e = 0; e < VEC; e++) mo_g[wv][r][VEC * dg + e] = o[r][e];
-        if (dg == 0) {
-          ml_g[wv][r][0] = m[r];
-          ml_g[wv][r][1] = l[r];
-        }
-      }
-    }
-    __syncthreads();
-    for (int idx = threadIdx.x; idx < nh * D; idx += 64 * NW) {
-      const int r = idx / D, d = idx % D;
-      float M = -3.402823466e38f;
-#pragma unroll
-      for (int w = 0; w < NW; w++) M = fmaxf(M, ml_g[w][r][0]);
-      float den = 0.0f, acc = 0.0f;
-#pragma unroll
-      for (int w = 0; w < NW; w++) {
-        const float f = __expf(ml_g[w][r][0] - M);
-        den = fmaf(f, ml_g[w][r][1], den);
-        acc = fmaf(f, mo_g[w][r][d], acc);
-      }
-      typename E::T* out = static_cast<typename E::T*>(a.out) + b * a.o_sb + (h0 + r) * a.o_sh + d;
-      *out = E::from_f32(den > 0.0f ? acc / den : 0.0f);
-    }
-    return;
-  }
   const bool merge_here = a.n_parts > 1 && a.counters;
   if (rs == 0) {
 #pragma unroll
@@ -616,43 +454,379 @@ __global__ void __launch_bounds__(64 * NW) fdecode_kernel(AttnArgs a, int rep_to
   fdecode_merge_rows<DT, D, REP>(a, b, h0, nh, lane);
 }
 
+// ------------------------------------------------------ 16-bit K/V
+
+constexpr int kWaves16 = 8;    // waves of a workgroup
+constexpr int kStep16 = 16;    // tokens of a wave's step
+constexpr float kTau = 8.0f;   // the running max lags a score by at most this
+constexpr float kLowest = -3.402823466e38f;
+
+typedef __attribute__((address_space(4))) const int32_t c_i32_t;
+
+// Registers a wave: 128 (four waves a SIMD, two workgroups a CU) where the
+// operands of a step (D / 4 registers), the queries and the accumulators
+// (8 a head) leave room for the rest; else two waves a SIMD.
+template <int D, int REP>
+constexpr int fd16_waves_per_simd() {
+  return D / 4 + D / 8 + 9 * REP <= 92 ? 4 : 2;
+}
+
+// Dense rows, dense rows under an array mask (its loads and 64-bit offsets
+// would cost the plain loop registers), or float pages.
+enum { kDense = 0, kMasked = 1, kPages = 2 };
+
+template <int DT, int D, int REP, int MODE>
+__global__ void __launch_bounds__(64 * kWaves16)
+    __attribute__((amdgpu_waves_per_eu(fd16_waves_per_simd<D, REP>())))
+    fdecode16_kernel(const AttnArgs a, int rep_total) {
+  using E = Elem<DT>;
+  constexpr bool PAGED = MODE == kPages;
+  constexpr int KS = D / 32;         // 32-dim K steps of a key row
+  constexpr int LPR = D / 8;         // lanes per value row
+  constexpr int NV = LPR / 4;        // value rows a lane reads a step (16 rows over 64 / LPR slots)
+  constexpr int NW = kWaves16;
+  __shared__ __attribute__((aligned(16))) float ps_g[NW][REP][kStep16];
+  __shared__ __attribute__((aligned(16))) float mo_g[NW][REP][D];
+  __shared__ float ml_g[NW][REP][2];
+  __shared__ int last_s;
+
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int part = blockIdx.x;
+  const int n_hg = (rep_total + REP - 1) / REP;
+  const int hk = blockIdx.y / n_hg, hg = blockIdx.y - hk * n_hg;
+  const int64_t b = blockIdx.z;
+  const int h0 = hk * rep_total + hg * REP;
+  const int nh = min(REP, rep_total - hg * REP);
+  const int T = a.kv.seq_lens ? min(a.kv.seq_lens[b], a.kv.T) : a.kv.T;
+  const int t_begin = part * a.part_tokens;
+  const int t_end = min(T, t_begin + a.part_tokens);
+  // parts of this row (its own length's); the others have nothing to add
+  const int np = T > 0 ? (T + a.part_tokens - 1) / a.part_tokens : 1;
+  const bool merge_here = a.counters != nullptr;
+  if (part >= np && (merge_here || a.n_parts == 1)) return;
+  const int nsteps = t_end > t_begin ? (t_end - t_begin + kStep16 - 1) / kStep16 : 0;
+
+  const int mrow = lane & 15, kgrp = lane >> 4;  // scores: token / head column, dims 8 kgrp
+  const int rs = lane / LPR, dg = lane % LPR;    // values: row slot (tokens NV rs ..), run
+  const uint8_t* kbase = a.kv.kc.ptr + hk * a.kv.kc.sh + (PAGED ? 0 : b * a.kv.kc.sb);
+  const uint8_t* vbase = a.kv.vc.ptr + hk * a.kv.vc.sh + (PAGED ? 0 : b * a.kv.vc.sb);
+  const int kst = static_cast<int>(a.kv.kc.st), vst = static_cast<int>(a.kv.vc.st);
+  // (the whole offset in the vector operand: the bound is checked against
+  // it less the scalar offset, which would wrap on an empty buffer)
+  const int koff = mrow * kst + 16 * kgrp, voff = NV * rs * vst + 16 * dg;
+  const int bs = a.kv.block_size;
+  // page of token t: the quotient by multiplication, in scalar registers (a
+  // division would hold vector registers through the loop)
+  auto page = [&](int t) __attribute__((always_inline)) {
+    return static_cast<int>(__umulhi(static_cast<uint32_t>(t), a.bs_mul) >> a.bs_sh);
+  };
+  c_i32_t* table = (c_i32_t*)(a.kv.table + (PAGED ? b * a.kv.table_stride : 0));
+  // step i of the part: its first token and (paged) block; steps past the
+  // end read nothing
+  auto block_of = [&](int i) __attribute__((always_inline)) {
+    const int t = t_begin + kStep16 * min(i, max(nsteps - 1, 0));
+    return nsteps > 0 ? table[page(t)] : 0;
+  };
+  u32x4_t kw[KS], vw[NV];
+  // non-temporal where one workgroup reads a row (at REP = 8 further head
+  // groups may): 8 x 6001 bf16 tokens 40.2 -> 37.6 us
+  constexpr int kNt = REP < 8 ? 2 : 0;
+  // K (or V) rows of step i, as a buffer whose end is the last row's
+  auto rows_of = [&](const uint8_t* base, const Comp& c, int st, int i, int blk) __attribute__((always_inline)) {
+    const int t0 = t_begin + kStep16 * i;
+    const int n = min(t_end - t0, kStep16);
+    const uint8_t* p = base;
+    if constexpr (PAGED)
+      p += blk * c.sb + static_cast<int64_t>(t0 - page(t0) * bs) * st;
+    else
+      p += static_cast<int64_t>(t0) * st;
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(p), 0,
+                                             n > 0 ? (n - 1) * st + 2 * D : 0, 0x00020000);
+  };
+  auto load_k = [&](int i, int blk) __attribute__((always_inline)) {
+    const auto r = rows_of(kbase, a.kv.kc, kst, i, blk);
+#pragma unroll
+    for (int s = 0; s < KS; s++) kw[s] = __builtin_amdgcn_raw_buffer_load_b128(r, koff + 64 * s, 0, kNt);
+  };
+  auto load_v = [&](int i, int blk) __attribute__((always_inline)) {
+    const auto r = rows_of(vbase, a.kv.vc, vst, i, blk);
+#pragma unroll
+    for (int k = 0; k < NV; k++) vw[k] = __builtin_amdgcn_raw_buffer_load_b128(r, voff + k * vst, 0, kNt);
+  };
+
+  int blk = 0, blk_next = 0;
+  if constexpr (PAGED) {
+    blk = block_of(wv);
+    blk_next = block_of(wv + NW);
+  }
+  // the queries, B operands: head mrow, dims 32 s + 8 kgrp .. + 7
+  u32x4_t qb[KS];
+  {
+    const uint16_t* qp = static_cast<const uint16_t*>(a.q) + b * a.q_sb +
+                         static_cast<int64_t>(h0 + min(mrow, nh - 1)) * a.q_sh + 8 * kgrp;
+    if (((reinterpret_cast<uintptr_t>(a.q) >> 1 | a.q_sb | a.q_sh) & 7) == 0) {
+#pragma unroll
+      for (int s = 0; s < KS; s++) qb[s] = *(g_u32x4_t*)(qp + 32 * s);
+    } else {
+#pragma unroll 1
+      for (int e = 0; e < 4; e++)
+#pragma unroll
+        for (int s = 0; s < KS; s++) {
+          const uint32_t w = qp[32 * s + 2 * e] | static_cast<uint32_t>(qp[32 * s + 2 * e + 1]) << 16;
+#pragma unroll
+          for (int x = 0; x < 4; x++) qb[s][x] = x == e ? w : qb[s][x];
+        }
+    }
+  }
+  load_k(wv, blk);
+  load_v(wv, blk);
+#pragma unroll
+  for (int s = 0; s < KS; s++)
+#pragma unroll
+    for (int e = 0; e < 4; e++) qb[s][e] = mrow < nh ? qb[s][e] : 0u;
+
+  float m_own = kLowest, l_own = 0.0f;  // this lane's head: running max, its share of the sum
+  // an attention sink is one more logit with a zero value row, counted once
+  // per row: the running max starts at it with sum 1 (sdpa_vector.h:93-96)
+  if (a.sinks && part == 0 && wv == 0 && mrow < nh) {
+    m_own = load_as<DT>(a.sinks, a.sinks_dtype, h0 + mrow);
+    l_own = kgrp == 0 ? 1.0f : 0.0f;
+  }
+  float o[REP][8];
+#pragma unroll
+  for (int r = 0; r < REP; r++)
+#pragma unroll
+    for (int e = 0; e < 8; e++) o[r][e] = 0.0f;
+
+  for (int i = wv; i < nsteps; i += NW) {
+    const int t0 = t_begin + kStep16 * i;
+    if (!PAGED && a.has_new && a.new_t >= t0 && a.new_t < t0 + kStep16) {
+      // a cache update's deferred token: its rows come from the caller's
+      // arrays, and the first head group writes them into the cache
+      const int at = static_cast<int>(a.new_t) - t0;
+      const uint8_t* nk = a.nk_ptr + b * a.nk_sb + hk * a.nk_sh + 16 * kgrp;
+      const uint8_t* nv = a.nv_ptr + b * a.nv_sb + hk * a.nv_sh + 16 * dg;
+      uint8_t* ck = const_cast<uint8_t*>(kbase) + a.new_t * kst + 16 * kgrp;
+      uint8_t* cv = const_cast<uint8_t*>(vbase) + a.new_t * vst + 16 * dg;
+      if (mrow == at) {
+#pragma unroll
+        for (int s = 0; s < KS; s++) {
+          kw[s] = *(g_u32x4_t*)(nk + 64 * s);
+          if (hg == 0) *reinterpret_cast<u32x4_t*>(ck + 64 * s) = kw[s];
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < NV; k++) {
+        if (NV * rs + k == at) {
+          vw[k] = *(g_u32x4_t*)nv;
+          if (hg == 0) *reinterpret_cast<u32x4_t*>(cv) = vw[k];
+        }
+      }
+    }
+    // ---- scores: lane (mrow, kgrp) ends with head mrow, tokens t0 + 4 kgrp + j
+    f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < KS; s++) acc = mfma16<DT>(kw[s], qb[s], acc);
+    load_k(i + NW, blk_next);
+    float x[4], mx = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const int t = t0 + 4 * kgrp + j;
+      float v = acc[j] * a.scale;
+      bool vis = t < t_end && mrow < nh;
+      if (MODE == kMasked && vis) {
+        const int64_t mo = b * a.m_sb + (h0 + mrow) * a.m_sh + t * a.m_st;
+        if (a.mask_mode == 2) {
+          vis = static_cast<const uint8_t*>(a.mask)[mo] != 0;
+        } else {
+          // the mask in the query dtype; keys below its lowest finite value
+          // are skipped (sdpa_vector.h:105-121)
+          const float add = load_as<DT>(a.mask, a.mask_dtype, mo);
+          vis = add >= -E::kMax;
+          v += add;
+        }
+      }
+      x[j] = vis ? v : -INFINITY;
+      mx = fmaxf(mx, x[j]);
+    }
+    if (__builtin_amdgcn_ballot_w64(mx > m_own + kTau)) {
+      // the head's new max over its four lanes, the accumulators rescaled
+      mx = fmaxf(mx, __shfl_xor(mx, 16));
+      mx = fmaxf(mx, __shfl_xor(mx, 32));
+      const float mn = fmaxf(m_own, mx);
+      const float al = __expf(m_own - mn);
+      m_own = mn;
+      l_own *= al;
+#pragma unroll
+      for (int r = 0; r < REP; r++) {
+        const float f = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(al), r));
+#pragma unroll
+        for (int e = 0; e < 8; e++) o[r][e] *= f;
+      }
+    }
+    f32x4_t p;
+#pragma unroll
+    for (int j = 0; j < 4; j++) p[j] = __expf(x[j] - m_own);
+    l_own += (p[0] + p[1]) + (p[2] + p[3]);
+    if (mrow < REP) *reinterpret_cast<f32x4_t*>(&ps_g[wv][mrow][4 * kgrp]) = p;
+    wave_lds_sync();
+    // ---- values: this lane's rows are tokens t0 + NV rs .. + NV
+    float pr[REP][NV];
+#pragma unroll
+    for (int r = 0; r < REP; r++)
+#pragma unroll
+      for (int k = 0; k < NV; k++) pr[r][k] = ps_g[wv][r][NV * rs + k];
+#pragma unroll
+    for (int k = 0; k < NV; k++) {
+      float vv[8];
+      unpack16<DT>(vw[k], vv);
+#pragma unroll
+      for (int r = 0; r < REP; r++)
+#pragma unroll
+        for (int e = 0; e < 8; e++) o[r][e] = fmaf(pr[r][k], vv[e], o[r][e]);
+    }
+    load_v(i + NW, blk_next);
+    if constexpr (PAGED) blk_next = block_of(i + 2 * NW);
+    wave_lds_sync();
+  }
+
+  // ---- the row slots of a run hold disjoint tokens: sum them
+#pragma unroll
+  for (int r = 0; r < REP; r++)
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      if constexpr (LPR <= 8) o[r][e] += swz_xor<8>(o[r][e]);
+      if constexpr (LPR <= 16) o[r][e] += swz_xor<16>(o[r][e]);
+      if constexpr (LPR <= 32) o[r][e] = add_xor32(o[r][e]);
+    }
+  l_own += __shfl_xor(l_own, 16);
+  l_own += __shfl_xor(l_own, 32);
+  // ---- the waves merge in LDS, then every thread takes two dims of a head
+  if (rs == 0) {
+#pragma unroll
+    for (int r = 0; r < REP; r++)
+#pragma unroll
+      for (int e = 0; e < 8; e += 4)
+        *reinterpret_cast<f32x4_t*>(&mo_g[wv][r][8 * dg + e]) =
+            f32x4_t{o[r][e], o[r][e + 1], o[r][e + 2], o[r][e + 3]};
+  }
+  if (lane < REP) {
+    ml_g[wv][lane][0] = m_own;
+    ml_g[wv][lane][1] = l_own;
+  }
+  __syncthreads();
+  const int pairs = nh * (D / 2);
+  for (int idx = threadIdx.x; idx < pairs; idx += 64 * NW) {
+    const int r = idx / (D / 2), d = 2 * (idx % (D / 2)), h = h0 + r;
+    float M = kLowest;
+#pragma unroll
+    for (int w = 0; w < NW; w++) M = fmaxf(M, ml_g[w][r][0]);
+    float den = 0.0f, a0 = 0.0f, a1 = 0.0f;
+#pragma unroll
+    for (int w = 0; w < NW; w++) {
+      const float f = __expf(ml_g[w][r][0] - M);
+      den = fmaf(f, ml_g[w][r][1], den);
+      a0 = fmaf(f, mo_g[w][r][d], a0);
+      a1 = fmaf(f, mo_g[w][r][d + 1], a1);
+    }
+    if (a.n_parts == 1 || (merge_here && np == 1)) {
+      typename E::T* out = static_cast<typename E::T*>(a.out) + b * a.o_sb + h * a.o_sh + d;
+      out[0] = E::from_f32(den > 0.0f ? a0 / den : 0.0f);
+      out[1] = E::from_f32(den > 0.0f ? a1 / den : 0.0f);
+    } else {
+      const int64_t slot = (b * a.Hq + h) * a.n_parts + part;
+      uint64_t* wo = reinterpret_cast<uint64_t*>(a.ws_o + slot * D + d);
+      uint64_t* wm = reinterpret_cast<uint64_t*>(a.ws_ml + slot * 2);
+      __hip_atomic_store(wo, pack_f2(a0, a1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (d == 0)
+        __hip_atomic_store(wm, pack_f2(M, den), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
+  if (a.n_parts == 1 || !merge_here || np == 1) return;
+  // ---- the parts merge in the workgroup that counts in last; every wave's
+  // partial stores are complete before the count
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  uint32_t* cnt = a.counters + (b * a.Hkv + hk) * n_hg + hg;
+  if (threadIdx.x == 0)
+    last_s = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+             static_cast<uint32_t>(np - 1);
+  __syncthreads();
+  if (!last_s) return;
+  if (threadIdx.x == 0) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  for (int idx = threadIdx.x; idx < pairs; idx += 64 * NW) {
+    const int r = idx / (D / 2), d = 2 * (idx % (D / 2)), h = h0 + r;
+    const int64_t slot = (b * a.Hq + h) * a.n_parts;
+    const uint64_t* wo = reinterpret_cast<const uint64_t*>(a.ws_o + slot * D + d);
+    const uint64_t* wm = reinterpret_cast<const uint64_t*>(a.ws_ml + slot * 2);
+    float M = kLowest, den = 0.0f, a0 = 0.0f, a1 = 0.0f;
+    constexpr int kP = 8;  // parts a round trip
+    for (int c = 0; c < np; c += kP) {
+      uint64_t ml[kP], ov[kP];
+#pragma unroll
+      for (int j = 0; j < kP; j++) {
+        const int q = min(c + j, np - 1);  // (clamped parts are selected away)
+        ml[j] = __hip_atomic_load(wm + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        ov[j] = __hip_atomic_load(wo + static_cast<int64_t>(q) * (D / 2), __ATOMIC_RELAXED,
+                                  __HIP_MEMORY_SCOPE_AGENT);
+      }
+      float Mc = M;
+#pragma unroll
+      for (int j = 0; j < kP; j++)
+        if (c + j < np) Mc = fmaxf(Mc, __uint_as_float(static_cast<uint32_t>(ml[j])));
+      const float f0 = __expf(M - Mc);
+      den *= f0;
+      a0 *= f0;
+      a1 *= f0;
+      M = Mc;
+#pragma unroll
+      for (int j = 0; j < kP; j++) {
+        if (c + j < np) {
+          const float f = __expf(__uint_as_float(static_cast<uint32_t>(ml[j])) - M);
+          den = fmaf(f, __uint_as_float(static_cast<uint32_t>(ml[j] >> 32)), den);
+          a0 = fmaf(f, __uint_as_float(static_cast<uint32_t>(ov[j])), a0);
+          a1 = fmaf(f, __uint_as_float(static_cast<uint32_t>(ov[j] >> 32)), a1);
+        }
+      }
+    }
+    typename E::T* out = static_cast<typename E::T*>(a.out) + b * a.o_sb + h * a.o_sh + d;
+    out[0] = E::from_f32(den > 0.0f ? a0 / den : 0.0f);
+    out[1] = E::from_f32(den > 0.0f ? a1 / den : 0.0f);
+  }
+}
+
+// Query heads a wave takes (its head group): all of a kv head's, up to 8,
+// so that each key row is read once for them.
+int fd_group_heads(int Hq, int Hkv) {
+  const int rep = Hq / Hkv;
+  return rep <= 1 ? 1 : rep <= 2 ? 2 : rep <= 4 ? 4 : 8;
+}
+
 template <int DT, int D, int R>
 void launch_r(const AttnArgs& a, int64_t rows, int rep, int n_hg, hipStream_t st) {
   const TimedLaunch tl = timing_prepare(kTimeFDecode);
-  if (a.wg_parts > 0) {
-    // one workgroup per (row, kv head, head group), its parts merged in LDS
-    if constexpr (fd_wg_ok<DT, D, R>()) {
-      constexpr int NW = fd_wg_waves<D, R>();
-      VKV_CHECK(a.wg_parts <= NW && a.n_parts == a.wg_parts, "workgroup parts");
-      const dim3 grid(1, a.Hkv * n_hg, static_cast<unsigned>(rows));
-      hipExtLaunchKernelGGL((fdecode_kernel<DT, D, R, NW>), grid, dim3(64 * NW), 0, st, tl.start,
-                            tl.stop, 0, a, rep);
-    } else {
-      throw Error("no workgroup float decode for this shape");
-    }
+  const dim3 grid(a.n_parts, a.Hkv * n_hg, static_cast<unsigned>(rows));
+  if constexpr (DT == kF32) {
+    hipExtLaunchKernelGGL((fdecode_kernel<DT, D, R>), grid, dim3(64), 0, st, tl.start, tl.stop, 0, a,
+                          rep);
   } else {
-    const dim3 grid(a.n_parts, a.Hkv * n_hg, static_cast<unsigned>(rows));
-    hipExtLaunchKernelGGL((fdecode_kernel<DT, D, R>), grid, dim3(64), 0, st, tl.start, tl.stop, 0,
-                          a, rep);
+    auto run = [&](auto M_) {
+      hipExtLaunchKernelGGL((fdecode16_kernel<DT, D, R, decltype(M_)::value>), grid,
+                            dim3(64 * kWaves16), 0, st, tl.start, tl.stop, 0, a, rep);
+    };
+    if (a.kv.table) run(std::integral_constant<int, kPages>{});
+    else if (a.mask_mode >= 2) run(std::integral_constant<int, kMasked>{});
+    else run(std::integral_constant<int, kDense>{});
   }
   VKV_HIP(hipGetLastError());
   timing_commit(tl);
 }
 
-// Query heads a wave takes (its head group): all of a kv head's, up to 8,
-// so that each key row is read once for them.  The workgroup form of a
-// launch of at most 512 (row, query head)s takes one head a workgroup: the
-// launch then has 4-8x the workgroups, each reading its K/V from L2 (config
-// 1, one row of 8 kv heads x 4: kernel 13.0 us at four heads, 10.2 at one).
-int fd_group_heads(int64_t rows, int Hkv, int rep, bool wg) {
-  if (wg && rows * Hkv * rep <= 512) return 1;
-  return rep <= 1 ? 1 : rep <= 2 ? 2 : rep <= 4 ? 4 : 8;
-}
-
 template <int DT, int D>
 void launch_d(const AttnArgs& a, int64_t rows, hipStream_t st) {
   const int rep = a.Hq / a.Hkv;
-  const int R = fd_group_heads(rows, a.Hkv, rep, a.wg_parts > 0);
+  const int R = fd_group_heads(a.Hq, a.Hkv);
   const int n_hg = (rep + R - 1) / R;
   if (R == 1) launch_r<DT, D, 1>(a, rows, rep, n_hg, st);
   else if (R == 2) launch_r<DT, D, 2>(a, rows, rep, n_hg, st);
@@ -670,59 +844,60 @@ void launch_dt(const AttnArgs& a, int64_t rows, hipStream_t st) {
 }  // namespace
 
 bool fdecode_supported(int dtype, int bits, bool qsem, const AttnArgs& a) {
-  if (bits != 0 || qsem || a.L != 1 || a.kv.table || a.kv.qfmt || a.kv.seq_lens) return false;
+  if (bits != 0 || qsem || a.L != 1 || a.kv.qfmt) return false;
   if (a.D != a.Dv || (a.D != 64 && a.D != 128 && a.D != 256)) return false;
   if (a.Hq % a.Hkv) return false;
   if (a.mask_mode < 0 || a.mask_mode > 3) return false;
-  // f32 rows at 128 dims with more than 4 query heads a kv head, or at 256
-  // dims with more than 2, need more registers than a wave has (the step's
-  // f32 key and value rows beside the group's accumulators): those variants
-  // spill hundreds of registers to scratch and ran 1.9-4.7x slower than the
-  // generic kernel, which therefore takes them
   const int rep = a.Hq / a.Hkv;
-  if (dtype == kF32 && ((a.D == 128 && rep > 4) || (a.D == 256 && rep > 2))) return false;
-  const int es = elem_bytes(dtype);
+  if (dtype == kF32) {
+    // dense rows of one length; f32 rows at 128 dims with more than 4 query
+    // heads a kv head, or at 256 dims with more than 2, need more registers
+    // than a wave has (the step's f32 key and value rows beside the group's
+    // accumulators): those variants spill hundreds of registers to scratch
+    // and ran 1.9-4.7x slower than the generic kernel, which therefore takes
+    // them
+    if (a.kv.table || a.kv.seq_lens) return false;
+    if ((a.D == 128 && rep > 4) || (a.D == 256 && rep > 2)) return false;
+  } else {
+    // a step's rows lie in one page, and within a 32-bit buffer
+    if (a.kv.table && (a.kv.block_size < kStep16 || a.kv.block_size % kStep16 || a.mask_mode >= 2))
+      return false;
+    for (const Comp* c : {&a.kv.kc, &a.kv.vc})
+      if (c->st < 2 * a.D || c->st >= (int64_t{1} << 26)) return false;
+    if (static_cast<int64_t>(a.Hkv) * rep > 65535) return false;
+  }
   // 16-byte loads of key and value rows
   auto al = [](const void* p, int64_t s0, int64_t s1, int64_t s2) {
     return reinterpret_cast<uintptr_t>(p) % 16 == 0 && s0 % 16 == 0 && s1 % 16 == 0 && s2 % 16 == 0;
   };
-  (void)es;
   return al(a.kv.kc.ptr, a.kv.kc.sb, a.kv.kc.sh, a.kv.kc.st) &&
          al(a.kv.vc.ptr, a.kv.vc.sb, a.kv.vc.sh, a.kv.vc.st);
 }
 
-int fdecode_parts(int64_t rows_x_heads, int64_t T, int32_t* part_tokens, int waves) {
-  // about `waves` (default 2048) waves, kStep-token steps
-  if (waves <= 0) waves = 2048;
-  int64_t parts = std::max<int64_t>(1, waves / std::max<int64_t>(1, rows_x_heads));
-  parts = std::min<int64_t>(parts, std::max<int64_t>(1, (T + kStep - 1) / kStep));
+int fdecode_parts(int dtype, int64_t rows, int Hq, int Hkv, int64_t T, int D, int32_t* part_tokens,
+                  int waves) {
+  int64_t parts, step;
+  if (dtype == kF32) {
+    // about `waves` (default 2048) one-wave workgroups
+    step = kStep;
+    parts = (waves > 0 ? waves : 2048) / std::max<int64_t>(1, rows * Hkv);
+    parts = std::min<int64_t>(parts, (T + step - 1) / step);
+  } else {
+    // two workgroups a CU, each of at least one step a wave (8 x 6001 tokens:
+    // 256, 512, 1024, 2048 workgroups 39.3, 40.2, 44.7, 54.8 us; pages of 16
+    // rows to 4096 tokens 46.1, 47.5, 53.1, 60.7: a workgroup's fixed chain
+    // is ~5 us)
+    const int R = fd_group_heads(Hq, Hkv);
+    const int64_t groups = rows * Hkv * ((Hq / Hkv + R - 1) / R);
+    step = kStep16;
+    parts = (waves > 0 ? waves / kWaves16 : 512) / std::max<int64_t>(1, groups);
+    parts = std::min<int64_t>(parts, (T + step * kWaves16 - 1) / (step * kWaves16));
+  }
+  parts = std::max<int64_t>(1, parts);
   int64_t pt = (T + parts - 1) / parts;
-  pt = std::max<int64_t>(kStep, (pt + kStep - 1) / kStep * kStep);
+  pt = std::max<int64_t>(step, (pt + step - 1) / step * step);
   *part_tokens = static_cast<int32_t>(pt);
   return static_cast<int>(std::max<int64_t>(1, (T + pt - 1) / pt));
-}
-
-int fdecode_wg_parts(int64_t rows, int Hq, int Hkv, int64_t T, int D, int dtype,
-                     int32_t* part_tokens) {
-  // launches of at most kWgBytes of K/V: few (row, head group)s whose parts
-  // the global merge would cost more than they save
-  constexpr int64_t kWgBytes = int64_t{8} << 20;
-  if (rows * Hkv * T * D * 2 * elem_bytes(dtype) > kWgBytes) return 0;
-  const int R = fd_group_heads(rows, Hkv, Hq / Hkv, true);
-  if (dtype == kF32 || !(D == 64 || (D == 128 && R <= 4))) return 0;  // fd_wg_ok
-  int nw = 8;
-  switch (D * 8 + R) {  // fd_wg_waves<D, R>()
-#define VKV_WG(DD, RR) case DD * 8 + RR: nw = fd_wg_waves<DD, RR>(); break;
-    VKV_WG(64, 1) VKV_WG(64, 2) VKV_WG(64, 4) VKV_WG(64, 8)
-    VKV_WG(128, 1) VKV_WG(128, 2) VKV_WG(128, 4)
-#undef VKV_WG
-    default: return 0;
-  }
-  const int64_t steps = std::max<int64_t>(1, (T + kStep - 1) / kStep);
-  const int64_t parts = std::min<int64_t>(nw, steps);
-  const int64_t pt = (steps + parts - 1) / parts * kStep;
-  *part_tokens = static_cast<int32_t>(pt);
-  return static_cast<int>((std::max<int64_t>(T, 1) + pt - 1) / pt);
 }
 
 void launch_fdecode(int dtype, const AttnArgs& a, int64_t rows, hipStream_t st) {
@@ -730,29 +905,32 @@ void launch_fdecode(int dtype, const AttnArgs& a, int64_t rows, hipStream_t st) 
   // a causal mask leaves one query token every key
   AttnArgs b = a;
   if (b.mask_mode == 1) b.mask_mode = 0;
+  if (b.kv.table) {
+    // t / block_size = mulhi(t, bs_mul) >> bs_sh for t < 2^31
+    int sh = 0;
+    while ((int64_t{1} << sh) < b.kv.block_size) sh++;
+    b.bs_mul = static_cast<uint32_t>((uint64_t{1} << (31 + sh)) / b.kv.block_size + 1);
+    b.bs_sh = sh - 1;
+  }
   switch (dtype) {
     case kF32: launch_dt<kF32>(b, rows, st); break;
     case kF16: launch_dt<kF16>(b, rows, st); break;
     case kBF16: launch_dt<kBF16>(b, rows, st); break;
     default: throw Error("unsupported dtype");
   }
-  if (b.n_parts > 1 && !b.counters && b.wg_parts == 0) launch_attn_combine(dtype, b, rows, st);
-}
-
-static int fdecode_heads_per_group(int Hq, int Hkv) {
-  const int rep = Hq / Hkv;
-  return rep <= 1 ? 1 : rep <= 2 ? 2 : rep <= 4 ? 4 : 8;
+  if (b.n_parts > 1 && !b.counters) launch_attn_combine(dtype, b, rows, st);
 }
 
 int fdecode_counter_count(int Hq, int Hkv) {
-  const int rep = Hq / Hkv, R = fdecode_heads_per_group(Hq, Hkv);
+  const int rep = Hq / Hkv, R = fd_group_heads(Hq, Hkv);
   return Hkv * ((rep + R - 1) / R);
 }
 
-bool fdecode_merge_here(int n_parts, int Dv, int Hq, int Hkv) {
+bool fdecode_merge_here(int dtype, int n_parts, int Dv, int Hq, int Hkv) {
+  if (dtype != kF32) return true;  // the whole workgroup merges
   // partial floats the last part of a head group reads back
   constexpr int64_t kMaxMergeFloats = 12288;
-  return static_cast<int64_t>(n_parts) * Dv * fdecode_heads_per_group(Hq, Hkv) <= kMaxMergeFloats;
+  return static_cast<int64_t>(n_parts) * Dv * fd_group_heads(Hq, Hkv) <= kMaxMergeFloats;
 }
 
 }  // namespace vkv

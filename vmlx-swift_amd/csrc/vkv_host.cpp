@@ -1460,20 +1460,22 @@ void Pool::append(int layer, const vkv_array& k, const vkv_array* v, const int32
     return;
   }
   const int passes = keys_only ? 1 : 2;
+  RowSrc src[2];
+  RowDst dst[2];
   for (int which = 0; which < passes; which++) {
     const vkv_array& a = which ? *v : k;
-    RowSrc src{a.data, 1, n, a.shape[1], 0, a.strides[0], a.strides[1]};
-    RowDst dst = affine_dst(base, block_bytes, head_bytes, p.block_size, L, which,
+    src[which] = RowSrc{a.data, 1, n, a.shape[1], 0, a.strides[0], a.strides[1]};
+    dst[which] = affine_dst(base, block_bytes, head_bytes, p.block_size, L, which,
                             p.bits ? p.head_dim / p.group_size : 0, keys_only);
-    dst.slots = slots;
-    dst.slot_limit = static_cast<int64_t>(p.num_blocks) * p.block_size;
-    if (p.bits == 0) {
-      launch_copy_rows(p.dtype, 1, src, dst, n * a.shape[1], static_cast<int>(a.shape[2]), st);
-    } else {
-      launch_quantize_rows(p.dtype, p.bits, p.group_size, 1, src, dst, n * a.shape[1],
+    dst[which].slots = slots;
+    dst[which].slot_limit = static_cast<int64_t>(p.num_blocks) * p.block_size;
+    if (p.bits)
+      launch_quantize_rows(p.dtype, p.bits, p.group_size, 1, src[which], dst[which], n * a.shape[1],
                            static_cast<int>(a.shape[2]), st);
-    }
   }
+  if (!p.bits)
+    launch_append_rows(p.dtype, src[0], src[1], dst[0], dst[1], n, k.shape[1],
+                       static_cast<int>(k.shape[2]), static_cast<int>(v->shape[2]), st);
 }
 
 KVSrc kvsrc_from_view(const vkv_paged_view& v) {
@@ -1950,6 +1952,18 @@ WsKey ws_key(hipStream_t st) {
   return {dev, st};
 }
 }  // namespace
+
+bool attention_scratch_ready(hipStream_t st, size_t floats, size_t counters) {
+  {
+    std::lock_guard<std::mutex> g(ws_mutex());
+    const StreamWorkspace& w = ws_map()[ws_key(st)];
+    if (w.cur.size() >= floats * sizeof(float) && w.counters.size() >= counters * sizeof(uint32_t))
+      return true;
+  }
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  VKV_HIP(hipStreamIsCapturing(st, &cs));
+  return cs == hipStreamCaptureStatusNone;
+}
 
 float* attention_workspace(hipStream_t st, size_t floats) {
   std::lock_guard<std::mutex> g(ws_mutex());

@@ -405,6 +405,9 @@ class PrefixManager {
 // them) until workspace_release(st), which frees them all and returns the
 // bytes released.  Growth during graph capture on `st` is an error.
 float* attention_workspace(hipStream_t st, size_t floats);
+// Whether the workspace and counters of a stream hold that much or may grow
+// (a stream under capture may not).
+bool attention_scratch_ready(hipStream_t st, size_t floats, size_t counters);
 // At least n zeroed uint32 counters of the stream, for kernels that count
 // arrivals and zero their counters again before they end (zeroed once, on
 // the stream, when the buffer is allocated or grown; growth during HIP

@@ -115,6 +115,9 @@ struct AttnArgs {
   const uint8_t* nk_ptr;
   const uint8_t* nv_ptr;
   int64_t nk_sb, nk_sh, nv_sb, nv_sh;
+  // float decode over pages: the page size's divisor (set by the launch)
+  uint32_t bs_mul;
+  int32_t bs_sh;
   // float decode only: one zeroed counter per (batch row, kv head, head
   // group); non-null merges the split partials inside the decode launch
   // (the last part of a row merges, then zeroes its counter again)
@@ -127,9 +130,6 @@ struct AttnArgs {
   uint8_t* mrow;
   uint8_t* mcls;
   int64_t mw_words, mw_b, mw_h;
-  // float decode only: > 0 = the launch is one workgroup of wg_parts waves
-  // per (row, kv head, head group) (n_parts == wg_parts), merged in LDS
-  int32_t wg_parts;
 };
 
 // Quantized attention with the reference's arithmetic (vkv_refattn.hip):
@@ -162,8 +162,10 @@ void launch_ref_softmax_bf16(uint16_t* sc, int64_t rows, int64_t tpad, const int
 // ---- launchers (vkv_kernels.hip) ----
 void launch_quantize_rows(int dtype, int bits, int group, int mode, const RowSrc& src,
                           const RowDst& dst, int64_t rows, int D, hipStream_t st);
-void launch_copy_rows(int dtype, int mode, const RowSrc& src, const RowDst& dst, int64_t rows,
-                      int D, hipStream_t st);
+// Float rows of ntok tokens x H heads of K and V into a pool's pages (explicit
+// slots; rows of the sources are (token, head)), one launch.
+void launch_append_rows(int dtype, const RowSrc& sk, const RowSrc& sv, const RowDst& dk,
+                        const RowDst& dv, int64_t ntok, int64_t H, int Dk, int Dv, hipStream_t st);
 // Paged append of ntok tokens x H heads of K (and V when with_v) in one
 // launch; rows of the sources are (token, head), D = head dim of both.
 bool append_affine_supported(int bits, int group, int D);
@@ -205,10 +207,6 @@ void launch_attention(int dtype, int bits, int group, bool quant_semantics,
                       const AttnArgs& a, int64_t rows, hipStream_t st);
 // The split-K merge of launch_attention's partials (a.n_parts > 1).
 void launch_attn_combine(int dtype, const AttnArgs& a, int64_t rows, hipStream_t st);
-// One-token decode over dense float K/V (vkv_fdecode.hip): whether a call
-// qualifies (float, L = 1, dense, D = Dv in {64, 128, 256}, 16-byte aligned
-// rows), its token split (about 2048 waves, 64-token steps), and the launch
-// (with the merge when a.n_parts > 1).
 // Multi-query attention (L >= 2) over dense bf16 / f16 K/V, D = 64, 128 or
 // 256, no, causal or bool array mask, on matrix cores (vkv_prefill.hip).  A
 // bool array is packed first (launch_prefill_mask, into prefill_mask_floats
@@ -222,16 +220,19 @@ bool prefill_mask_fits(const AttnArgs& a, int64_t batch);
 size_t prefill_mask_floats(const AttnArgs& a, int64_t batch);
 void prefill_mask_parts(const AttnArgs& a, int64_t T, int32_t* part_tokens, int32_t* n_parts);
 void launch_prefill_mask(AttnArgs& a, int64_t batch, float* ws, hipStream_t st);
+// One-token decode over float K/V (vkv_fdecode.hip): whether a call
+// qualifies (float, L = 1, D = Dv in {64, 128, 256}, 16-byte aligned rows;
+// bf16 / f16 also over float pages and rows of unequal length), its token
+// split (fdecode_waves > 0 overrides the waves aimed for), and the launch
+// (with the merge when a.n_parts > 1).
 bool fdecode_supported(int dtype, int bits, bool qsem, const AttnArgs& a);
-int fdecode_parts(int64_t rows_x_heads, int64_t T, int32_t* part_tokens, int waves);
+int fdecode_parts(int dtype, int64_t rows, int Hq, int Hkv, int64_t T, int D, int32_t* part_tokens,
+                  int waves);
 void launch_fdecode(int dtype, const AttnArgs& a, int64_t rows, hipStream_t st);
 // counters per batch row the float decode's in-launch merge uses, and
-// whether a launch merges inside (a small merge) or in attn_combine_kernel
+// whether a launch merges inside or in attn_combine_kernel
 int fdecode_counter_count(int Hq, int Hkv);
-bool fdecode_merge_here(int n_parts, int Dv, int Hq, int Hkv);
-// parts of a workgroup-per-row launch (0: not a small launch), and their tokens
-int fdecode_wg_parts(int64_t rows, int Hq, int Hkv, int64_t T, int D, int dtype,
-                     int32_t* part_tokens);
+bool fdecode_merge_here(int dtype, int n_parts, int Dv, int Hq, int Hkv);
 // MFMA decode attention over paged affine bf16 KV (vkv_decode.hip).
 struct DecodeArgs {
   const uint16_t* q;         // [n_seqs][Hq][D] bf16 / f16

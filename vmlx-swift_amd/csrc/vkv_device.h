@@ -5,6 +5,8 @@
 #include <hip/hip_fp16.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace vkv {
 
 enum DType { kF32 = 0, kF16 = 1, kBF16 = 2 };
@@ -133,6 +135,14 @@ __device__ __forceinline__ uint64_t pack_f2(float lo, float hi) {
   return static_cast<uint64_t>(__float_as_uint(lo)) | (static_cast<uint64_t>(__float_as_uint(hi)) << 32);
 }
 
+// Quotient of non-negative indices, in 32 bits where both fit (a 64-bit
+// division is ~100 instructions).
+__device__ __forceinline__ int64_t index_div(int64_t a, int64_t b) {
+  if (__builtin_expect(((a | b) >> 31) == 0, 1))
+    return static_cast<uint32_t>(a) / static_cast<uint32_t>(b);
+  return a / b;
+}
+
 __device__ __forceinline__ float wave_max(float v, int width) {
   for (int o = width / 2; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, width));
   return v;
@@ -156,10 +166,37 @@ __device__ __forceinline__ float wave_sum(float v, int width) {
 //   (:2436-2443);
 //   code = min(round((w - bias) / scale), n_bins) with the unrounded scale
 //   (:2458); the caller stores scale and bias rounded to T (:2447-2450).
+//
+// The 8 divisions by one scale are products with its correctly rounded
+// reciprocal and two correction steps: the first makes the quotient
+// faithful, the second then correctly rounded (P. Markstein, IBM J. Res.
+// Dev. 34, 1990), so the codes are the division's (no difference in 2.2e9
+// random and near-tie cases).  The theorem leaves out a divisor whose
+// mantissa is all ones, and the steps a scale so large or small that they
+// could overflow or lose bits: a wave holding such a group divides.
+// round(q) of q >= 0 is trunc(q + pred(1/2)); the bounds are applied before
+// the conversion.  About 9 instructions a value instead of 22: the vector
+// ALUs bound a large append (see append_affine_kernel).
+template <int TEAM>
+__device__ __forceinline__ float team_max(float v) {
+  // partners 1 and 2 lanes apart by quad permutes, then the mirror images
+  // within 8 and 16 lanes (whose quads hold equal values by then)
+  auto mov = [](float x, auto C) {
+    return __int_as_float(
+        __builtin_amdgcn_update_dpp(0, __float_as_int(x), decltype(C)::value, 0xF, 0xF, true));
+  };
+  v = fmaxf(v, mov(v, std::integral_constant<int, 0xB1>{}));
+  v = fmaxf(v, mov(v, std::integral_constant<int, 0x4E>{}));
+  if constexpr (TEAM >= 8) v = fmaxf(v, mov(v, std::integral_constant<int, 0x141>{}));
+  if constexpr (TEAM >= 16) v = fmaxf(v, mov(v, std::integral_constant<int, 0x140>{}));
+  return v;
+}
+
 template <int DT, int BITS, int GROUP>
 __device__ __forceinline__ void affine_quantize8(const float (&v)[8], uint32_t (&code)[8],
                                                  float& scale_out, float& bias_out) {
   constexpr int TEAM = GROUP / 8;
+  static_assert(TEAM == 4 || TEAM == 8 || TEAM == 16, "groups of 32, 64 or 128");
   constexpr float n_bins = static_cast<float>((1 << BITS) - 1);
   float w_min = Elem<DT>::kMax, w_max = 0.0f;
 #pragma unroll
@@ -167,8 +204,8 @@ __device__ __forceinline__ void affine_quantize8(const float (&v)[8], uint32_t (
     w_min = fminf(w_min, v[e]);
     w_max = fmaxf(w_max, v[e]);
   }
-  w_min = wave_min(w_min, TEAM);
-  w_max = wave_max(w_max, TEAM);
+  w_min = -team_max<TEAM>(-w_min);
+  w_max = team_max<TEAM>(w_max);
   float scale = fmaxf((w_max - w_min) / n_bins, 1e-7f);
   const bool side = fabsf(w_min) > fabsf(w_max);
   scale = side ? scale : -scale;
@@ -177,10 +214,24 @@ __device__ __forceinline__ void affine_quantize8(const float (&v)[8], uint32_t (
   const bool at_zero = q0 == 0.0f;
   scale = at_zero ? scale : edge / q0;
   const float bias = at_zero ? 0.0f : edge;
+  const float mag = fabsf(scale);
+  const bool fast = mag > 1e-30f && mag < 1e30f && (__float_as_uint(scale) & 0x7fffffu) != 0x7fffffu;
+  if (__builtin_amdgcn_ballot_w64(!fast) == 0) {
+    const float inv = 1.0f / scale;
 #pragma unroll
-  for (int e = 0; e < 8; e++) {
-    const float x = fminf(roundf((v[e] - bias) / scale), n_bins);
-    code[e] = x > 0.0f ? static_cast<uint32_t>(x) : 0u;
+    for (int e = 0; e < 8; e++) {
+      const float x = v[e] - bias;
+      float q = x * inv;
+      q = fmaf(fmaf(-q, scale, x), inv, q);
+      q = fmaf(fmaf(-q, scale, x), inv, q);
+      code[e] = static_cast<uint32_t>(fmaxf(fminf(q + 0.49999997f, n_bins), 0.0f));
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      const float x = fminf(roundf((v[e] - bias) / scale), n_bins);
+      code[e] = x > 0.0f ? static_cast<uint32_t>(x) : 0u;
+    }
   }
   scale_out = scale;
   bias_out = bias;

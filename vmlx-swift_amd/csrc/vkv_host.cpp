@@ -280,21 +280,7 @@ std::unique_ptr<Cache> SimpleCache::to_quantized(int group, int bits, hipStream_
     q->reserve(k_.B, k_.H, k_.D, offset, k_.dtype, st);
     if (v_.D != k_.D) throw Error("toQuantized needs equal key and value head dims");
     if (offset > k_.cap) throw Error("toQuantized: offset is past the cached tokens");
-    vkv_array kv[2] = {k_.view(offset), v_.view(offset)};
-    for (int which = 0; which < 2; which++) {
-      const vkv_array& a = kv[which];
-      RowSrc src{a.data, a.shape[0], a.shape[2], a.shape[1], a.strides[0], a.strides[2], a.strides[1]};
-      ChunkLayout L = chunk_layout(bits, a.dtype, QuantizedCache::kBlock, static_cast<int>(q->D_),
-                                   static_cast<int>(q->D_), group, false);
-      RowDst dst = affine_dst(q->store_.bytes(), q->block_bytes_, q->head_bytes_,
-                              QuantizedCache::kBlock, L, which, static_cast<int>(q->D_) / group, false);
-      dst.table = static_cast<const int32_t*>(q->table_.get());
-      dst.table_stride = static_cast<int32_t>(q->nblk_);
-      dst.seq_S = static_cast<int32_t>(offset);
-      dst.start = 0;
-      launch_quantize_rows(a.dtype, bits, group, 1, src, dst, a.shape[0] * a.shape[1] * a.shape[2],
-                           static_cast<int>(a.shape[3]), st);
-    }
+    q->write_tokens(k_.view(offset), v_.view(offset), 0, st);
   }
   return base;
 }
@@ -1113,7 +1099,7 @@ void QuantizedCache::write_tokens(const vkv_array& k, const vkv_array& v, int64_
   const vkv_array* arr[2] = {&k, &v};
   ChunkLayout L = chunk_layout(bits_, dtype_, kBlock, static_cast<int>(D_), static_cast<int>(D_), group_,
                                false);
-  if (append_affine_supported(bits_, group_, static_cast<int>(D_))) {
+  if (append_affine_supported(bits_, group_, static_cast<int>(D_)) && k.dtype == v.dtype) {
     // K and V in one launch; a chunk of whole 8-token groups writes its
     // 4-bit V words with plain stores instead of per-nibble atomics
     const int G = static_cast<int>(D_ / group_);

@@ -20,11 +20,25 @@ namespace vkv {
 // ----------------------------------------------------------------- helpers
 
 __device__ __forceinline__ const uint8_t* row_ptr(const RowSrc& s, int64_t row, int esize) {
-  int64_t i2 = row % s.e2;
-  int64_t r1 = row / s.e2;
-  int64_t i1 = r1 % s.e1;
-  int64_t i0 = r1 / s.e1;
+  const int64_t r1 = index_div(row, s.e2), i0 = index_div(r1, s.e1);
+  const int64_t i2 = row - r1 * s.e2, i1 = r1 - i0 * s.e1;
   return static_cast<const uint8_t*>(s.ptr) + (i0 * s.s0 + i1 * s.s1 + i2 * s.s2) * esize;
+}
+
+// Quotients by a fixed divisor: x / n = mulhi(x, mul) >> (sh - 1) for x <
+// 2^31, with mul = 2^(31 + sh) / n + 1 and 2^sh >= n.
+struct FastDiv {
+  uint32_t n, mul, sh;
+  __device__ __forceinline__ uint32_t quot(uint32_t x) const {
+    return n == 1 ? x : __umulhi(x, mul) >> (sh - 1);
+  }
+};
+static FastDiv fast_div(int64_t n) {
+  FastDiv f{};
+  f.n = static_cast<uint32_t>(n);
+  while ((int64_t{1} << f.sh) < n) f.sh++;
+  f.mul = static_cast<uint32_t>((uint64_t{1} << (31 + f.sh)) / static_cast<uint64_t>(n) + 1);
+  return f;
 }
 
 // Slot (block * block_size + offset) of paged token n; < 0 means skip (so
@@ -34,19 +48,20 @@ __device__ __forceinline__ int64_t token_slot(const RowDst& d, int64_t n) {
     const int64_t s = d.slots[n];
     return (d.slot_limit > 0 && s >= d.slot_limit) ? -1 : s;
   }
-  int64_t b = n / d.seq_S;
-  int64_t pos = d.start + n % d.seq_S;
-  int32_t blk = d.table[b * d.table_stride + pos / d.block_size];
+  const int64_t b = index_div(n, d.seq_S);
+  const int64_t pos = d.start + (n - b * d.seq_S), pb = index_div(pos, d.block_size);
+  const int32_t blk = d.table[b * d.table_stride + pb];
   if (blk < 0) return -1;
-  return static_cast<int64_t>(blk) * d.block_size + pos % d.block_size;
+  return static_cast<int64_t>(blk) * d.block_size + (pos - pb * d.block_size);
 }
 
 template <int DT>
 __device__ __forceinline__ void load8(const uint8_t* p, float* v) {
   using E = Elem<DT>;
-  const typename E::T* q = reinterpret_cast<const typename E::T*>(p);
+  typename E::T q[8];  // (16-byte loads at any element alignment)
+  __builtin_memcpy(q, p, sizeof(q));
 #pragma unroll
-  for (int i = 0; i < 8; i++) v[i] = E::load(q + i);
+  for (int i = 0; i < 8; i++) v[i] = E::to_f32(q[i]);
 }
 
 // Store the 8 codes of dims [8j, 8j+8) of token `tib` into a paged chunk
@@ -100,8 +115,8 @@ __global__ void __launch_bounds__(256) quantize_rows_kernel(RowSrc src, RowDst d
   constexpr int TEAM = GROUP / 8;
   const int tpr = D / 8;
   const int64_t gtid = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  const int64_t row = gtid / tpr;
-  const int j = static_cast<int>(gtid % tpr);
+  const int64_t row = index_div(gtid, tpr);
+  const int j = static_cast<int>(gtid - row * tpr);
   const bool active = row < rows;
 
   float v[8];
@@ -139,12 +154,12 @@ __global__ void __launch_bounds__(256) quantize_rows_kernel(RowSrc src, RowDst d
       static_cast<typename E::T*>(dst.biases)[row * G + g] = b_t;
     }
   } else {
-    const int64_t n = row / src.e2;
-    const int64_t h = row % src.e2;
+    const int64_t n = index_div(row, src.e2);
+    const int64_t h = row - n * src.e2;
     const int64_t slot = token_slot(dst, n);
     if (slot < 0) return;
-    const int64_t blk = slot / dst.block_size;
-    const int tib = static_cast<int>(slot % dst.block_size);
+    const int64_t blk = index_div(slot, dst.block_size);
+    const int tib = static_cast<int>(slot - blk * dst.block_size);
     uint8_t* chunk = dst.base + blk * dst.block_bytes + h * dst.head_bytes;
     store_chunk_codes<BITS>(chunk, dst, tib, j, D, code);
     if (group_leader) {
@@ -158,83 +173,143 @@ __global__ void __launch_bounds__(256) quantize_rows_kernel(RowSrc src, RowDst d
 // Paged append of K and V in one launch (Pool::append): block = 8
 // consecutive tokens x HB heads x the D/8 threads of a row (256 threads);
 // blockIdx.z selects K (0) or V (1).  The arithmetic is that of
-// quantize_rows_kernel.  4-bit V words hold 8 tokens of one dim: when the
-// block's 8 tokens fill exactly one aligned 8-token group of a block (a
-// prefill chunk), the words are assembled in LDS and written with plain
-// stores; otherwise (decode tokens of different sequences, ragged groups)
-// each nibble is merged atomically.
+// quantize_rows_kernel.  V words hold 8 (4-bit) or 4 (8-bit) tokens of one
+// dim; they are assembled from the block's 8 tokens in LDS: whole aligned
+// 8-token groups (a prefill chunk) are plain stores, and of a 4-bit group
+// that the block holds part of, each run of tokens is merged into the word
+// with one pair of atomics (8-bit codes are then stored byte by byte).
+// Bound by the vector ALUs on large appends (affine_quantize8), by the
+// chain slot -> page -> stores on a step's few tokens.  Measured (8 x 4096
+// bf16 tokens x 8 heads x 128, K and V, 172 MB moved): 130 -> 61 us from the
+// divisions by multiplication (values: affine_quantize8; indexes: AppendDiv);
+// 246K tokens of which no group of 8 starts on a page boundary, 5.2 -> 0.7 ms
+// from one atomic pair a run instead of one a nibble.
+// Tokens and positions are below 2^31 and divide by multiplication (dv).
+struct AppendDiv {
+  FastDiv e1;   // tokens of a batch row (the source's, and the table's seq_S)
+  FastDiv bs;   // tokens of a block
+};
+
 template <int DT, int BITS, int GROUP>
 __global__ void __launch_bounds__(256) append_affine_kernel(RowSrc sk, RowSrc sv, RowDst dk, RowDst dv,
-                                                            int64_t ntok, int H, int D) {
+                                                            uint32_t ntok, int H, int D, AppendDiv dq) {
   using E = Elem<DT>;
   constexpr int TEAM = GROUP / 8;
   const int which = blockIdx.z;
-  const RowSrc src = which ? sv : sk;
-  const RowDst dst = which ? dv : dk;
-  const int tpr = D / 8, hb = 256 / (8 * tpr);
+  const RowSrc& src = which ? sv : sk;
+  const RowDst& dst = which ? dv : dk;
+  const int lt = 31 - __builtin_clz(D / 8);  // D = 32 .. 256, a power of two
+  const int tpr = 1 << lt, hb = 32 >> lt;
   const int tid = threadIdx.x;
-  const int i = tid / (hb * tpr), hl = (tid / tpr) % hb, j = tid % tpr;
-  const int64_t n = static_cast<int64_t>(blockIdx.x) * 8 + i;
+  const int i = tid >> 5, hl = (tid >> lt) & (hb - 1), j = tid & (tpr - 1);
+  const uint32_t n = blockIdx.x * 8 + i;
   const int h = blockIdx.y * hb + hl;
   const bool active = n < ntok && h < H;
-  // the token's slot (a block-table read) goes out with the row's load
-  const int64_t slot = active ? token_slot(dst, n) : -1;
+  const uint32_t i0 = dq.e1.quot(n), i1 = n - i0 * static_cast<uint32_t>(src.e1);
 
+  // the token's block and place in it (-1: skipped); its read goes out with
+  // the row's load
+  int blk = -1, tib = 0;
   float v[8];
-  if (active) {
-    load8<DT>(row_ptr(src, n * H + h, E::kBytes) + static_cast<int64_t>(j) * 8 * E::kBytes, v);
-  } else {
 #pragma unroll
-    for (int e = 0; e < 8; e++) v[e] = 0.0f;
+  for (int e = 0; e < 8; e++) v[e] = 0.0f;
+  if (active) {
+    uint32_t pos;
+    int32_t at;
+    if (dst.slots) {
+      at = dst.slots[n];
+    } else {
+      pos = dst.start + i1;
+      const uint32_t pb = dq.bs.quot(pos);
+      tib = static_cast<int>(pos - pb * static_cast<uint32_t>(dst.block_size));
+      at = dst.table[static_cast<int64_t>(i0) * dst.table_stride + pb];
+    }
+    load8<DT>(static_cast<const uint8_t*>(src.ptr) +
+                  (i0 * src.s0 + i1 * src.s1 + h * src.s2 + 8 * j) * E::kBytes,
+              v);
+    blk = at;
+    if (dst.slots && at >= 0) {
+      blk = static_cast<int>(dq.bs.quot(at));
+      tib = at - blk * dst.block_size;
+      if (dst.slot_limit > 0 && at >= dst.slot_limit) blk = -1;
+    }
   }
   uint32_t code[8];
   float scale, bias;
   affine_quantize8<DT, BITS, GROUP>(v, code, scale, bias);
-  const int g = (j * 8) / GROUP;
-  if (slot >= 0 && (j % TEAM) == 0) {
-    uint8_t* chunk = dst.base + (slot / dst.block_size) * dst.block_bytes + h * dst.head_bytes;
-    const int tib = static_cast<int>(slot % dst.block_size);
+  uint8_t* chunk = dst.base + blk * dst.block_bytes + h * dst.head_bytes;
+  if (blk >= 0 && (j % TEAM) == 0) {
+    const int g = (j * 8) / GROUP;
     typename E::T* sbp = reinterpret_cast<typename E::T*>(chunk + dst.s_off);
     sbp[qsb_index(tib, dst.is_v, g, 0, dst.G, dst.keys_only)] = E::from_f32(scale);
     sbp[qsb_index(tib, dst.is_v, g, 1, dst.G, dst.keys_only)] = E::from_f32(bias);
   }
-  if (BITS == 8 || which == 0) {  // K words and 8-bit V bytes are whole stores
-    if (slot >= 0) {
-      uint8_t* chunk = dst.base + (slot / dst.block_size) * dst.block_bytes + h * dst.head_bytes;
-      store_chunk_codes<BITS>(chunk, dst, static_cast<int>(slot % dst.block_size), j, D, code);
-    }
+  if (which == 0) {  // K words are whole stores
+    if (blk >= 0) store_chunk_codes<BITS>(chunk, dst, tib, j, D, code);
     return;
   }
-  // ---- 4-bit V
-  __shared__ int64_t tok_slot[8];
-  __shared__ uint8_t vcode[8][256];  // [token][head * D + dim], hb * D = 256
-  if (hl == 0 && j == 0) tok_slot[i] = slot;  // hl 0: a head below H, so slot is n's
+  // ---- V
+  __shared__ int2 tok[8];  // block and place of each token
+  __shared__ __attribute__((aligned(8))) uint8_t vcode[8][256];  // [token][head * D + dim], hb * D = 256
+  if (hl == 0 && j == 0) tok[i] = make_int2(blk, tib);  // hl 0: a head below H
+  uint2 c8;
+  c8.x = code[0] | code[1] << 8 | code[2] << 16 | code[3] << 24;
+  c8.y = code[4] | code[5] << 8 | code[6] << 16 | code[7] << 24;
+  *reinterpret_cast<uint2*>(&vcode[i][hl * D + 8 * j]) = c8;
   __syncthreads();
-  const int64_t s0 = tok_slot[0];
-  bool aligned = s0 >= 0 && s0 % 8 == 0;
+  // the 8 tokens are one aligned 8-token group (its block's size is a
+  // multiple of 8)
+  const int2 t0 = tok[0];
+  bool whole = t0.x >= 0 && t0.y % 8 == 0;
 #pragma unroll
-  for (int t = 1; t < 8; t++) aligned = aligned && tok_slot[t] == s0 + t;
-  if (!aligned) {
-    if (slot >= 0) {
-      uint8_t* chunk = dst.base + (slot / dst.block_size) * dst.block_bytes + h * dst.head_bytes;
-      store_chunk_codes<BITS>(chunk, dst, static_cast<int>(slot % dst.block_size), j, D, code);
-    }
+  for (int t = 1; t < 8; t++) whole = whole && tok[t].x == t0.x && tok[t].y == t0.y + t;
+  if (BITS == 8 && !whole) {  // bytes are whole stores
+    if (blk >= 0) store_chunk_codes<BITS>(chunk, dst, tib, j, D, code);
     return;
   }
-#pragma unroll
-  for (int e = 0; e < 8; e++) vcode[i][hl * D + 8 * j + e] = static_cast<uint8_t>(code[e]);
-  __syncthreads();
-  // thread (head hh, dim d) writes the word of the 8 tokens
-  const int hh = tid / D, d = tid % D;
-  if (tid < hb * D && blockIdx.y * hb + hh < H) {
-    uint32_t w = 0;
-#pragma unroll
-    for (int t = 0; t < 8; t++) w |= static_cast<uint32_t>(vcode[t][hh * D + d]) << (4 * t);
-    uint8_t* chunk = dst.base + (s0 / dst.block_size) * dst.block_bytes +
-                     static_cast<int64_t>(blockIdx.y * hb + hh) * dst.head_bytes;
+  // thread (head hh, dim d) writes the words of its dim
+  const int hh = tid >> (lt + 3), d = tid & (D - 1);
+  if (blockIdx.y * hb + hh >= H) return;
+  uint8_t* vbase = dst.base + static_cast<int64_t>(blockIdx.y * hb + hh) * dst.head_bytes + dst.c_off;
+  auto word_at = [&](const int2& p) {
     int sh;
-    const int64_t off = qv_word_off(s0 % dst.block_size, d, D, 4, &sh);
-    *reinterpret_cast<uint32_t*>(chunk + dst.c_off + off) = w;
+    return vbase + p.x * dst.block_bytes + qv_word_off(p.y, d, D, BITS, &sh);
+  };
+  if (whole) {
+    uint2 w = {0, 0};
+#pragma unroll
+    for (int t = 0; t < 8; t++) {
+      if constexpr (BITS == 4)
+        w.x |= static_cast<uint32_t>(vcode[t][tid]) << (4 * t);
+      else
+        (t < 4 ? w.x : w.y) |= static_cast<uint32_t>(vcode[t][tid]) << (8 * (t & 3));
+    }
+    if constexpr (BITS == 4)
+      *reinterpret_cast<uint32_t*>(word_at(t0)) = w.x;
+    else
+      *reinterpret_cast<uint2*>(word_at(t0)) = w;
+    return;
+  }
+  if constexpr (BITS == 4) {
+    // runs of tokens of one group: other tokens' nibbles of a word may be
+    // written concurrently
+    uint32_t w = 0, m = 0;
+    int2 cur = make_int2(-1, 0);
+#pragma unroll 1
+    for (int t = 0; t <= 8; t++) {
+      const int2 p = t < 8 ? tok[t] : make_int2(-1, 0);
+      if (m && (p.x != cur.x || p.y >> 3 != cur.y >> 3)) {
+        uint32_t* at = reinterpret_cast<uint32_t*>(word_at(cur));
+        atomicAnd(at, ~m);
+        atomicOr(at, w);
+        w = m = 0;
+      }
+      if (p.x < 0) continue;
+      cur = p;
+      const int sh = 4 * (p.y & 7);
+      w = (w & ~(15u << sh)) | static_cast<uint32_t>(vcode[t][tid]) << sh;
+      m |= 15u << sh;
+    }
   }
 }
 
@@ -467,6 +542,120 @@ __global__ void __launch_bounds__(256) gather_dequant8_kernel(GatherArgs g) {
   }
 }
 
+// Codes, scales and biases of paged affine chunks in the reference layout.
+// blockIdx.y is the (seq, head) plane.  Keys: a thread writes 4 words of a
+// token's row (the chunk keeps a row's words permuted).  Values: a thread
+// reads the words of 8 dims of an aligned 8-token group (dim-major in the
+// chunk) and transposes them in registers, so every word is read once; lanes
+// take neighbouring words of the chunk, then the two halves of a 16-dim tile.
+// HBM bound: 8 x 4096 tokens x 8 heads x 128 at 4 bits (38 MB read, 38
+// written) take 9.6 us a matrix, 48 with a thread per (token, 8 dims) that
+// read 8 words for 8 nibbles and divided in 64 bits.
+template <int DT, int BITS>
+__global__ void __launch_bounds__(256) gather_codes_kernel(GatherArgs g) {
+  using T = typename Elem<DT>::T;
+  const KVSrc& kv = g.kv;
+  const int plane = blockIdx.y, s = plane / g.H, h = plane - s * g.H;
+  // tokens [t_begin, t_end) of this row
+  const int t_end =
+      min(g.t_begin + g.T, static_cast<int>(kv.seq_lens ? kv.seq_lens[s] : kv.T));
+  const int D = g.D, G = D / g.group, W = D * BITS / 32;
+  const int64_t row0 = static_cast<int64_t>(plane) * (g.out_cap ? g.out_cap : g.T) + g.out_t0 - g.t_begin;
+  uint32_t* wq = static_cast<uint32_t*>(g.out);
+  const int which = g.which, idx = blockIdx.x * 256 + static_cast<int>(threadIdx.x);
+  auto chunk_of = [&](int t, int& tib) {
+    const int b = t / kv.block_size;
+    tib = t - b * kv.block_size;
+    const int64_t blk = kv.table[static_cast<int64_t>(s) * kv.table_stride + b];
+    return kv.base + blk * kv.block_bytes + h * kv.head_bytes;
+  };
+  auto scales = [&](const uint8_t* chunk, int tib, int t, int gi) {
+    const T* sb = reinterpret_cast<const T*>(chunk + kv.sb_off);
+    static_cast<T*>(g.out_s)[(row0 + t) * G + gi] = sb[qsb_index(tib, which, gi, 0, kv.G, kv.keys_only)];
+    static_cast<T*>(g.out_b)[(row0 + t) * G + gi] = sb[qsb_index(tib, which, gi, 1, kv.G, kv.keys_only)];
+  };
+  if (which == 0) {
+    const int per = W / 4, ti = idx / per, q = idx - ti * per, t = g.t_begin + ti;
+    if (t >= t_end) return;
+    int tib;
+    const uint8_t* chunk = chunk_of(t, tib);
+    const uint32_t* row = reinterpret_cast<const uint32_t*>(chunk + kv.kc_off) + static_cast<int64_t>(tib) * W;
+    uint32_t w[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const int o = 4 * q + e, p = BITS == 4 ? o : o >> 1;  // original word; its 8-dim unit
+      const int pos = (p & 3) * (D / 32) + (p >> 2);
+      w[e] = row[BITS == 4 ? pos : 2 * pos + (o & 1)];
+    }
+    uint32_t* o = wq + (row0 + t) * W + 4 * q;
+    *reinterpret_cast<uint4*>(o) = make_uint4(w[0], w[1], w[2], w[3]);
+    for (int gi = q; gi < G; gi += per) scales(chunk, tib, t, gi);
+    return;
+  }
+  // values: 8-token groups counted from the aligned one holding t_begin; a
+  // thread takes dims 16 mt + 8 hf .. + 8, mt fastest
+  const int NT = D / 16, per = D / 8;
+  const int gq = idx / per, r = idx - gq * per, hf = r / NT, mt = r - hf * NT;
+  const int t8 = (g.t_begin & ~7) + 8 * gq;
+  if (t8 >= t_end) return;
+  int tib;
+  const uint8_t* chunk = chunk_of(t8, tib);
+  const uint32_t* vb = reinterpret_cast<const uint32_t*>(chunk + kv.vc_off) +
+                       static_cast<int64_t>(tib >> 5) * (D * BITS / 4);
+  const int kg = (tib & 31) >> 3;
+  uint32_t w[8][BITS / 4];
+#pragma unroll
+  for (int e = 0; e < 8; e++)
+#pragma unroll
+    for (int x = 0; x < BITS / 4; x++)
+      w[e][x] = vb[((kg * 16 + 8 * hf + e) * NT + mt) * (BITS / 4) + x];
+  // w[dim e]: codes of 8 tokens -> token k: codes of 8 dims
+  auto swap = [](uint32_t& a, uint32_t& b, int sh, uint32_t m) __attribute__((always_inline)) {
+    const uint32_t t = ((a >> sh) ^ b) & m;
+    b ^= t;
+    a ^= t << sh;
+  };
+  uint32_t out[8][BITS / 4];
+  if constexpr (BITS == 4) {
+#pragma unroll
+    for (int e = 0; e < 4; e++) swap(w[e][0], w[e + 4][0], 16, 0x0000FFFFu);
+#pragma unroll
+    for (int e = 0; e < 8; e += (e & 1) ? 3 : 1) swap(w[e][0], w[e + 2][0], 8, 0x00FF00FFu);
+#pragma unroll
+    for (int e = 0; e < 8; e += 2) swap(w[e][0], w[e + 1][0], 4, 0x0F0F0F0Fu);
+#pragma unroll
+    for (int k = 0; k < 8; k++) out[k][0] = w[k][0];
+  } else {
+    // two 4 x 4 byte transposes per half of the tokens
+#pragma unroll
+    for (int x = 0; x < 2; x++)
+#pragma unroll
+      for (int y = 0; y < 2; y++) {
+        uint32_t a = w[4 * y][x], b = w[4 * y + 1][x], c = w[4 * y + 2][x], d = w[4 * y + 3][x];
+        swap(a, c, 16, 0x0000FFFFu);
+        swap(b, d, 16, 0x0000FFFFu);
+        swap(a, b, 8, 0x00FF00FFu);
+        swap(c, d, 8, 0x00FF00FFu);
+        out[4 * x][y] = a;
+        out[4 * x + 1][y] = b;
+        out[4 * x + 2][y] = c;
+        out[4 * x + 3][y] = d;
+      }
+  }
+#pragma unroll
+  for (int k = 0; k < 8; k++) {
+    const int t = t8 + k;
+    if (t < g.t_begin || t >= t_end) continue;
+    uint32_t* o = wq + (row0 + t) * W + (2 * mt + hf) * (BITS / 4);
+    if constexpr (BITS == 4) *o = out[k][0];
+    else *reinterpret_cast<uint2*>(o) = make_uint2(out[k][0], out[k][1]);
+  }
+  for (int x = r; x < 8 * G; x += per) {
+    const int k = x / G, t = t8 + k;
+    if (t >= g.t_begin && t < t_end) scales(chunk, tib + k, t, x - k * G);
+  }
+}
+
 // Reference-layout affine rows -> paged chunks (inverse of the code gather).
 template <int ESIZE, int BITS>
 __global__ void __launch_bounds__(256) scatter_codes_kernel(ScatterCodesArgs a) {
@@ -514,20 +703,15 @@ __global__ void __launch_bounds__(256) scatter_codes_kernel(ScatterCodesArgs a) 
 // ------------------------------------------------------------ copy4d
 
 // A strided 4-D copy in units of the widest aligned run (1 to 16 bytes):
-// extents and unit strides, outermost first, and the divisors that turn a
-// unit's index into its coordinates (index < 2^31: mul = 2^(31 + sh) / n + 1
-// with 2^sh >= n, so mulhi >> (sh - 1) is the exact quotient).
+// extents (as divisors that turn a unit's index, below 2^31, into its
+// coordinates) and unit strides, outermost first.
 struct CopyPlan {
   const void* src;
   void* dst;
-  uint32_t total, n[4];
+  uint32_t total;
+  FastDiv n[4];
   int64_t s[4], d[4];
-  uint32_t mul[4], sh[4];
 };
-
-__device__ __forceinline__ uint32_t plan_div(const CopyPlan& p, int k, uint32_t x) {
-  return p.n[k] == 1 ? x : __umulhi(x, p.mul[k]) >> (p.sh[k] - 1);
-}
 
 // Up to two copies in one launch (blockIdx.y picks one: a cache update
 // writes its K and V tokens with one launch), N units a thread, all loaded
@@ -548,8 +732,8 @@ __global__ void __launch_bounds__(256) copy_units_kernel(CopyPlan p0, CopyPlan p
 #pragma unroll
   for (int j = 0; j < N; j++) {
     const uint32_t i = min(i0 + 256u * j, p.total - 1);  // (clamped copies are not stored)
-    const uint32_t r3 = plan_div(p, 3, i), r2 = plan_div(p, 2, r3), r1 = plan_div(p, 1, r2);
-    const int64_t c3 = i - r3 * p.n[3], c2 = r3 - r2 * p.n[2], c1 = r2 - r1 * p.n[1], c0 = r1;
+    const uint32_t r3 = p.n[3].quot(i), r2 = p.n[2].quot(r3), r1 = p.n[1].quot(r2);
+    const int64_t c3 = i - r3 * p.n[3].n, c2 = r3 - r2 * p.n[2].n, c1 = r2 - r1 * p.n[1].n, c0 = r1;
     to[j] = c0 * p.d[0] + c1 * p.d[1] + c2 * p.d[2] + c3 * p.d[3];
     v[j] = src[c0 * p.s[0] + c1 * p.s[1] + c2 * p.s[2] + c3 * p.s[3]];
   }
@@ -954,10 +1138,11 @@ static void append_dispatch(int bits, int group, const RowSrc& sk, const RowSrc&
                             const RowDst& dv, int64_t ntok, int H, int D, bool with_v, hipStream_t st) {
   const int hb = 256 / D;
   const dim3 grid(static_cast<unsigned>((ntok + 7) / 8), (H + hb - 1) / hb, with_v ? 2 : 1);
+  const AppendDiv dq{fast_div(sk.e1), fast_div(dk.block_size)};
   const TimedLaunch tl = timing_prepare(kTimeAppend);
 #define VKV_A(B, G)                                                                            \
   hipExtLaunchKernelGGL((append_affine_kernel<DT, B, G>), grid, dim3(256), 0, st, tl.start, tl.stop, \
-                        0, sk, sv, dk, dv, ntok, H, D)
+                        0, sk, sv, dk, dv, static_cast<uint32_t>(ntok), H, D, dq)
 #define VKV_AG(B)                         \
   do {                                    \
     if (group == 32) VKV_A(B, 32);        \
@@ -982,6 +1167,10 @@ void launch_append_affine(int dtype, int bits, int group, const RowSrc& sk, cons
                           hipStream_t st) {
   if (ntok <= 0) return;
   VKV_CHECK(append_affine_supported(bits, group, D), "append_affine: unsupported geometry");
+  // (a table's batch rows are the source's; both matrices share the tokens)
+  VKV_CHECK(ntok < (int64_t{1} << 31) && sk.e1 > 0 && sv.e1 == sk.e1 &&
+                (dk.slots || (dk.seq_S == sk.e1 && dk.start + sk.e1 < (int64_t{1} << 31))),
+            "append_affine: token range");
   switch (dtype) {
     case kF32: append_dispatch<kF32>(bits, group, sk, sv, dk, dv, ntok, H, D, with_v, st); break;
     case kF16: append_dispatch<kF16>(bits, group, sk, sv, dk, dv, ntok, H, D, with_v, st); break;
@@ -1088,6 +1277,18 @@ static void gather_dispatch_kind(const GatherArgs& g, int out_kind, hipStream_t 
     hipLaunchKernelGGL((gather_kernel<DT, BITS, 0>), dim3(nb), dim3(256), 0, st, g);
   } else {
     if constexpr (BITS > 0) {
+      // paged chunks take whole words; other layouts (tuples, the values of a
+      // keys-only view, outputs off 16 bytes) go code by code
+      const int64_t planes = static_cast<int64_t>(g.n_seqs) * g.H;
+      const int64_t groups = (static_cast<int64_t>(g.T) + (g.t_begin & 7) + 7) / 8;
+      const int64_t threads =
+          g.which ? groups * (g.D / 8) : static_cast<int64_t>(g.T) * (g.D * BITS / 128);
+      if (g.kv.qfmt && g.kv.table && !(g.which && g.kv.keys_only) && g.D == g.kv.D && g.D % 32 == 0 &&
+          planes <= 65535 && threads < (1 << 30) && reinterpret_cast<uintptr_t>(g.out) % 16 == 0) {
+        hipLaunchKernelGGL((gather_codes_kernel<DT, BITS>),
+                           dim3(blocks_for(threads), static_cast<unsigned>(planes)), dim3(256), 0, st, g);
+        return;
+      }
       hipLaunchKernelGGL((gather_kernel<DT, BITS, 1>), dim3(nb), dim3(256), 0, st, g);
     } else {
       throw Error("code gather needs an affine view");
@@ -1176,11 +1377,9 @@ CopyPlan copy_plan(const Copy4D& c, int es, int unit) {
   for (int i = 0; i < 4; i++) {
     const bool inner = i == 3;
     const int64_t n = inner ? c.n[i] / k : c.n[i];
-    p.n[i] = static_cast<uint32_t>(n);
+    p.n[i] = fast_div(n);
     p.s[i] = inner ? c.s[i] : c.s[i] / k;
     p.d[i] = inner ? c.d[i] : c.d[i] / k;
-    while ((uint64_t{1} << p.sh[i]) < static_cast<uint64_t>(n)) p.sh[i]++;
-    p.mul[i] = static_cast<uint32_t>((uint64_t{1} << (31 + p.sh[i])) / static_cast<uint64_t>(n) + 1);
     total *= n;
   }
   p.total = static_cast<uint32_t>(total);

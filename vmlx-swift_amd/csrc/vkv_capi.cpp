@@ -19,6 +19,7 @@ thread_local std::string g_error;
 
 template <class F>
 int guard(F&& f) {
+  CallScope scope;
   try {
     f();
     g_error.clear();

@@ -19,8 +19,31 @@
 
 namespace vkv {
 
-// Owned device allocation.  hipFree synchronizes the device, so a buffer can
-// be dropped while work that reads it is still queued.
+// The stream of the C call a thread is in, set by S(); the scope of a call
+// puts back what the call around it had.
+struct CallStream {
+  hipStream_t stream = nullptr;
+  bool known = false;
+};
+inline thread_local CallStream t_call;
+struct CallScope {
+  CallStream before = t_call;
+  ~CallScope() { t_call = before; }
+};
+
+// Device blocks that objects gave back, kept for the next allocation of about
+// their size (vkv_host.cpp): take() and give() stand in for hipMalloc and
+// hipFree.
+struct DevPool {
+  static void* take(size_t bytes, size_t* cap, int* dev);
+  static void give(void* p, size_t cap, int dev);
+  static void flush();  // frees every kept block of the current device
+};
+
+// Owned device allocation.  A buffer can be dropped while work that reads it
+// is still queued, on any stream: its block is used again only after the
+// device has been waited for since (DevPool), or it goes back by hipFree,
+// which waits.
 class DevBuf {
  public:
   DevBuf() = default;
@@ -28,12 +51,18 @@ class DevBuf {
   ~DevBuf() { release(); }
   DevBuf(const DevBuf&) = delete;
   DevBuf& operator=(const DevBuf&) = delete;
-  DevBuf(DevBuf&& o) noexcept : p_(o.p_), n_(o.n_) { o.p_ = nullptr; o.n_ = 0; }
+  DevBuf(DevBuf&& o) noexcept : p_(o.p_), n_(o.n_), cap_(o.cap_), dev_(o.dev_), direct_(o.direct_) {
+    o.p_ = nullptr;
+    o.n_ = 0;
+  }
   DevBuf& operator=(DevBuf&& o) noexcept {
     if (this != &o) {
       release();
       p_ = o.p_;
       n_ = o.n_;
+      cap_ = o.cap_;
+      dev_ = o.dev_;
+      direct_ = o.direct_;
       o.p_ = nullptr;
       o.n_ = 0;
     }
@@ -41,9 +70,12 @@ class DevBuf {
   }
   void alloc(size_t bytes) {
     release();
-    if (bytes) VKV_HIP(hipMalloc(&p_, bytes));
+    if (bytes && direct_) VKV_HIP(hipMalloc(&p_, bytes));
+    else if (bytes) p_ = DevPool::take(bytes, &cap_, &dev_);
     n_ = bytes;
   }
+  // Allocate and free at the device, not through the pool.
+  void set_direct() { direct_ = true; }
   // Grow to at least `bytes` (contents are not kept); a buffer that is
   // large enough stays where it is, so views into it and work already
   // queued on it keep their address, and no hipFree stalls the device.
@@ -51,7 +83,8 @@ class DevBuf {
     if (bytes > n_) alloc(bytes);
   }
   void release() {
-    if (p_) (void)hipFree(p_);
+    if (p_ && direct_) (void)hipFree(p_);
+    else if (p_) DevPool::give(p_, cap_, dev_);
     p_ = nullptr;
     n_ = 0;
   }
@@ -62,9 +95,15 @@ class DevBuf {
  private:
   void* p_ = nullptr;
   size_t n_ = 0;
+  size_t cap_ = 0;  // the block's bytes
+  int dev_ = 0;
+  bool direct_ = false;
 };
 
-inline hipStream_t S(void* s) { return static_cast<hipStream_t>(s); }
+inline hipStream_t S(void* s) {
+  t_call = {static_cast<hipStream_t>(s), true};
+  return t_call.stream;
+}
 
 // A dense [B,H,cap,D] float buffer with the reference's 4-D array semantics.
 struct Dense4 {

@@ -388,6 +388,20 @@ struct TqDecodeArgs {
   int32_t out_dtype, t0;
   int64_t osb, osh, ost;
 };
+// Exact tokens of a unified buffer [B, H, cap, D]: n_sink from 0, n_tail from
+// tail_at (contiguous sources [B, H, n, D]), n_zero zeros from zero_at.
+struct TqExactArgs {
+  void* out;
+  int64_t row_elems;  // cap * D
+  int32_t dtype, D;
+  const void* sink;
+  const void* tail;
+  int32_t sink_dtype, tail_dtype;
+  int32_t n_sink, n_tail, tail_at, n_zero, zero_at;
+};
+void launch_tq_exact(const TqExactArgs& a, int64_t bh, hipStream_t st);
+bool tq_encode_needs_zero_codes(const TqEncodeArgs& a);
+bool tq_encode_needs_zero_signs(const TqEncodeArgs& a);
 void launch_tq_encode(const TqEncodeArgs& a, hipStream_t st);
 void launch_tq_decode(const TqDecodeArgs& a, hipStream_t st);
 // Zeros in `rows` runs of run_bytes, pitch_bytes apart (2-byte units).

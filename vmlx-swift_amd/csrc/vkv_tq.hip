@@ -16,14 +16,15 @@
 // and 256 (one Hadamard block) take the row kernels, which keep each vector
 // in the registers of eight lanes (tq_encode_rows / tq_decode_rows); other
 // dims take the tile kernels, which stage the tile in LDS.  The two matrix
-// products run as f32 fused multiply-add chains in index order (register
-// tiles of outputs, the matrix read from L2), the row sums in double; the
-// same orders are what the CPU restatement fixes, so the codes, signs,
-// norms and decoded values are bit-exact with it.  Contraction is off in
+// products run as f32 fused multiply-add chains in index order (on the f32
+// matrix cores in the row kernels), the row sums in double; the same orders
+// are what the CPU restatement fixes, so the codes, signs, norms and decoded
+// values are bit-exact with it.  Contraction is off in
 // this file: every other product and sum rounds as the reference writes it.
 #include <hip/hip_ext.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "vkv_device.h"
 #include "vkv_internal.h"
@@ -48,6 +49,28 @@ __device__ __forceinline__ uint16_t f16_of(float v) {
 __device__ __forceinline__ float round_dt(float v, int dt) {
   if (dt == kF16) return f16_to_f32(f16_of(v));
   if (dt == kBF16) return bf16_to_f32(f32_to_bf16(v));
+  return v;
+}
+
+// round_dt of a pair for a dtype known at compile time: bf16 by the packed
+// hardware conversion (round to nearest even, as f32_to_bf16).
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+template <int DT>
+__device__ __forceinline__ void round_pair(float& a, float& b) {
+  if constexpr (DT == kBF16) {
+    const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{a, b}, bf16x2_t));
+    a = __uint_as_float(w << 16);
+    b = __uint_as_float(w & 0xFFFF0000u);
+  } else if constexpr (DT == kF16) {
+    a = f16_to_f32(f16_of(a));
+    b = f16_to_f32(f16_of(b));
+  }
+}
+template <int DT>
+__device__ __forceinline__ float round_one(float v) {
+  float b = 0.0f;
+  round_pair<DT>(v, b);
   return v;
 }
 
@@ -113,72 +136,16 @@ __device__ void pack_tile(const uint8_t* vals, int64_t e0, int64_t e1, int64_t t
   }
 }
 
-// acc[r][j] = sum_i a[r][i] * M[i * D + j], an f32 fma chain in i order, for
-// the tile's rows, handed to f(r, j, acc) for rows below `rows`; the left
-// operand is read as floats, or (SGN) as +-1 from bytes.  DT = D (a power of
-// two dividing 256) keeps a register tile of kRows * D / 256 outputs per
-// thread; DT = 0 walks (row, j) pairs.  f must not write the operands.
-template <int DT, bool SGN, class F>
-__device__ void tile_matmul(const float* a, const uint8_t* sa, int rows, int D, const float* M,
-                            F&& f) {
-  const int tid = threadIdx.x;
-  if constexpr (DT > 0) {
-    // thread: 4 adjacent columns x RPT rows; a wave's lanes share rows in
-    // groups, so the row operand is an LDS broadcast read
-    constexpr int C = 4;
-    constexpr int GC = DT / C;             // column groups
-    constexpr int GR = kThreads / GC;      // row groups
-    constexpr int RPT = kRows / GR;        // rows per thread
-    const int j0 = (tid % GC) * C, rg = tid / GC;
-    float acc[RPT][C];
-#pragma unroll
-    for (int k = 0; k < RPT; ++k)
-#pragma unroll
-      for (int c = 0; c < C; ++c) acc[k][c] = 0.0f;
-#pragma unroll 2
-    for (int i0 = 0; i0 < DT; i0 += 4) {
-      float4 m[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) m[u] = *reinterpret_cast<const float4*>(M + (i0 + u) * DT + j0);
-#pragma unroll
-      for (int k = 0; k < RPT; ++k) {
-        const int r = rg * RPT + k;
-        float x[4];
-        if constexpr (SGN) {
-          const uint32_t w = *reinterpret_cast<const uint32_t*>(sa + r * DT + i0);
-#pragma unroll
-          for (int u = 0; u < 4; ++u) x[u] = ((w >> (8 * u)) & 0xffu) ? 1.0f : -1.0f;
-        } else {
-          const float4 v = *reinterpret_cast<const float4*>(a + r * DT + i0);
-          x[0] = v.x; x[1] = v.y; x[2] = v.z; x[3] = v.w;
-        }
-        // each output's chain stays in i order
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          acc[k][0] = fmaf(x[u], m[u].x, acc[k][0]);
-          acc[k][1] = fmaf(x[u], m[u].y, acc[k][1]);
-          acc[k][2] = fmaf(x[u], m[u].z, acc[k][2]);
-          acc[k][3] = fmaf(x[u], m[u].w, acc[k][3]);
-        }
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < RPT; ++k) {
-      const int r = rg * RPT + k;
-      if (r < rows)
-#pragma unroll
-        for (int c = 0; c < C; ++c) f(r, j0 + c, acc[k][c]);
-    }
-  } else {
-    for (int p = tid; p < rows * D; p += kThreads) {
-      const int r = p / D, j = p - r * D;
-      float acc = 0.0f;
-      for (int i = 0; i < D; ++i) {
-        const float x = SGN ? (sa[r * D + i] ? 1.0f : -1.0f) : a[r * D + i];
-        acc = fmaf(x, M[static_cast<int64_t>(i) * D + j], acc);
-      }
-      f(r, j, acc);
-    }
+// sum_i a[r][i] * M[i * D + j], an f32 fma chain in i order, for the tile's
+// rows below `rows`, handed to f(r, j, sum); a(r, i) reads the left operand.
+// f must not write the operands.
+template <class A, class F>
+__device__ void tile_matmul(A&& a, int rows, int D, const float* M, F&& f) {
+  for (int p = threadIdx.x; p < rows * D; p += kThreads) {
+    const int r = p / D, j = p - r * D;
+    float acc = 0.0f;
+    for (int i = 0; i < D; ++i) acc = fmaf(a(r, i), M[static_cast<int64_t>(i) * D + j], acc);
+    f(r, j, acc);
   }
   __syncthreads();
 }
@@ -212,10 +179,9 @@ __device__ void row_offsets(int64_t* off, int64_t r0, int nr, int H, int Tc, int
   }
 }
 
-template <int DT>
 __global__ void __launch_bounds__(kThreads) tq_encode_kernel(TqEncodeArgs a) {
   extern __shared__ float lds[];
-  const int D = DT > 0 ? DT : a.D;
+  const int D = a.D;
   float* y = lds;                                                   // [kRows][D] f32
   uint8_t* codes = reinterpret_cast<uint8_t*>(y + kRows * D);       // [kRows][D]
   uint8_t* sg = codes + kRows * D;                                  // [kRows][D]
@@ -283,8 +249,8 @@ __global__ void __launch_bounds__(kThreads) tq_encode_kernel(TqEncodeArgs a) {
         if (part == 0 && r < nr) a.res_norms[r0 + r] = f16_of(sqrtf(static_cast<float>(s)));
       }
       // 6. projection through S (S^T as the right operand), signs p >= 0
-      tile_matmul<DT, false>(y, nullptr, nr, D, a.St,
-                             [&](int r, int j, float v) { sg[r * D + j] = v >= 0.0f; });
+      tile_matmul([&](int r, int i) { return y[r * D + i]; }, nr, D, a.St,
+                  [&](int r, int j, float v) { sg[r * D + j] = v >= 0.0f; });
     }
     // 7. pack codes and signs into the flat words
     const int64_t e0 = r0 * D, e1 = (r0 + nr) * D;
@@ -311,10 +277,9 @@ __device__ void unpack_tile(const uint32_t* words, int64_t e0, int64_t e1, int b
   }
 }
 
-template <int DT>
 __global__ void __launch_bounds__(kThreads) tq_decode_kernel(TqDecodeArgs a) {
   extern __shared__ float lds[];
-  const int D = DT > 0 ? DT : a.D;
+  const int D = a.D;
   float* z = lds;                                                   // [kRows][D]
   uint8_t* codes = reinterpret_cast<uint8_t*>(z + kRows * D);       // [kRows][D]
   uint8_t* sg = codes + kRows * D;                                  // [kRows][D]
@@ -343,9 +308,8 @@ __global__ void __launch_bounds__(kThreads) tq_decode_kernel(TqDecodeArgs a) {
       for (int e = nr * D + tid; e < kRows * D; e += kThreads) sg[e] = 0;
       __syncthreads();
       // z += (sqrt(pi/2) / d * |r|) * (signs . S)
-      tile_matmul<DT, true>(nullptr, sg, nr, D, a.S, [&](int r, int j, float v) {
-        z[r * D + j] = z[r * D + j] + cr[r] * v;
-      });
+      tile_matmul([&](int r, int i) { return sg[r * D + i] ? 1.0f : -1.0f; }, nr, D, a.S,
+                  [&](int r, int j, float v) { z[r * D + j] = z[r * D + j] + cr[r] * v; });
     }
     hadamard_tile(z, kRows, D, a.blocks);
     for (int e = tid; e < nr * D; e += kThreads) {
@@ -371,8 +335,16 @@ __global__ void __launch_bounds__(kThreads) tq_decode_kernel(TqDecodeArgs a) {
 // formed by the same operation on the same operands as in the tile kernels
 // above (the norms' double sums take their terms in another order; a sum of
 // at most 256 f32 terms is exact in double unless they span more than 29
-// binades, so its f32 rounding is the same).  LDS keeps only the bytes to
-// pack or unpack and, for keys, the projection's operand rows.
+// binades, so its f32 rounding is the same).  LDS keeps only the code bytes
+// to pack or unpack and, for keys, the projection's operand rows.
+//
+// Bound: at 128 dims the f32 matrix product takes ~55 us of 251 904 keys
+// (4.1 GMAC; [8, 8, 3936] of a compressed layer), the vector work (norm,
+// division, rotation, codes) ~65; the two overlap little, all waves of a CU
+// being in step, and giving waves different priorities by slot did not part
+// them (129 / 133 us).  Measured there: encode keys 197 -> 127 us (vector FMA
+// chains and true divisions before), decode keys 189 -> 125; values, without
+// a projection, 81 -> 61 and 53 -> 54.
 
 // The value of lane (lane ^ M) for M in {1, 2, 4}: the partner inside an
 // aligned group of eight lanes.
@@ -537,42 +509,123 @@ __device__ void unpack_rows(const uint32_t* words, int64_t r0, int nr, int D, in
   }
 }
 
-// The tile's QJL sign bits as +-1.0f (the projection's left operand): one
-// thread per word, D a multiple of 32 so words never cross a tile.
-__device__ void unpack_signs_rows(const uint32_t* words, int64_t r0, int nr, int D, float* out) {
-  const int64_t w0 = r0 * (D / 32);
-  const int nw = nr * (D / 32);
-  for (int lw = threadIdx.x; lw < nw; lw += kThreads) {
-    const uint32_t word = words[w0 + lw];
-    float4* o4 = reinterpret_cast<float4*>(out + lw * 32);
+// acc(r, j) = sum_i a(r, i) M(i, j) of a tile of 32 rows, on f32 matrix
+// cores: v_mfma_f32_16x16x4_f32 adds its four products in index order with a
+// fused multiply-add each (checked bit for bit against fmaf chains, normal
+// and denormal), so a chain of D / 4 of them is the f32 chain in i order that
+// the codec fixes, at twice the rate of unpacked vector FMAs and beside them.
+// Wave w takes columns [w D / 4, (w + 1) D / 4): CT tiles of 16 columns x 2 of
+// 16 rows.  A operand of step s: lane (r, g) holds a(r, 4 s + g); B: M(4 s +
+// g, j0 + r); acc[rt][ct][i]: row 16 rt + 4 g + i, column j0 + 16 ct + r.
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+template <int D>
+struct RowsMatrix {
+  static constexpr int CT = D / 64, S = D / 4;
+  // M's operands stay in registers up to 128 dims (64 of them); at 256 they
+  // are read per step
+  static constexpr bool kHeld = D <= 128;
+  float b[kHeld ? CT : 1][kHeld ? S : 1];
+  const float* base;
+  __device__ __forceinline__ void load(const float* M) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    base = M + (lane >> 4) * D + w * (D / 4) + (lane & 15);
+    if constexpr (kHeld) {
 #pragma unroll
-    for (int k = 0; k < 8; ++k)
-      o4[k] = make_float4((word >> (4 * k)) & 1u ? 1.0f : -1.0f,
-                          (word >> (4 * k + 1)) & 1u ? 1.0f : -1.0f,
-                          (word >> (4 * k + 2)) & 1u ? 1.0f : -1.0f,
-                          (word >> (4 * k + 3)) & 1u ? 1.0f : -1.0f);
+      for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+        for (int s = 0; s < S; ++s) b[ct][s] = base[4 * s * D + 16 * ct];
+    }
   }
+  // a4(rt, s4): the four A operands of steps 4 s4 .. + 3 of row tile rt
+  template <class A>
+  __device__ __forceinline__ void run(A&& a4, f32x4_t (&acc)[2][CT]) const {
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) acc[rt][ct] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    auto quad = [&](int s4) __attribute__((always_inline)) {
+      f32x4_t x[2] = {a4(0, s4), a4(1, s4)};
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) {
+          float m;
+          if constexpr (kHeld) m = b[ct][4 * s4 + u];
+          else m = base[4 * (4 * s4 + u) * D + 16 * ct];
+#pragma unroll
+          for (int rt = 0; rt < 2; ++rt)
+            acc[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[rt][u], m, acc[rt][ct], 0, 0, 0);
+        }
+    };
+    if constexpr (kHeld) {
+#pragma unroll
+      for (int s4 = 0; s4 < S / 4; ++s4) quad(s4);
+    } else {
+#pragma unroll 2
+      for (int s4 = 0; s4 < S / 4; ++s4) quad(s4);
+    }
+  }
+};
+
+// x[k] / den rounded to DT, for the run of a vector: by the correctly rounded
+// reciprocal and two correction steps, as the quantizer divides
+// (affine_quantize8), where no step can lose bits: a divisor in [2^-60,
+// 2^20] whose mantissa is not all ones, values that are zero or at least
+// 2^-100 (quotients of 2^-120 and more: none is denormal, and every
+// remainder is a multiple of 2^-147); a wave that holds others divides.  The
+// sign of a zero is lost, which no later step sees.
+template <int DT, int E>
+__device__ __forceinline__ void unit_run(float (&x)[E], float den) {
+  uint32_t least = ~0u;
+#pragma unroll
+  for (int k = 0; k < E; ++k) least = min(least, (__float_as_uint(x[k]) & 0x7fffffffu) - 1u);
+  const bool fast = den >= 0x1p-60f && den <= 0x1p20f && least >= __float_as_uint(0x1p-100f) - 1u &&
+                    (__float_as_uint(den) & 0x7fffffu) != 0x7fffffu;
+  if (__builtin_amdgcn_ballot_w64(!fast) == 0) {
+    const float inv = 1.0f / den;
+#pragma unroll
+    for (int k = 0; k < E; ++k) {
+      float q = x[k] * inv;
+      q = fmaf(fmaf(-q, den, x[k]), inv, q);
+      x[k] = fmaf(fmaf(-q, den, x[k]), inv, q);
+    }
+  } else {
+#pragma unroll
+    for (int k = 0; k < E; ++k) x[k] = x[k] / den;
+  }
+#pragma unroll
+  for (int k = 0; k < E; k += 2) round_pair<DT>(x[k], x[k + 1]);
 }
 
+// Waves a SIMD: three hide a tile's barriers under the others' matrix and
+// vector work where the held matrix (64 registers at 128 dims) leaves room.
 template <int D, bool KEYS>
-__global__ void __launch_bounds__(kThreads) tq_encode_rows(TqEncodeArgs a) {
-  constexpr int E = D / 8;
+constexpr int tq_waves() {
+  return KEYS && D == 128 ? 3 : 1;
+}
+
+template <int D, bool KEYS, int DT>
+__global__ void __launch_bounds__(kThreads)
+    __attribute__((amdgpu_waves_per_eu(tq_waves<D, KEYS>()))) tq_encode_rows(TqEncodeArgs a) {
+  constexpr int E = D / 8, S = D / 4, CT = D / 64;
+  constexpr int kPitch = D + 4;  // floats of a residual row: rows start 4 banks apart
   extern __shared__ float lds[];
-  uint8_t* codes = reinterpret_cast<uint8_t*>(lds);          // [kRows][D]
-  uint8_t* sg = codes + kRows * D;                            // keys: [kRows][D]
-  float* y = reinterpret_cast<float*>(sg + kRows * D);        // keys: [kRows][D] residuals
+  float* y = lds;                                             // keys: [kRows][kPitch] residuals
+  uint8_t* codes = reinterpret_cast<uint8_t*>(lds + (KEYS ? kRows * kPitch : 0));  // [kRows][D]
   __shared__ float cb_s[256], bnd_s[256];
   const int tid = threadIdx.x, r = tid >> 3, part = tid & 7;
+  const int lane = tid & 63, wave = tid >> 6;
   const int64_t rows = static_cast<int64_t>(a.B) * a.H * a.Tc;
-  constexpr bool keys = KEYS;
   const int nb = a.nc - 1;
   for (int i = tid; i < a.nc; i += kThreads) cb_s[i] = a.codebook[i];
   for (int i = tid; i < nb; i += kThreads) bnd_s[i] = a.bounds[i];
   float rs[E];
 #pragma unroll
   for (int k = 0; k < E; ++k) rs[k] = a.signs[part * E + k];
+  RowsMatrix<KEYS ? D : 64> mat;
+  if constexpr (KEYS) mat.load(a.St);
   const float scale = a.blocks.scale[0];
-  const float eps = round_dt(1e-8f, a.dtype);
+  const float eps = round_one<DT>(1e-8f);
   __syncthreads();
   for (int64_t r0 = static_cast<int64_t>(blockIdx.x) * kRows; r0 < rows;
        r0 += static_cast<int64_t>(gridDim.x) * kRows) {
@@ -581,8 +634,7 @@ __global__ void __launch_bounds__(kThreads) tq_encode_rows(TqEncodeArgs a) {
     // 1. the lane's run of the vector (rows past the end are zeros)
     float x[E];
     if (live) {
-      load_run<E>(a.x, a.dtype,
-                  row_offset(r0 + r, a.H, a.Tc, a.t0, a.sb, a.sh, a.st) + part * E, x);
+      load_run<E>(a.x, DT, row_offset(r0 + r, a.H, a.Tc, a.t0, a.sb, a.sh, a.st) + part * E, x);
     } else {
 #pragma unroll
       for (int k = 0; k < E; ++k) x[k] = 0.0f;
@@ -590,14 +642,20 @@ __global__ void __launch_bounds__(kThreads) tq_encode_rows(TqEncodeArgs a) {
     // 2. norm in T, the divisor T(norm + T(1e-8))
     double s = 0.0;
 #pragma unroll
-    for (int k = 0; k < E; ++k) s += static_cast<double>(round_dt(x[k] * x[k], a.dtype));
+    for (int k = 0; k < E; k += 2) {
+      float u = x[k] * x[k], v = x[k + 1] * x[k + 1];
+      round_pair<DT>(u, v);
+      s += static_cast<double>(u);
+      s += static_cast<double>(v);
+    }
     s = group8_sum_d(s);
-    const float nrm = round_dt(sqrtf(round_dt(static_cast<float>(s), a.dtype)), a.dtype);
-    const float den = round_dt(nrm + eps, a.dtype);
+    const float nrm = round_one<DT>(sqrtf(round_one<DT>(static_cast<float>(s))));
+    const float den = round_one<DT>(nrm + eps);
     if (part == 0 && live) a.vec_norms[r0 + r] = f16_of(nrm);
     // 3. unit vector in T, times the rotation signs, rotated
+    unit_run<DT>(x, den);
 #pragma unroll
-    for (int k = 0; k < E; ++k) x[k] = round_dt(x[k] / den, a.dtype) * rs[k];
+    for (int k = 0; k < E; ++k) x[k] = x[k] * rs[k];
     row_butterflies<E>(x, part, scale);
     // 4. codes; keys keep the residual y - level
     int idx[E];
@@ -616,7 +674,7 @@ __global__ void __launch_bounds__(kThreads) tq_encode_rows(TqEncodeArgs a) {
                 (static_cast<uint32_t>(idx[4 * u + 2]) << 16) |
                 (static_cast<uint32_t>(idx[4 * u + 3]) << 24);
     }
-    if constexpr (keys) {
+    if constexpr (KEYS) {
       // 5. residual norm: f32(sum f32(r_i^2)) -> sqrt -> f16
       double q = 0.0;
 #pragma unroll
@@ -627,60 +685,133 @@ __global__ void __launch_bounds__(kThreads) tq_encode_rows(TqEncodeArgs a) {
       }
       q = group8_sum_d(q);
       if (part == 0 && live) a.res_norms[r0 + r] = f16_of(sqrtf(static_cast<float>(q)));
-      float4* y4 = reinterpret_cast<float4*>(y + r * D + part * E);
+      // the residuals in the matrix product's operand order: element 4 s + g
+      // of a row at g S + s
 #pragma unroll
-      for (int u = 0; u < E / 4; ++u)
-        y4[u] = make_float4(x[4 * u], x[4 * u + 1], x[4 * u + 2], x[4 * u + 3]);
+      for (int g = 0; g < 4; ++g) {
+        float* yg = y + r * kPitch + g * S + part * (E / 4);
+        if constexpr (E == 8) {
+          *reinterpret_cast<float2*>(yg) = make_float2(x[g], x[4 + g]);
+        } else {
+#pragma unroll
+          for (int u = 0; u < E / 16; ++u)
+            reinterpret_cast<float4*>(yg)[u] =
+                make_float4(x[16 * u + g], x[16 * u + 4 + g], x[16 * u + 8 + g], x[16 * u + 12 + g]);
+        }
+      }
     }
     __syncthreads();
-    // 6. projection through S (S^T as the right operand), signs p >= 0
-    if constexpr (keys)
-      tile_matmul<D, false>(y, nullptr, nr, D, a.St,
-                            [&](int rr, int j, float v) { sg[rr * D + j] = v >= 0.0f; });
-    // 7. pack codes and signs into the flat words
-    const bool last = r0 + nr == rows;
-    pack_rows(codes, r0, nr, D, last, a.bits, a.indices);
-    if constexpr (keys) pack_rows(sg, r0, nr, D, last, 1, a.qjl);
+    // 6. projection through S (S^T as the right operand), signs p >= 0: a
+    // ballot holds 16 columns of 4 rows, lane row < 32 stores its row's words
+    if constexpr (KEYS) {
+      f32x4_t acc[2][CT];
+      const float* ya = y + (lane & 15) * kPitch + (lane >> 4) * S;
+      mat.run([&](int rt, int s4) __attribute__((always_inline)) {
+        return *reinterpret_cast<const f32x4_t*>(ya + 16 * rt * kPitch + 4 * s4);
+      }, acc);
+      uint32_t bits[CT];
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) {
+        bits[ct] = 0;
+#pragma unroll
+        for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const uint64_t bal = __builtin_amdgcn_ballot_w64(acc[rt][ct][i] >= 0.0f);
+            if ((lane >> 4) == rt && (lane & 3) == i)
+              bits[ct] = static_cast<uint32_t>(bal >> (16 * ((lane >> 2) & 3))) & 0xFFFFu;
+          }
+      }
+      if (lane < nr) {
+        uint16_t* q16 = reinterpret_cast<uint16_t*>(a.qjl) + (r0 + lane) * (D / 16) + wave * CT;
+        if constexpr (CT == 1) {
+          *q16 = static_cast<uint16_t>(bits[0]);
+        } else {
+#pragma unroll
+          for (int c = 0; c < CT; c += 2)
+            *reinterpret_cast<uint32_t*>(q16 + c) = bits[c] | bits[c + 1] << 16;
+        }
+      }
+    }
+    // 7. pack the codes into the flat words
+    pack_rows(codes, r0, nr, D, r0 + nr == rows, a.bits, a.indices);
     __syncthreads();
   }
 }
 
 template <int D, bool KEYS>
-__global__ void __launch_bounds__(kThreads) tq_decode_rows(TqDecodeArgs a) {
-  constexpr int E = D / 8;
+__global__ void __launch_bounds__(kThreads)
+    __attribute__((amdgpu_waves_per_eu(tq_waves<D, KEYS>()))) tq_decode_rows(TqDecodeArgs a) {
+  constexpr int E = D / 8, CT = D / 64;
+  constexpr int kPitch = D + 4;
   extern __shared__ float lds[];
-  uint8_t* codes = reinterpret_cast<uint8_t*>(lds);          // [kRows][D]
-  float* sgf = reinterpret_cast<float*>(codes + kRows * D);   // keys: [kRows][D] +-1
-  float* z = sgf + kRows * D;                                 // keys: [kRows][D]
+  float* z = lds;                                             // keys: [kRows][kPitch]
+  uint8_t* codes = reinterpret_cast<uint8_t*>(lds + (KEYS ? kRows * kPitch : 0));  // [kRows][D]
   __shared__ float cb_s[256], cr_s[kRows];
   const int tid = threadIdx.x, r = tid >> 3, part = tid & 7;
+  const int lane = tid & 63, wave = tid >> 6;
   const int64_t rows = static_cast<int64_t>(a.B) * a.H * a.Tc;
-  constexpr bool keys = KEYS;
   for (int i = tid; i < (1 << a.bits); i += kThreads) cb_s[i] = a.codebook[i];
   float rs[E];
 #pragma unroll
   for (int k = 0; k < E; ++k) rs[k] = a.signs[part * E + k];
+  RowsMatrix<KEYS ? D : 64> mat;
+  if constexpr (KEYS) mat.load(a.S);
   const float scale = a.blocks.scale[0];
   for (int64_t r0 = static_cast<int64_t>(blockIdx.x) * kRows; r0 < rows;
        r0 += static_cast<int64_t>(gridDim.x) * kRows) {
     const int nr = static_cast<int>(rows - r0 < kRows ? rows - r0 : kRows);
     const bool live = r < nr;
-    unpack_rows(a.indices, r0, nr, D, a.bits, codes);
-    if constexpr (keys) {
-      unpack_signs_rows(a.qjl, r0, nr, D, sgf);
+    // keys: the sign words of this lane's rows of the matrix product (rows
+    // past the end repeat the last)
+    constexpr int W = D / 32;
+    uint32_t sw[2][KEYS ? W : 1];
+    if constexpr (KEYS) {
+#pragma unroll
+      for (int rt = 0; rt < 2; ++rt) {
+        const int row = min(16 * rt + (lane & 15), nr - 1);
+#pragma unroll
+        for (int w = 0; w < W; ++w) sw[rt][w] = a.qjl[(r0 + row) * W + w];
+      }
       if (tid < nr) cr_s[tid] = a.qs * f16_to_f32(a.res_norms[r0 + tid]);
     }
+    unpack_rows(a.indices, r0, nr, D, a.bits, codes);
     const float vn = live ? f16_to_f32(a.vec_norms[r0 + r]) : 0.0f;
     __syncthreads();
     float x[E];
-    if constexpr (keys) {
+    if constexpr (KEYS) {
       // z = level + (sqrt(pi/2) / d * |r|) * (signs . S); fma(+-1, S, q) is
-      // the sum or difference the reference's sign product rounds.  The rows
-      // past the end read stale operands and are not kept.
-      tile_matmul<D, false>(sgf, nullptr, nr, D, a.S, [&](int rr, int j, float v) {
-        z[rr * D + j] = cb_s[codes[rr * D + j]] + cr_s[rr] * v;
-      });
-      const float4* z4 = reinterpret_cast<const float4*>(z + r * D + part * E);
+      // the sum or difference the reference's sign product rounds.  Operand
+      // 4 s + g of a row is +-1 by bit 4 s + g of its words.
+      f32x4_t acc[2][CT];
+#pragma unroll
+      for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+        for (int w = 0; w < W; ++w) sw[rt][w] = ~sw[rt][w] >> (lane >> 4);
+      mat.run([&](int rt, int s4) __attribute__((always_inline)) {
+        f32x4_t v;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int s = 4 * s4 + u;
+          v[u] = __uint_as_float((sw[rt][s / 8] << (31 - 4 * (s & 7)) & 0x80000000u) | 0x3F800000u);
+        }
+        return v;
+      }, acc);
+#pragma unroll
+      for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int rr = 16 * rt + 4 * (lane >> 4) + i;
+          // (rows past the end hold stale codes and are not kept)
+          const float cr = cr_s[rr];
+#pragma unroll
+          for (int ct = 0; ct < CT; ++ct) {
+            const int j = wave * (D / 4) + 16 * ct + (lane & 15);
+            z[rr * kPitch + j] = cb_s[codes[rr * D + j]] + cr * acc[rt][ct][i];
+          }
+        }
+      __syncthreads();
+      const float4* z4 = reinterpret_cast<const float4*>(z + r * kPitch + part * E);
 #pragma unroll
       for (int u = 0; u < E / 4; ++u) {
         const float4 v = live ? z4[u] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -751,6 +882,38 @@ __global__ void __launch_bounds__(256) cast4d_kernel(const void* src, int sdt, i
   }
 }
 
+// The exact tokens and the empty window of a unified buffer in one launch:
+// per (b, h) row (blockIdx.y) the sink tokens, the tail tokens (cast as
+// cast4d_kernel casts, a copy where the dtypes agree) and zeros, kExactTokens
+// a workgroup.  A compressed layer has 324 such tokens a row: five launches
+// of ~5 us before.
+constexpr int kExactTokens = 8;
+__global__ void __launch_bounds__(256) tq_exact_kernel(TqExactArgs a) {
+  const int64_t row = blockIdx.y;
+  const int64_t n = static_cast<int64_t>(a.n_sink) + a.n_tail + a.n_zero;
+  for (int e = threadIdx.x; e < kExactTokens * a.D; e += 256) {
+    const int u = e / a.D, d = e - u * a.D;
+    const int64_t t = static_cast<int64_t>(blockIdx.x) * kExactTokens + u;
+    if (t >= n) return;
+    const bool tail = t >= a.n_sink, zero = t >= static_cast<int64_t>(a.n_sink) + a.n_tail;
+    const int64_t k = t - (tail ? a.n_sink : 0);  // token of its source
+    const int64_t at = zero ? a.zero_at + (k - a.n_tail) : tail ? a.tail_at + k : t;
+    const int64_t o = row * a.row_elems + at * a.D + d;
+    const void* src = tail ? a.tail : a.sink;
+    const int sdt = tail ? a.tail_dtype : a.sink_dtype;
+    const int64_t s = (row * (tail ? a.n_tail : a.n_sink) + k) * a.D + d;
+    if (a.dtype == kF32) {
+      static_cast<float*>(a.out)[o] = zero ? 0.0f : load_f32(src, sdt, s);
+    } else {
+      uint16_t v = 0;
+      if (!zero)
+        v = sdt == a.dtype ? static_cast<const uint16_t*>(src)[s]
+            : a.dtype == kF16 ? f16_of(load_f32(src, sdt, s)) : f32_to_bf16(load_f32(src, sdt, s));
+      static_cast<uint16_t*>(a.out)[o] = v;
+    }
+  }
+}
+
 // Zeros over `rows` runs of `run` units of T, `pitch` units apart.
 template <class T>
 __global__ void __launch_bounds__(256) zero_runs_kernel(T* base, int64_t pitch, int64_t run,
@@ -763,9 +926,14 @@ __global__ void __launch_bounds__(256) zero_runs_kernel(T* base, int64_t pitch, 
   }
 }
 
-int grid_for(int64_t rows) {
+int grid_for(int64_t rows, int64_t most = 2048) {
   const int64_t t = (rows + kRows - 1) / kRows;
-  return static_cast<int>(t < 2048 ? (t > 0 ? t : 1) : 2048);
+  return static_cast<int>(t < most ? (t > 0 ? t : 1) : most);
+}
+// The workgroups of a row launch: with the matrix held in registers, those
+// that run at once (three a CU at 128 dims), so that each loads it once.
+int rows_grid(int64_t rows, int D, bool keys) {
+  return grid_for(rows, keys && D == 128 ? 768 : 2048);
 }
 
 // The row kernels take head dims 64, 128 and 256 (one Hadamard block) over
@@ -779,32 +947,45 @@ bool rows_kernel_fits(int D, const TqBlocks& bl, const void* base, int es, int64
 
 }  // namespace
 
+// Whether the launch of these arguments writes every word of the packed codes
+// (and signs) itself; otherwise words shared by tiles are OR-ed into zeros.
+static bool tq_rows_launch(const TqEncodeArgs& a) {
+  return rows_kernel_fits(a.D, a.blocks, a.x, a.dtype == kF32 ? 4 : 2, a.sb, a.sh, a.st);
+}
+bool tq_encode_needs_zero_codes(const TqEncodeArgs& a) {
+  const int vpw = 32 / a.bits;  // widths that divide a row: no word crosses a tile
+  return !(tq_rows_launch(a) && (vpw & 3) == 0 && a.D % vpw == 0);
+}
+bool tq_encode_needs_zero_signs(const TqEncodeArgs& a) { return !tq_rows_launch(a); }
+
 void launch_tq_encode(const TqEncodeArgs& a, hipStream_t st) {
   const int64_t rows = static_cast<int64_t>(a.B) * a.H * a.Tc;
   if (rows <= 0) return;
   VKV_CHECK(rows < (int64_t{1} << 31), "TurboQuant encodes fewer than 2^31 vectors per call");
   VKV_CHECK(a.D >= 2 && a.D <= 256, "TurboQuant head dims must be in [2, 256]");
   VKV_CHECK(a.bits >= 1 && a.bits <= 8, "TurboQuant index bits must be in [1, 8]");
-  const dim3 g(grid_for(rows)), b(kThreads);
+  const dim3 g(tq_rows_launch(a) ? rows_grid(rows, a.D, a.St != nullptr) : grid_for(rows)), b(kThreads);
   // the key launch (the QJL projection) is the one the timing aid records
   const TimedLaunch tl = a.St ? timing_prepare(kTimeTqEncode) : TimedLaunch{};
-  const int es = a.dtype == kF32 ? 4 : 2;
-  if (rows_kernel_fits(a.D, a.blocks, a.x, es, a.sb, a.sh, a.st)) {
-    const size_t lds = static_cast<size_t>(kRows) * a.D * (a.St ? 6 : 1);
-    switch (a.D) {
-      case 64: a.St ? hipExtLaunchKernelGGL((tq_encode_rows<64, true>), g, b, lds, st, tl.start, tl.stop, 0, a)
-              : hipExtLaunchKernelGGL((tq_encode_rows<64, false>), g, b, lds, st, tl.start, tl.stop, 0, a);
-      break;
-      case 128: a.St ? hipExtLaunchKernelGGL((tq_encode_rows<128, true>), g, b, lds, st, tl.start, tl.stop, 0, a)
-              : hipExtLaunchKernelGGL((tq_encode_rows<128, false>), g, b, lds, st, tl.start, tl.stop, 0, a);
-      break;
-      default: a.St ? hipExtLaunchKernelGGL((tq_encode_rows<256, true>), g, b, lds, st, tl.start, tl.stop, 0, a)
-              : hipExtLaunchKernelGGL((tq_encode_rows<256, false>), g, b, lds, st, tl.start, tl.stop, 0, a);
-      break;
-    }
+  if (tq_rows_launch(a)) {
+    const size_t lds = static_cast<size_t>(kRows) * (a.St ? 4 * (a.D + 4) + a.D : a.D);
+    auto run = [&](auto D_, auto K_, auto T_) {
+      hipExtLaunchKernelGGL((tq_encode_rows<decltype(D_)::value, decltype(K_)::value, decltype(T_)::value>),
+                            g, b, lds, st, tl.start, tl.stop, 0, a);
+    };
+    using std::integral_constant;
+    auto dims = [&](auto K_, auto T_) {
+      if (a.D == 64) run(integral_constant<int, 64>{}, K_, T_);
+      else if (a.D == 128) run(integral_constant<int, 128>{}, K_, T_);
+      else run(integral_constant<int, 256>{}, K_, T_);
+    };
+    auto kind = [&](auto T_) { a.St ? dims(std::true_type{}, T_) : dims(std::false_type{}, T_); };
+    if (a.dtype == kBF16) kind(integral_constant<int, kBF16>{});
+    else if (a.dtype == kF16) kind(integral_constant<int, kF16>{});
+    else kind(integral_constant<int, kF32>{});
   } else {
     const size_t lds = static_cast<size_t>(kRows) * a.D * (4 + 1 + 1);
-    hipExtLaunchKernelGGL(tq_encode_kernel<0>, g, b, lds, st, tl.start, tl.stop, 0, a);
+    hipExtLaunchKernelGGL(tq_encode_kernel, g, b, lds, st, tl.start, tl.stop, 0, a);
   }
   VKV_HIP(hipGetLastError());
   if (a.St) timing_commit(tl);
@@ -816,11 +997,11 @@ void launch_tq_decode(const TqDecodeArgs& a, hipStream_t st) {
   VKV_CHECK(rows < (int64_t{1} << 31), "TurboQuant decodes fewer than 2^31 vectors per call");
   VKV_CHECK(a.D >= 2 && a.D <= 256, "TurboQuant head dims must be in [2, 256]");
   VKV_CHECK(a.bits >= 1 && a.bits <= 8, "TurboQuant index bits must be in [1, 8]");
-  const dim3 g(grid_for(rows)), b(kThreads);
+  const bool fits = rows_kernel_fits(a.D, a.blocks, a.out, a.out_dtype == kF32 ? 4 : 2, a.osb, a.osh, a.ost);
+  const dim3 g(fits ? rows_grid(rows, a.D, a.S != nullptr) : grid_for(rows)), b(kThreads);
   const TimedLaunch tl = a.S ? timing_prepare(kTimeTqDecode) : TimedLaunch{};
-  const int es = a.out_dtype == kF32 ? 4 : 2;
-  if (rows_kernel_fits(a.D, a.blocks, a.out, es, a.osb, a.osh, a.ost)) {
-    const size_t lds = static_cast<size_t>(kRows) * a.D * (a.S ? 9 : 1);
+  if (fits) {
+    const size_t lds = static_cast<size_t>(kRows) * (a.S ? 4 * (a.D + 4) + a.D : a.D);
     switch (a.D) {
       case 64: a.S ? hipExtLaunchKernelGGL((tq_decode_rows<64, true>), g, b, lds, st, tl.start, tl.stop, 0, a)
               : hipExtLaunchKernelGGL((tq_decode_rows<64, false>), g, b, lds, st, tl.start, tl.stop, 0, a);
@@ -834,10 +1015,29 @@ void launch_tq_decode(const TqDecodeArgs& a, hipStream_t st) {
     }
   } else {
     const size_t lds = static_cast<size_t>(kRows) * a.D * (4 + 1 + 1);
-    hipExtLaunchKernelGGL(tq_decode_kernel<0>, g, b, lds, st, tl.start, tl.stop, 0, a);
+    hipExtLaunchKernelGGL(tq_decode_kernel, g, b, lds, st, tl.start, tl.stop, 0, a);
   }
   VKV_HIP(hipGetLastError());
   if (a.S) timing_commit(tl);
+}
+
+void launch_tq_exact(const TqExactArgs& a, int64_t bh, hipStream_t st) {
+  const int64_t n = static_cast<int64_t>(a.n_sink) + a.n_tail + a.n_zero;
+  if (n <= 0 || bh <= 0) return;
+  for (int64_t r0 = 0; r0 < bh; r0 += 65535) {
+    TqExactArgs b = a;
+    const int es = a.dtype == kF32 ? 4 : 2;
+    b.out = static_cast<uint8_t*>(a.out) + r0 * a.row_elems * es;
+    auto at = [&](const void* p, int dt, int64_t tokens) {
+      return p ? static_cast<const uint8_t*>(p) + r0 * tokens * a.D * (dt == kF32 ? 4 : 2) : nullptr;
+    };
+    b.sink = at(a.sink, a.sink_dtype, a.n_sink);
+    b.tail = at(a.tail, a.tail_dtype, a.n_tail);
+    const dim3 grid(static_cast<unsigned>((n + kExactTokens - 1) / kExactTokens),
+                    static_cast<unsigned>(std::min<int64_t>(65535, bh - r0)));
+    hipLaunchKernelGGL(tq_exact_kernel, grid, dim3(256), 0, st, b);
+    VKV_HIP(hipGetLastError());
+  }
 }
 
 void launch_zero_runs(void* base, int64_t pitch_bytes, int64_t run_bytes, int64_t rows,

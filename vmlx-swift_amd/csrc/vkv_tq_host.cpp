@@ -384,19 +384,31 @@ std::shared_ptr<TqEncoded> encode(const vkv_array& x, bool keys, int bits, int s
   const int64_t rows = B * H * mid, n = rows * D;
   e->indices.alloc(words_for(n, ib) * 4);
   e->vec_norms.alloc(rows * 2);
-  launch_fill_i32(static_cast<int32_t*>(e->indices.get()), words_for(n, ib), 0, st);
   if (keys) {
     e->qjl.alloc(words_for(n, 1) * 4);
     e->res_norms.alloc(rows * 2);
-    launch_fill_i32(static_cast<int32_t*>(e->qjl.get()), words_for(n, 1), 0, st);
   }
-  if (pre) {
-    e->sink = alloc_dense(B, H, pre, D, x.dtype, false, st);
-    copy_tokens(e->sink, 0, x, 0, pre, st);
-  }
-  if (tl) {
-    e->tail = alloc_dense(B, H, tl, D, x.dtype, false, st);
-    copy_tokens(e->tail, 0, x, T - tl, tl, st);
+  // the exact tokens, both ends in one launch
+  Copy4D ends[2];
+  auto end = [&](Dense4& d, int64_t t0, int64_t len) {
+    d = alloc_dense(B, H, len, D, x.dtype, false, st);
+    Copy4D c;
+    c.src = static_cast<const uint8_t*>(x.data) + t0 * x.strides[2] * elem_bytes(x.dtype);
+    c.dst = d.buf->get();
+    const int64_t nn[4] = {B, H, len, D}, dd[4] = {H * len * D, len * D, D, 1};
+    for (int i = 0; i < 4; i++) {
+      c.n[i] = nn[i];
+      c.s[i] = x.strides[i];
+      c.d[i] = dd[i];
+    }
+    return c;
+  };
+  if (pre) ends[0] = end(e->sink, 0, pre);
+  if (tl) ends[1] = end(e->tail, T - tl, tl);
+  if (pre && tl) launch_copy4d_pair(elem_bytes(x.dtype), ends[0], ends[1], st);
+  else if (pre || tl) {
+    const Copy4D& c = ends[pre ? 0 : 1];
+    launch_copy4d(elem_bytes(x.dtype), c.src, c.n, c.s, c.dst, c.d, st);
   }
   TqEncodeArgs a{};
   a.x = x.data;
@@ -420,17 +432,36 @@ std::shared_ptr<TqEncoded> encode(const vkv_array& x, bool keys, int bits, int s
   a.qjl = keys ? static_cast<uint32_t*>(e->qjl.get()) : nullptr;
   a.vec_norms = static_cast<uint16_t*>(e->vec_norms.get());
   a.res_norms = keys ? static_cast<uint16_t*>(e->res_norms.get()) : nullptr;
+  if (tq_encode_needs_zero_codes(a))
+    launch_fill_i32(static_cast<int32_t*>(e->indices.get()), words_for(n, ib), 0, st);
+  if (keys && tq_encode_needs_zero_signs(a))
+    launch_fill_i32(static_cast<int32_t*>(e->qjl.get()), words_for(n, 1), 0, st);
   launch_tq_encode(a, st);
   return e;
 }
 
 // TQEncoder.decodeKeys / decodeValues (TQEncoder.swift:214-255, :315-345)
-// into dst tokens [0, e.tokens()): sink, decoded middle, tail.  The state
-// is EncoderState(dim, keyBits: index_bits + 1 | valueBits, seed).
-void decode_into(const TqEncoded& e, const Dense4& dst, hipStream_t st) {
+// into dst tokens [0, e.tokens()): sink, decoded middle, tail, then `window`
+// zero tokens.  The state is EncoderState(dim, keyBits: index_bits + 1 |
+// valueBits, seed).
+void decode_into(const TqEncoded& e, const Dense4& dst, int64_t window, hipStream_t st) {
   const TqTables& tb = tables(static_cast<int>(e.D), e.index_bits, e.seed, e.keys);
   const int64_t pre = e.sink_count();
-  if (pre) cast_tokens(dst, 0, e.sink.view(pre), 0, pre, st);
+  TqExactArgs x{};
+  x.out = dst.buf->get();
+  x.row_elems = dst.cap * dst.D;
+  x.dtype = dst.dtype;
+  x.D = static_cast<int32_t>(dst.D);
+  x.sink = pre ? e.sink.buf->get() : nullptr;
+  x.sink_dtype = e.sink.dtype;
+  x.n_sink = static_cast<int32_t>(pre);
+  x.tail = e.tail_count() ? e.tail.buf->get() : nullptr;
+  x.tail_dtype = e.tail.dtype;
+  x.n_tail = static_cast<int32_t>(e.tail_count());
+  x.tail_at = static_cast<int32_t>(pre + e.Tc);
+  x.n_zero = static_cast<int32_t>(window);
+  x.zero_at = static_cast<int32_t>(e.tokens());
+  launch_tq_exact(x, e.B * e.H, st);
   TqDecodeArgs a{};
   a.indices = static_cast<const uint32_t*>(e.indices.get());
   a.qjl = e.keys ? static_cast<const uint32_t*>(e.qjl.get()) : nullptr;
@@ -453,8 +484,6 @@ void decode_into(const TqEncoded& e, const Dense4& dst, hipStream_t st) {
   a.osh = dst.cap * dst.D;
   a.ost = dst.D;
   launch_tq_decode(a, st);
-  const int64_t tl = e.tail_count();
-  if (tl) cast_tokens(dst, pre + e.Tc, e.tail.view(tl), 0, tl, st);
 }
 
 }  // namespace
@@ -515,10 +544,8 @@ void TurboQuantCache::seat(std::shared_ptr<TqEncoded> ek, std::shared_ptr<TqEnco
   const int64_t n = ek->tokens();
   Dense4 uk = alloc_dense(ek->B, ek->H, n + kWindowStep, ek->D, ek->decoded_dtype(), false, st);
   Dense4 uv = alloc_dense(ev->B, ev->H, n + kWindowStep, ev->D, ev->decoded_dtype(), false, st);
-  zero_token_range(uk, n, kWindowStep, st);
-  zero_token_range(uv, n, kWindowStep, st);
-  decode_into(*ek, uk, st);
-  decode_into(*ev, uv, st);
+  decode_into(*ek, uk, kWindowStep, st);
+  decode_into(*ev, uv, kWindowStep, st);
   reset();
   ck_ = std::move(ek);
   cv_ = std::move(ev);

@@ -17,12 +17,25 @@
 // CU) owns a block of 256 query rows of one (row of the batch, kv head) and
 // one key range; a query row is one (query head of the group, position),
 // position-major.  Wave w owns rows 32w .. 32w + 31.  Each 32-token key tile
-// takes two phases separated by workgroup barriers: a matrix phase (the
-// scores of the tile, the P.V of the tile before) and a softmax phase.
-// Waves 4..7 run one phase behind waves 0..3, so the two waves of a SIMD are
-// always in different phases: one wave's MFMAs overlap the other's softmax
-// (ping-pong), and the wave in its matrix phase issues at the higher
-// priority.  Per tile:
+// takes two phases: a matrix phase (the scores of the tile, the P.V of the
+// tile before) and a softmax phase.  Waves 4..7 run one phase behind waves
+// 0..3, so the two waves of a SIMD are in different phases: one wave's MFMAs
+// overlap the other's softmax (ping-pong), and the wave in its matrix phase
+// issues at the higher priority.  At 256 dims a workgroup barrier ends every
+// phase; up to 128 dims a wave reads the tile's V operands in the softmax
+// phase before, and one barrier a tile is enough (see the tile loop).
+//
+// Bound: the matrix rate the card sustains on non-zero data (1.85 PFLOP/s
+// dense bf16: 18 ns a 32x32x16 MFMA and SIMD) and the softmax's vector
+// instructions, which overlap it in part.  Measured (512-token chunk over
+// 4608 4-bit keys, 32 / 8 heads x 128: 24 MFMAs a tile and wave, 36 tiles):
+// 67 -> 60 us, of which 31 are the matrix cores', 9 the launch and the
+// prologue, 5 the 33 MB of partials; per tile 1.30 us, where the MFMAs alone
+// take 0.86 and the softmax alone 0.9.  No variant spills: with the masked
+// and the open softmax as two copies in the tail loop it did (24 to 60
+// registers), and a scratch reload waits for the tile loads in flight.
+//
+// Per tile:
 //   * K and V tiles (32 rows of D elements each) go HBM -> LDS with
 //     global_load_lds_dwordx4 two tiles ahead into four stages (each wave
 //     loads one 1 KB piece of each); the per-lane source offsets place each
@@ -93,6 +106,7 @@ struct PfCfg {
   static constexpr int kSlots = D / 8;              // 16-byte pieces per row
   static constexpr int kKLoads = kTileB / 1024;     // 1 KB loads of a K (or V) tile
   static constexpr int kLoads = 2 * kKLoads / kWaves;  // 1 KB loads per wave per tile
+  static constexpr bool kAhead = D <= 128;  // V operands read a phase ahead, one barrier a tile
   static_assert(D == 64 || D == 128 || D == 256, "head dims 64, 128, 256");
   static_assert(kLoads >= 1 && kLoads * kWaves == 2 * kKLoads, "loads split evenly");
 };
@@ -276,7 +290,7 @@ __global__ void __launch_bounds__(512) mask_pack_kernel(const AttnArgs a, int re
 // tiles some row of it sees, the wholly visible ones first (the order of the
 // keys does not matter to the online softmax), and each wave loads its rows'
 // words of a tile beside the tile.  Measured (512-token chunk on a 1024-token
-// window, 16/8 heads x 256, 1535 keys): 55 us and 4.7 us for the packing, where
+// window, 16/8 heads x 256, 1535 keys): 40 us and 4.3 us for the packing, where
 // the generic kernel took 1780 us.
 template <int DT, bool QSEM, int D, bool ARR>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
@@ -304,7 +318,7 @@ prefill_kernel(const AttnArgs a, int rep) {
   // heads each XCD serves one head, and that head's K/V, re-read by every
   // row block and part, stays in the XCD's L2
   const int L = a.L;
-  const int rblocks = static_cast<int>((static_cast<int64_t>(L) * rep + kRows - 1) / kRows);
+  const int rblocks = static_cast<int>((static_cast<uint32_t>(L) * rep + kRows - 1) / kRows);
   // parts of this launch: all, or a window part0 .. part0 + parts_run - 1
   const int prun = a.parts_run > 0 ? a.parts_run : a.n_parts;
   int id = blockIdx.x;
@@ -317,11 +331,13 @@ prefill_kernel(const AttnArgs a, int rep) {
   // keys of this row of the batch: its own length when the rows are ragged
   // (query l of a row of length T sees keys up to T - L + l when causal)
   const int64_t T = a.kv.seq_lens ? min<int64_t>(a.kv.seq_lens[b], a.kv.T) : a.kv.T;
-  const int64_t nrows = static_cast<int64_t>(L) * rep;  // query rows of (b, hk)
-  const int64_t row0 = static_cast<int64_t>(rblk) * kRows;
+  // query rows of (b, hk): below 2^30 (prefill_supported), so that the row
+  // arithmetic is 32-bit
+  const int nrows = L * rep;
+  const int row0 = rblk * kRows;
   // keys of this workgroup: the part's range, and for a causal mask the
   // range its last position can see
-  const int64_t rlast = min<int64_t>(nrows, row0 + kRows) - 1;
+  const int rlast = min(nrows, row0 + kRows) - 1;
   int64_t k_end = min<int64_t>(T, static_cast<int64_t>(part + 1) * a.part_tokens);
   // QSEM: a query that sees no key (a ragged row shorter than the chunk)
   // has every score at T's lowest value in the reference (where(mask, s,
@@ -342,12 +358,14 @@ prefill_kernel(const AttnArgs a, int rep) {
   // ---- this lane's query row and its queries: B operand of score step c
   // = dims 16c + 8 kg .. +8
   using E = Elem<DT>;
-  const int64_t qrow = row0 + 32 * rb + l32;
+  const int qrow = row0 + 32 * rb + l32;
+  const int qr = min(qrow, nrows - 1);  // (rows past the end repeat the last)
+  const int qpos = static_cast<uint32_t>(qr) / static_cast<uint32_t>(rep);
+  const int qhead = hk * rep + (qr - qpos * rep);
   bool none = false;   // ARR: the row sees no key at all (QSEM averages V then)
   uint32_t mrow_off = 0;  // ARR: byte offset of the row's mask words
   if constexpr (ARR) {
-    const int64_t qr = min<int64_t>(qrow, nrows - 1);
-    const int64_t mr = b * a.mw_b + (hk * rep + qr % rep) * a.mw_h + qr / rep;
+    const int64_t mr = b * a.mw_b + qhead * a.mw_h + qpos;
     mrow_off = static_cast<uint32_t>(4 * mr * a.mw_words);
     if constexpr (QSEM) {
       // (whole 32-bit words: the row's bytes are padded to 4)
@@ -394,12 +412,9 @@ prefill_kernel(const AttnArgs a, int rep) {
   int64_t kmax;  // last key the row may see
   u32x4_t qf[kChunks];
   {
-    const int64_t qr = min<int64_t>(qrow, nrows - 1);
-    const int64_t pos = qr / rep;
-    const int r = static_cast<int>(qr % rep);
-    kmax = a.mask_mode == 1 ? T - L + pos : T - 1;
+    kmax = a.mask_mode == 1 ? T - L + qpos : T - 1;
     const typename E::T* qp = static_cast<const typename E::T*>(a.q) + b * a.q_sb +
-                              static_cast<int64_t>(hk * rep + r) * a.q_sh + pos * a.q_sl + 8 * kg;
+                              static_cast<int64_t>(qhead) * a.q_sh + qpos * a.q_sl + 8 * kg;
 #pragma unroll
     for (int c = 0; c < kChunks; c++) qf[c] = *(const g_u32x4_t*)(qp + 16 * c);
   }
@@ -426,8 +441,7 @@ prefill_kernel(const AttnArgs a, int rep) {
   // zero value row, counted once per row (sdpa_vector.h:93-96): the running
   // max (log2 units) starts at it with sum 1
   if (!QSEM && a.sinks && part == 0) {
-    const int64_t qr = min<int64_t>(qrow, nrows - 1);
-    m_run = load_as<DT>(a.sinks, a.sinks_dtype, hk * rep + static_cast<int>(qr % rep)) * kLog2e;
+    m_run = load_as<DT>(a.sinks, a.sinks_dtype, qhead) * kLog2e;
     l_run = kg == 0 ? 1.f : 0.f;  // the two lane halves' sums are added at the end
   }
 #pragma unroll
@@ -506,55 +520,61 @@ prefill_kernel(const AttnArgs a, int rep) {
     // and, with PV, O^T += V^T P^T for the tile at LDS base vb (V rows).
     // Every LDS read is issued before the first MFMA, so the MFMAs run
     // back to back instead of each waiting for its operand's read.
-    auto matrix = [&](uint32_t kb, uint32_t vb, auto PV_) __attribute__((always_inline)) {
-      constexpr bool PV = decltype(PV_)::value;
-      u32x4_t kf[kChunks];
+    u32x4_t kf[kChunks], vf[kDBw][2];
+    auto read_k = [&](uint32_t kb) __attribute__((always_inline)) {
 #pragma unroll
       for (int c = 0; c < kChunks; c++)
         kf[c] = *lds_ptr<const u32x4_t>(kb + 16 * ((2 * c + kg) ^ kx));
-      u32x4_t vf[kDBw][2];
-      if constexpr (PV) {
+    };
+    auto read_v = [&](uint32_t vb) __attribute__((always_inline)) {
 #pragma unroll
-        for (int db = 0; db < kDBw; db++)
+      for (int db = 0; db < kDBw; db++)
 #pragma unroll
-          for (int ks = 0; ks < 2; ks++) {
-            // rows 16 ks + 8 hf + 4 (a4 / 2) + e (row & 3 = e): piece
-            // 4 gdb + vpc (gdb = the global dim block) at slot (4 gdb + vpc) ^ vswz(e)
-            const uint32_t slot = 16 * ((4 * (dh * kDBw + db) + vpc) ^ vx);
-            const uint32_t off0 = (16 * ks) * kRowB + slot;
-            const uint32_t off1 = (16 * ks + 8) * kRowB + slot;
-            const i16x4_t x0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(lds_ptr<i16x4_t>(vb + off0));
-            const i16x4_t x1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(lds_ptr<i16x4_t>(vb + off1));
-            const u32x2_t w0 = __builtin_bit_cast(u32x2_t, x0), w1 = __builtin_bit_cast(u32x2_t, x1);
-            vf[db][ks] = u32x4_t{w0[0], w0[1], w1[0], w1[1]};
-          }
-      }
+        for (int ks = 0; ks < 2; ks++) {
+          // rows 16 ks + 8 hf + 4 (a4 / 2) + e (row & 3 = e): piece
+          // 4 gdb + vpc (gdb = the global dim block) at slot (4 gdb + vpc) ^ vswz(e)
+          const uint32_t slot = 16 * ((4 * (dh * kDBw + db) + vpc) ^ vx);
+          const uint32_t off0 = (16 * ks) * kRowB + slot;
+          const uint32_t off1 = (16 * ks + 8) * kRowB + slot;
+          const i16x4_t x0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(lds_ptr<i16x4_t>(vb + off0));
+          const i16x4_t x1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(lds_ptr<i16x4_t>(vb + off1));
+          const u32x2_t w0 = __builtin_bit_cast(u32x2_t, x0), w1 = __builtin_bit_cast(u32x2_t, x1);
+          vf[db][ks] = u32x4_t{w0[0], w0[1], w1[0], w1[1]};
+        }
+    };
+    auto matrix = [&](uint32_t kb, uint32_t vb, auto PV_) __attribute__((always_inline)) {
+      constexpr bool PV = decltype(PV_)::value;
+      read_k(kb);
+      if constexpr (!Cfg::kAhead && PV) read_v(vb);
       x = f32x16_t{};
       if constexpr (PV) {
         // the score chain (8 dependent MFMAs) interleaved with the P.V
         // MFMAs (one chain per 32-dim block)
         constexpr int kPv = (HL ? 4 : 2) * kDBw;  // P.V MFMAs
+        auto pv = [&](auto J) __attribute__((always_inline)) {  // n-th P.V MFMA
+          constexpr int n = decltype(J)::value, db = n % kDBw, q = n / kDBw;
+          constexpr int ks = HL ? q / 2 : q;  // HL: ks hi, ks lo; else ks
+          if constexpr (HL && q % 2 == 1)
+            o[db] = mfma<DT>(vf[db][ks], pl[ks], o[db]);
+          else
+            o[db] = mfma<DT>(vf[db][ks], pb[ks], o[db]);
+        };
+        // operands read ahead: the first kFirst P.V MFMAs run while the key
+        // reads arrive
+        constexpr int kFirst = Cfg::kAhead ? kPv / 2 : 0, kRest = kPv - kFirst;
+        sfor<kFirst>(pv);
+        if constexpr (Cfg::kAhead) __builtin_amdgcn_sched_barrier(0);
         sfor<kChunks>([&](auto C) {
           constexpr int c = decltype(C)::value;
           x = mfma<DT>(kf[c], qf[c], x);
           // the P.V MFMAs spread evenly over the score steps
-          sfor<kPv>([&](auto J) {
-            constexpr int n = decltype(J)::value;  // n-th P.V MFMA
-            if constexpr (n >= c * kPv / kChunks && n < (c + 1) * kPv / kChunks) {
-              constexpr int db = n % kDBw;
-              constexpr int q = n / kDBw;  // HL: ks hi, ks lo; else ks
-              constexpr int ks = HL ? q / 2 : q;
-              if constexpr (HL && q % 2 == 1)
-                o[db] = mfma<DT>(vf[db][ks], pl[ks], o[db]);
-              else
-                o[db] = mfma<DT>(vf[db][ks], pb[ks], o[db]);
-            }
+          sfor<kRest>([&](auto J) {
+            constexpr int n = decltype(J)::value;
+            if constexpr (n >= c * kRest / kChunks && n < (c + 1) * kRest / kChunks)
+              pv(std::integral_constant<int, kFirst + n>{});
           });
         });
-        if constexpr (D <= 128) {
-          __builtin_amdgcn_sched_group_barrier(0x100, kChunks + 4 * kDBw, 0);  // LDS reads
-          __builtin_amdgcn_sched_group_barrier(0x008, kChunks + kPv, 0);       // MFMAs
-        } else {
+        if constexpr (!Cfg::kAhead) {
           // at 256 dims every read at once would not fit the registers:
           // eight rounds of reads, each followed by its share of MFMAs
           sfor<8>([&](auto) {
@@ -580,10 +600,10 @@ prefill_kernel(const AttnArgs a, int rep) {
       pin(x);
     };
     // softmax of the row over tile i's scores x: the running max and sum,
-    // the rescale of o, and the P operands.  EDGE: keys past the range or
-    // the causal limit of some row are masked
+    // the rescale of o, and the P operands.  EDGE and `masked`: keys past the
+    // range or the causal limit of some row are masked
     // (ARR: the mask words of the tile, in its stage)
-    auto softmax = [&](int i, auto EDGE_) __attribute__((always_inline)) {
+    auto softmax = [&](int i, bool masked, auto EDGE_) __attribute__((always_inline)) {
       constexpr bool EDGE = decltype(EDGE_)::value;
       const int64_t t0 = k_begin + static_cast<int64_t>(kTok) * i;
       if constexpr (QSEM) {
@@ -597,7 +617,9 @@ prefill_kernel(const AttnArgs a, int rep) {
           x[j + 1] = E::to_f32(static_cast<typename E::T>(w >> 16));
         }
       }
-      if constexpr (EDGE && ARR) {
+      if (EDGE && !masked) {
+        // a tile of the tail loop that every row sees whole
+      } else if constexpr (EDGE && ARR) {
         uint32_t w = mwords[i % kStages][wave][lane];
         if (QSEM && some_none) {
           // rows that see no key: equal scores (0) on the row's keys
@@ -670,55 +692,88 @@ prefill_kernel(const AttnArgs a, int rep) {
       pin(l_run);
     };
 
-    // ---- the tile loop, in two phases per tile separated by workgroup
-    // barriers: a matrix phase (loads of tile i + 2, scores of tile i,
-    // O += V P of tile i - 1) and a softmax phase (tile i).  Group 1 runs
-    // one phase behind group 0, so on each SIMD one wave's MFMAs overlap the
-    // other wave's softmax.  Tile i lives in stage i % 4: its K is read in
-    // the matrix phases of i, its V in those of i + 1 (the last read, by
-    // group 1, ends before the phase in which tile i + 4 is loaded over it).
-    // Tiles that every row sees whole run unrolled by the stage count, so
-    // every LDS address is a per-lane base plus an immediate offset; the
-    // rest (masked) run with the stage computed.
+    // ---- the tile loop, in two phases per tile: a matrix phase (scores of
+    // tile i, O += V P of tile i - 1) and a softmax phase (tile i).  Group 1
+    // runs one phase behind group 0, so on each SIMD one wave's MFMAs overlap
+    // the other wave's softmax.  Tile i lives in stage i % 4.
+    //   Two barriers a tile (256 dims): tile i's K is read in the matrix
+    // phases of i, its V in those of i + 1; the matrix phase of tile i + 1
+    // loads tile i + 3 (the last read of the stage, by group 1, ended at the
+    // barrier before).
+    //   One barrier a tile (up to 128): step i of group 0 is softmax i, matrix
+    // i + 1; of group 1 matrix i, softmax i; a barrier ends each step.  V of
+    // tile i is read into registers in softmax i, so step i reads K of tiles
+    // i and i + 1 and V of tile i: it may load tile i + 3 over tile i - 1, and
+    // tile i + 1 is whole when it begins (its loads were issued in step i - 2,
+    // and the barrier of step i - 1 waits for all loads but the newest
+    // tile's).
+    // The first tiles that every row sees whole run unrolled by the stage
+    // count, so every LDS address is a per-lane base plus an immediate offset;
+    // the rest run with the stage computed and mask what is to be masked (all
+    // tiles under an array mask at 256 dims, which has few).
     const uint32_t stage_b = 2 * kTileB;
+    constexpr bool kOne = Cfg::kAhead;
+    // tile that the matrix phase of tile 1 loads
+    const int lead = kOne ? 3 + grp : 3;
+    // the barrier after group g's phase, entering one of priority PRIO
+    auto phase_end = [&](int g, auto PRIO_) __attribute__((always_inline)) {
+      constexpr int PRIO = decltype(PRIO_)::value;
+      if (!kOne || grp == g) {
+        phase_barrier<PRIO, kLoads>();
+      } else {
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_setprio(PRIO);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    constexpr auto kToMatrix = std::integral_constant<int, 1>{};
+    constexpr auto kToSoftmax = std::integral_constant<int, 0>{};
     load_tile(0, 0);
     load_tile(1, 1);
     phase_barrier<1, kLoads>();
+    if constexpr (kOne) load_tile(2, 2);
     if (grp) phase_barrier<1, kLoads>();
-    load_tile(2, 2);
+    if (!kOne || grp) load_tile(lead - 1, lead - 1);
     matrix(ka, 0, std::false_type{});
-    phase_barrier<0, kLoads>();
+    phase_end(0, kToSoftmax);
+    auto ahead = [&](int s) __attribute__((always_inline)) {
+      if constexpr (Cfg::kAhead) {
+        read_v(va + s * stage_b);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
     // softmax of tile i, then the matrix phase of tile i + 1
     auto open_tile = [&](int i, auto S_) __attribute__((always_inline)) {
       constexpr int S = decltype(S_)::value;
-      softmax(i, std::false_type{});
-      phase_barrier<1, kLoads>();
-      load_tile(i + 3, (S + 3) % kStages);
+      ahead(S);
+      softmax(i, false, std::false_type{});
+      phase_end(1, kToMatrix);
+      load_tile(i + lead, (S + lead) % kStages);
       // past the last tile this scores the clamped copy of the last tile
       // (loaded and complete like any other): unused, but no branch
       matrix(ka + ((S + 1) % kStages) * stage_b, va + S * stage_b, std::true_type{});
-      phase_barrier<0, kLoads>();
+      phase_end(0, kToSoftmax);
     };
     int i = 0;
-    for (; i + kStages <= n_open; i += kStages) {
-      open_tile(i, std::integral_constant<int, 0>{});
-      open_tile(i + 1, std::integral_constant<int, 1>{});
-      open_tile(i + 2, std::integral_constant<int, 2>{});
-      open_tile(i + 3, std::integral_constant<int, 3>{});
+    if constexpr (!(ARR && D == 256)) {
+      for (; i + kStages <= n_open; i += kStages) {
+        open_tile(i, std::integral_constant<int, 0>{});
+        open_tile(i + 1, std::integral_constant<int, 1>{});
+        open_tile(i + 2, std::integral_constant<int, 2>{});
+        open_tile(i + 3, std::integral_constant<int, 3>{});
+      }
     }
     for (; i < ntiles; i++) {
       const int s = i % kStages;
-      if (i < n_open)
-        softmax(i, std::false_type{});
-      else
-        softmax(i, std::true_type{});
-      phase_barrier<1, kLoads>();
-      load_tile(i + 3, (s + 3) % kStages);
+      ahead(s);
+      softmax(i, i >= n_open, std::true_type{});
+      phase_end(1, kToMatrix);
+      load_tile(i + lead, (s + lead) % kStages);
       matrix(ka + ((s + 1) % kStages) * stage_b, va + s * stage_b, std::true_type{});
-      phase_barrier<0, kLoads>();
+      phase_end(0, kToSoftmax);
     }
     // group 0 has one barrier fewer: it meets group 1's last one here
-    if (!grp) phase_barrier<0, kLoads>();
+    if (!kOne && !grp) phase_barrier<0, kLoads>();
     tile_wait_all();  // the clamped loads issued past the end
   }
 
@@ -726,12 +781,10 @@ prefill_kernel(const AttnArgs a, int rep) {
   // 32 db + 8 (j / 4) + 4 kg + j % 4
   const float lt = l_run + __shfl_xor(l_run, 32);
   if (qrow >= nrows) return;
-  const int64_t pos = qrow / rep;
-  const int h = hk * rep + static_cast<int>(qrow % rep);
-  const int64_t grow = b * L + pos;  // row of the batch x L
+  const int64_t grow = b * L + qpos;  // row of the batch x L
   if (a.n_parts == 1) {
     const float inv = lt > 0.f ? 1.0f / lt : 0.f;
-    typename E::T* op = static_cast<typename E::T*>(a.out) + b * a.o_sb + h * a.o_sh + pos * a.o_sl;
+    typename E::T* op = static_cast<typename E::T*>(a.out) + b * a.o_sb + qhead * a.o_sh + qpos * a.o_sl;
 #pragma unroll
     for (int db = 0; db < kDBw; db++)
 #pragma unroll
@@ -744,7 +797,7 @@ prefill_kernel(const AttnArgs a, int rep) {
       }
   } else {
     // unnormalized partial; (max, sum) with the max in natural-log units
-    const int64_t base = (grow * a.Hq + h) * a.n_parts + part;
+    const int64_t base = (grow * a.Hq + qhead) * a.n_parts + part;
     float* wo = a.ws_o + base * D + 32 * dh * kDBw;
 #pragma unroll
     for (int db = 0; db < kDBw; db++)
@@ -763,6 +816,8 @@ bool prefill_supported(int dtype, int bits, const AttnArgs& a) {
   if (bits != 0 || a.kv.table || a.kv.qfmt) return false;
   if (dtype != kBF16 && dtype != kF16) return false;
   if (a.L < 2 || a.Dv != a.D || a.Hq % a.Hkv) return false;
+  // 32-bit query rows
+  if (static_cast<int64_t>(a.L) * (a.Hq / a.Hkv) >= (int64_t{1} << 30)) return false;
   if (a.D != 64 && a.D != 128 && a.D != 256) return false;
   // none, causal, or a bool array (additive arrays are the generic kernel's);
   // an array's scores are compared before the scale, so scale > 0, and its

@@ -350,7 +350,7 @@ def config1_measure(torch, vkv, steps, warmup):
         "decode_tokens_per_s": round(1e3 / step_ms, 1),
         "decode_kv_gbs": round(kv_bytes / (pass_ms * 1e-3) / 1e9, 1),
         "prefill_update_us": round(pre_ms * 1e3, 2),
-        "roofline": _roofline(kv_bytes / N, k_ms, "fdecode_kernel"),
+        "roofline": _roofline(kv_bytes / N, k_ms, "fdecode16_kernel"),
         "note": "2.1-2.4 MB per step: launch-latency bound, not bandwidth bound",
     }
 
@@ -471,7 +471,7 @@ def config4_measure(torch, vkv, steps, warmup):
         "window_layer_pct_hbm_peak": round(100 * win_bytes / (w_ms / n_win * 1e-3) / 1e9
                                            / HBM_PEAK_GBS, 2),
         "global_layer_us": round(g_ms * 1e3, 2),
-        "roofline_window": _roofline(win_bytes, wk_ms, "fdecode_kernel"),
+        "roofline_window": _roofline(win_bytes, wk_ms, "fdecode16_kernel"),
         "roofline_global": _roofline(glob_bytes, gk_ms, "qdecode_kernel"),
         "finite": finite,
     }

@@ -733,7 +733,7 @@ enum {
   VKV_OPTION_GENERIC_ATTENTION = 0,
   VKV_OPTION_DECODE_WAVES = 1,
   VKV_OPTION_MLA_SPLITS = 2,
-  VKV_OPTION_FDECODE_WAVES = 3, /* 0 = 2048: waves the float decode kernel aims for */
+  VKV_OPTION_FDECODE_WAVES = 3, /* waves the float decode kernel aims for; 0: 4096 (16-bit), 2048 (f32) */
   VKV_OPTION_GATHER_TOKENS = 4, /* 0 = a 256 MiB copy: key window of a gathered chunk */
   VKV_OPTION_REFERENCE_SOFTMAX = 5, /* quantized attention with the reference's arithmetic */
   VKV_OPTION_SEPARATE_TOKEN_WRITE = 6, /* the router's quantized decode token in its own launch */

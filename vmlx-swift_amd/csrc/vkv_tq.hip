@@ -338,8 +338,8 @@ __global__ void __launch_bounds__(kThreads) tq_decode_kernel(TqDecodeArgs a) {
 // binades, so its f32 rounding is the same).  LDS keeps only the code bytes
 // to pack or unpack and, for keys, the projection's operand rows.
 //
-// Bound: at 128 dims the f32 matrix product takes ~55 us of 251 904 keys
-// (4.1 GMAC; [8, 8, 3936] of a compressed layer), the vector work (norm,
+// Bound: at 128 dims the f32 matrix product takes ~54 us of 257 792 keys
+// (4.2 GMAC; [8, 8, 4028] of a compressed layer), the vector work (norm,
 // division, rotation, codes) ~65; the two overlap little, all waves of a CU
 // being in step, and giving waves different priorities by slot did not part
 // them (129 / 133 us).  Measured there: encode keys 197 -> 127 us (vector FMA
@@ -884,32 +884,56 @@ __global__ void __launch_bounds__(256) cast4d_kernel(const void* src, int sdt, i
 
 // The exact tokens and the empty window of a unified buffer in one launch:
 // per (b, h) row (blockIdx.y) the sink tokens, the tail tokens (cast as
-// cast4d_kernel casts, a copy where the dtypes agree) and zeros, kExactTokens
-// a workgroup.  A compressed layer has 324 such tokens a row: five launches
-// of ~5 us before.
-constexpr int kExactTokens = 8;
+// cast4d_kernel casts, a copy where the dtypes agree) and zeros, U dims a
+// thread (8 where rows are whole 16-byte units).  A compressed layer has 324
+// such tokens a row (64 rows x 128 to f32: 10.6 MB written): five launches of
+// ~5 us before; 9.0 us at one dim a thread, 5.5 at eight.
+template <int U>
 __global__ void __launch_bounds__(256) tq_exact_kernel(TqExactArgs a) {
+  const uint32_t per = static_cast<uint32_t>(a.D) / U, tokens = 256u / per;  // D <= 256
+  const uint32_t u = threadIdx.x / per, d = (threadIdx.x - u * per) * U;
+  const int64_t t = static_cast<int64_t>(blockIdx.x) * tokens + u;
+  if (u >= tokens || t >= static_cast<int64_t>(a.n_sink) + a.n_tail + a.n_zero) return;
   const int64_t row = blockIdx.y;
-  const int64_t n = static_cast<int64_t>(a.n_sink) + a.n_tail + a.n_zero;
-  for (int e = threadIdx.x; e < kExactTokens * a.D; e += 256) {
-    const int u = e / a.D, d = e - u * a.D;
-    const int64_t t = static_cast<int64_t>(blockIdx.x) * kExactTokens + u;
-    if (t >= n) return;
-    const bool tail = t >= a.n_sink, zero = t >= static_cast<int64_t>(a.n_sink) + a.n_tail;
-    const int64_t k = t - (tail ? a.n_sink : 0);  // token of its source
-    const int64_t at = zero ? a.zero_at + (k - a.n_tail) : tail ? a.tail_at + k : t;
-    const int64_t o = row * a.row_elems + at * a.D + d;
-    const void* src = tail ? a.tail : a.sink;
-    const int sdt = tail ? a.tail_dtype : a.sink_dtype;
-    const int64_t s = (row * (tail ? a.n_tail : a.n_sink) + k) * a.D + d;
-    if (a.dtype == kF32) {
-      static_cast<float*>(a.out)[o] = zero ? 0.0f : load_f32(src, sdt, s);
+  const bool tail = t >= a.n_sink, zero = t >= static_cast<int64_t>(a.n_sink) + a.n_tail;
+  const int64_t k = t - (tail ? a.n_sink : 0);  // token of its source
+  const int64_t at = zero ? a.zero_at + (k - a.n_tail) : tail ? a.tail_at + k : t;
+  const int64_t o = row * a.row_elems + at * a.D + d;
+  const void* src = tail ? a.tail : a.sink;
+  const int sdt = tail ? a.tail_dtype : a.sink_dtype;
+  const int64_t s = (row * (tail ? a.n_tail : a.n_sink) + k) * a.D + d;
+  if constexpr (U == 8) {
+    if (a.dtype != kF32 && (zero || sdt == a.dtype)) {
+      uint4 v = make_uint4(0u, 0u, 0u, 0u);
+      if (!zero) v = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(src) + s);
+      *reinterpret_cast<uint4*>(static_cast<uint16_t*>(a.out) + o) = v;
+      return;
+    }
+  }
+  float x[U];
+  if (zero) {
+#pragma unroll
+    for (int e = 0; e < U; ++e) x[e] = 0.0f;
+  } else if constexpr (U == 8) {
+    load_run<8>(src, sdt, s, x);
+  } else {
+    x[0] = load_f32(src, sdt, s);
+  }
+  if (a.dtype == kF32) {
+    float* q = static_cast<float*>(a.out) + o;
+    if constexpr (U == 8) {
+      reinterpret_cast<float4*>(q)[0] = make_float4(x[0], x[1], x[2], x[3]);
+      reinterpret_cast<float4*>(q)[1] = make_float4(x[4], x[5], x[6], x[7]);
     } else {
-      uint16_t v = 0;
-      if (!zero)
-        v = sdt == a.dtype ? static_cast<const uint16_t*>(src)[s]
-            : a.dtype == kF16 ? f16_of(load_f32(src, sdt, s)) : f32_to_bf16(load_f32(src, sdt, s));
-      static_cast<uint16_t*>(a.out)[o] = v;
+      *q = x[0];
+    }
+  } else {
+    uint16_t* q = static_cast<uint16_t*>(a.out) + o;
+    if (U == 1 && !zero && sdt == a.dtype) {
+      *q = static_cast<const uint16_t*>(src)[s];
+    } else {
+#pragma unroll
+      for (int e = 0; e < U; ++e) q[e] = a.dtype == kF16 ? f16_of(x[e]) : f32_to_bf16(x[e]);
     }
   }
 }
@@ -1024,6 +1048,11 @@ void launch_tq_decode(const TqDecodeArgs& a, hipStream_t st) {
 void launch_tq_exact(const TqExactArgs& a, int64_t bh, hipStream_t st) {
   const int64_t n = static_cast<int64_t>(a.n_sink) + a.n_tail + a.n_zero;
   if (n <= 0 || bh <= 0) return;
+  VKV_CHECK(a.D >= 1 && a.D <= 256, "TurboQuant head dims must be in [2, 256]");
+  // 16-byte units: every row of every array starts on one
+  auto aligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+  const bool wide = a.D % 8 == 0 && a.row_elems % 8 == 0 && aligned(a.out) && aligned(a.sink) && aligned(a.tail);
+  const int64_t tokens = 256 / (wide ? a.D / 8 : a.D);
   for (int64_t r0 = 0; r0 < bh; r0 += 65535) {
     TqExactArgs b = a;
     const int es = a.dtype == kF32 ? 4 : 2;
@@ -1033,9 +1062,12 @@ void launch_tq_exact(const TqExactArgs& a, int64_t bh, hipStream_t st) {
     };
     b.sink = at(a.sink, a.sink_dtype, a.n_sink);
     b.tail = at(a.tail, a.tail_dtype, a.n_tail);
-    const dim3 grid(static_cast<unsigned>((n + kExactTokens - 1) / kExactTokens),
+    const dim3 grid(static_cast<unsigned>((n + tokens - 1) / tokens),
                     static_cast<unsigned>(std::min<int64_t>(65535, bh - r0)));
-    hipLaunchKernelGGL(tq_exact_kernel, grid, dim3(256), 0, st, b);
+    if (wide)
+      hipLaunchKernelGGL(tq_exact_kernel<8>, grid, dim3(256), 0, st, b);
+    else
+      hipLaunchKernelGGL(tq_exact_kernel<1>, grid, dim3(256), 0, st, b);
     VKV_HIP(hipGetLastError());
   }
 }

@@ -72,3 +72,31 @@ def test_release_empties_the_pool():
     before = torch.cuda.mem_get_info()[0]
     vkv.workspace_release()
     assert torch.cuda.mem_get_info()[0] >= before + 2 * x.numel() * 2
+
+
+def test_release_while_another_thread_converts():
+    bad, done = [], threading.Event()
+
+    def convert():
+        st = torch.cuda.Stream()
+        with torch.cuda.stream(st):
+            for i in range(60):
+                x = torch.full((2, 4, 512 + 64 * (i % 3), 128), float(i + 1), device="cuda").half()
+                c = vkv.KVCacheSimple()
+                c.update(x, x)
+                back = c.to_quantized(64, 8).to_unquantized().state[0]
+                st.synchronize()
+                if not bool((back == i + 1).all()):
+                    bad.append(i)
+        done.set()
+
+    def release():
+        st = torch.cuda.Stream()
+        with torch.cuda.stream(st):
+            while not done.wait(0.002):
+                vkv.workspace_release()
+
+    ts = [threading.Thread(target=f) for f in (convert, release)]
+    [t.start() for t in ts]
+    [t.join(60) for t in ts]
+    assert not bad and done.is_set()

@@ -3,6 +3,7 @@
 // observable behaviour it reproduces (paths relative to the vmlx-swift
 // checkout); device work is issued through the launchers in
 // vkv_kernels.hip.
+#include "vkv_blockpool.h"
 #include "vkv_host.h"
 
 #include <string.h>
@@ -1911,7 +1912,7 @@ void timing_read(int kind, double* total_ms, int* count) {
 // ------------------------------------------------------------ workspace
 
 namespace {
-// DevPool.  Converting a cache or rotating one past its window replaces
+// DevPool (bookkeeping: vkv_blockpool.h).  Converting a cache or rotating one past its window replaces
 // buffers on every call, and a hipMalloc with the hipFree that follows costs
 // 20-100 us a buffer and waits for the device each time (8 x 4096 tokens of 8
 // heads x 128 to 4 bits and the state: 495 us a call with them, 133
@@ -1921,45 +1922,38 @@ namespace {
 // (it then costs little), else for several generations of blocks at a time: an
 // allocation that only waiting blocks would fit takes new memory (60 us) while
 // fewer than kFenceFits of them and less than kFenceBytes in all wait, then
-// waits for the device once and has all of them.  At most kPoolBytes and kPoolBlocks are kept on a device,
-// the oldest going back by hipFree; memory the device runs out of, and
-// vkv_workspace_release, empty the pool.  A call whose stream is being
+// waits for the device once and has all of them.  At most kPoolBytes and
+// kPoolBlocks are kept on a device, the oldest going back by hipFree; a buffer
+// the device has no memory for, and vkv_workspace_release, empty the pool.  A call whose stream is being
 // captured, or that names no stream, allocates by hipMalloc (which a capture
 // refuses) and never takes a kept block.
 constexpr size_t kPoolBytes = size_t{1} << 30;
-constexpr size_t kBlockBytes = kPoolBytes / 2;      // larger blocks are not kept
 constexpr size_t kFenceBytes = size_t{256} << 20;
 constexpr size_t kPoolBlocks = 1024;
 constexpr int kFenceFits = 4;
-struct PoolBlock {
-  void* p;
-  size_t cap;
-  uint64_t age;
-};
-struct PoolDevice {
-  std::list<PoolBlock> ready, waiting;  // oldest first
-  size_t bytes = 0, waiting_bytes = 0;
-};
-std::mutex& pool_mutex() {
-  static auto* mu = new std::mutex();
-  return *mu;
-}
-PoolDevice& pool_device(int dev) {
-  static auto* m = new std::map<int, PoolDevice>();
-  return (*m)[dev];
-}
-// The smallest block of at least `bytes` and at most an eighth more, and how
-// many such there are.
-std::list<PoolBlock>::iterator pool_fit(std::list<PoolBlock>& l, size_t bytes, int* fits = nullptr) {
-  auto best = l.end();
-  int n = 0;
-  for (auto it = l.begin(); it != l.end(); ++it) {
-    if (it->cap < bytes || it->cap > bytes + bytes / 8 + 4096) continue;
-    n++;
-    if (best == l.end() || it->cap < best->cap) best = it;
+struct HipMem {
+  static bool alloc(void** p, size_t bytes, bool* full) {
+    const hipError_t e = hipMalloc(p, bytes);
+    *full = e == hipErrorOutOfMemory;
+    if (*full) (void)hipGetLastError();
+    else if (e != hipSuccess) throw Error(std::string("hipMalloc: ") + hipGetErrorString(e));
+    return !*full;
   }
-  if (fits) *fits = n;
-  return best;
+  static void release(void* p) { (void)hipFree(p); }
+  static bool wait() {
+    const bool done = hipDeviceSynchronize() == hipSuccess;
+    if (!done) (void)hipGetLastError();
+    return done;
+  }
+  static bool idle() {
+    const bool done = hipStreamQuery(t_call.stream) == hipSuccess;
+    if (!done) (void)hipGetLastError();
+    return done;
+  }
+};
+BlockPool<HipMem>& block_pool() {
+  static auto* pool = new BlockPool<HipMem>({kPoolBytes, kPoolBytes / 2, kPoolBlocks, kFenceFits, kFenceBytes});
+  return *pool;
 }
 bool call_is_captured() {
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -2005,94 +1999,25 @@ WsKey ws_key(hipStream_t st) {
 void* DevPool::take(size_t bytes, size_t* cap, int* dev) {
   VKV_HIP(hipGetDevice(dev));
   const size_t want = (bytes + 511) / 512 * 512;
-  *cap = want;
+  if (t_call.known && !call_is_captured())
+    if (void* p = block_pool().take(*dev, want, cap)) return p;
   void* p = nullptr;
-  if (t_call.known && !call_is_captured()) {
-    std::unique_lock<std::mutex> g(pool_mutex());
-    PoolDevice& d = pool_device(*dev);
-    auto from_ready = [&]() -> bool {
-      auto it = pool_fit(d.ready, want);
-      if (it == d.ready.end()) return false;
-      p = it->p;
-      *cap = it->cap;
-      d.bytes -= it->cap;
-      d.ready.erase(it);
-      return true;
-    };
-    if (from_ready()) return p;
-    auto idle = [] {
-      const bool done = hipStreamQuery(t_call.stream) == hipSuccess;
-      if (!done) (void)hipGetLastError();
-      return done;
-    };
-    int fits = 0;
-    pool_fit(d.waiting, want, &fits);
-    if (fits > 0 && (fits >= kFenceFits || d.waiting_bytes >= kFenceBytes || idle())) {
-      // blocks given back during the wait are not covered by it
-      std::list<PoolBlock> fenced;
-      fenced.swap(d.waiting);
-      const size_t n = d.waiting_bytes;
-      d.waiting_bytes = 0;
-      g.unlock();
-      const hipError_t e = hipDeviceSynchronize();
-      g.lock();
-      if (e == hipSuccess) {
-        d.ready.splice(d.ready.end(), fenced);
-        if (from_ready()) return p;
-      } else {
-        (void)hipGetLastError();  // (another thread captures): new memory below
-        d.waiting.splice(d.waiting.begin(), fenced);
-        d.waiting_bytes += n;
-      }
-    }
-  }
-  hipError_t e = hipMalloc(&p, want);
-  if (e == hipErrorOutOfMemory) {
-    (void)hipGetLastError();
-    flush();
-    e = hipMalloc(&p, want);
-  }
-  if (e != hipSuccess) throw Error(std::string("hipMalloc: ") + hipGetErrorString(e));
+  if (!block_pool().fresh(*dev, want, &p))
+    throw Error(std::string("hipMalloc: ") + hipGetErrorString(hipErrorOutOfMemory));
+  *cap = want;
   return p;
 }
 
 void DevPool::give(void* p, size_t cap, int dev) {
-  if (cap > kBlockBytes || call_is_captured()) {
+  if (call_is_captured())
     (void)hipFree(p);
-    return;
-  }
-  std::vector<void*> drop;
-  {
-    std::lock_guard<std::mutex> g(pool_mutex());
-    static uint64_t age = 0;
-    PoolDevice& d = pool_device(dev);
-    d.waiting.push_back({p, cap, age++});
-    d.waiting_bytes += cap;
-    d.bytes += cap;
-    while (d.bytes > kPoolBytes || d.ready.size() + d.waiting.size() > kPoolBlocks) {
-      const bool r = !d.ready.empty() && (d.waiting.empty() || d.ready.front().age < d.waiting.front().age);
-      auto& l = r ? d.ready : d.waiting;
-      drop.push_back(l.front().p);
-      d.bytes -= l.front().cap;
-      if (!r) d.waiting_bytes -= l.front().cap;
-      l.pop_front();
-    }
-  }
-  for (void* x : drop) (void)hipFree(x);
+  else
+    block_pool().give(p, cap, dev);
 }
 
 void DevPool::flush() {
   int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return;
-  std::list<PoolBlock> all;
-  {
-    std::lock_guard<std::mutex> g(pool_mutex());
-    PoolDevice& d = pool_device(dev);
-    all.splice(all.end(), d.ready);
-    all.splice(all.end(), d.waiting);
-    d.bytes = d.waiting_bytes = 0;
-  }
-  for (auto& b : all) (void)hipFree(b.p);
+  if (hipGetDevice(&dev) == hipSuccess) block_pool().flush(dev);
 }
 
 bool attention_scratch_ready(hipStream_t st, size_t floats, size_t counters) {

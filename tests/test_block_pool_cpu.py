@@ -1,6 +1,7 @@
 """The bookkeeping of the kept device blocks (csrc/vkv_blockpool.h) over a host
 allocator: counts, limits and lists while another thread waits for the device,
-refused waits, a full device, and threads that release while others allocate."""
+refused waits, a full device, and threads that release while others allocate;
+and the library's device allocations on a device that is nearly full."""
 import os
 import subprocess
 
@@ -24,4 +25,19 @@ def check(tmp_path_factory):
                                   "refused_wait", "limits", "full_device", "threads"])
 def test_block_pool(check, case):
     r = subprocess.run([check, case], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+def test_scratch_on_a_full_device(tmp_path):
+    """The library over a host allocator: where the device is full, a stream's
+    scratch gets the memory of the kept blocks."""
+    lib = os.path.join(ROOT, "vmlx-swift_amd")
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    exe = str(tmp_path / "device_memory_check")
+    # (exported: the library's HIP calls resolve to the program's functions)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-g", "-Wall", "-rdynamic", "-I", f"{rocm}/include",
+                    os.path.join(ROOT, "tests", "native", "device_memory_check.cpp"), "-o", exe,
+                    f"-L{lib}", "-l:libvkv.so", f"-Wl,-rpath,{lib}", f"-L{rocm}/lib", "-lamdhip64",
+                    f"-Wl,-rpath,{rocm}/lib"], check=True)
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr

@@ -75,20 +75,21 @@ def test_release_empties_the_pool():
 
 
 def test_release_while_another_thread_converts():
-    bad, done = [], threading.Event()
+    good, done = [], threading.Event()
 
     def convert():
         st = torch.cuda.Stream()
-        with torch.cuda.stream(st):
-            for i in range(60):
-                x = torch.full((2, 4, 512 + 64 * (i % 3), 128), float(i + 1), device="cuda").half()
-                c = vkv.KVCacheSimple()
-                c.update(x, x)
-                back = c.to_quantized(64, 8).to_unquantized().state[0]
-                st.synchronize()
-                if not bool((back == i + 1).all()):
-                    bad.append(i)
-        done.set()
+        try:
+            with torch.cuda.stream(st):
+                for i in range(60):
+                    x = torch.full((2, 4, 512 + 64 * (i % 3), 128), float(i + 1), device="cuda").half()
+                    c = vkv.KVCacheSimple()
+                    c.update(x, x)
+                    back = c.to_quantized(64, 8).to_unquantized().state[0]
+                    st.synchronize()
+                    good.append(bool((back == i + 1).all()))
+        finally:
+            done.set()
 
     def release():
         st = torch.cuda.Stream()
@@ -99,4 +100,4 @@ def test_release_while_another_thread_converts():
     ts = [threading.Thread(target=f) for f in (convert, release)]
     [t.start() for t in ts]
     [t.join(60) for t in ts]
-    assert not bad and done.is_set()
+    assert len(good) == 60 and all(good)

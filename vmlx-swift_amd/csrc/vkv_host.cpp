@@ -1924,7 +1924,8 @@ namespace {
 // fewer than kFenceFits of them and less than kFenceBytes in all wait, then
 // waits for the device once and has all of them.  At most kPoolBytes and
 // kPoolBlocks are kept on a device, the oldest going back by hipFree; a buffer
-// the device has no memory for, and vkv_workspace_release, empty the pool.  A call whose stream is being
+// (or a stream's scratch) that the device has no memory for, and
+// vkv_workspace_release, empty the pool.  A call whose stream is being
 // captured, or that names no stream, allocates by hipMalloc (which a capture
 // refuses) and never takes a kept block.
 constexpr size_t kPoolBytes = size_t{1} << 30;
@@ -2001,10 +2002,16 @@ void* DevPool::take(size_t bytes, size_t* cap, int* dev) {
   const size_t want = (bytes + 511) / 512 * 512;
   if (t_call.known && !call_is_captured())
     if (void* p = block_pool().take(*dev, want, cap)) return p;
-  void* p = nullptr;
-  if (!block_pool().fresh(*dev, want, &p))
-    throw Error(std::string("hipMalloc: ") + hipGetErrorString(hipErrorOutOfMemory));
   *cap = want;
+  return fresh(want);
+}
+
+void* DevPool::fresh(size_t bytes) {
+  int dev = 0;
+  VKV_HIP(hipGetDevice(&dev));
+  void* p = nullptr;
+  if (!block_pool().fresh(dev, bytes, &p))
+    throw Error(std::string("hipMalloc: ") + hipGetErrorString(hipErrorOutOfMemory));
   return p;
 }
 

@@ -33,9 +33,11 @@ struct CallScope {
 
 // Device blocks that objects gave back, kept for the next allocation of about
 // their size (vkv_host.cpp): take() and give() stand in for hipMalloc and
-// hipFree.
+// hipFree; fresh() is hipMalloc, where a device that is full gets the kept
+// blocks back first.  Every allocation of the library is one of the two.
 struct DevPool {
   static void* take(size_t bytes, size_t* cap, int* dev);
+  static void* fresh(size_t bytes);
   static void give(void* p, size_t cap, int dev);
   static void flush();  // frees every kept block of the current device
 };
@@ -70,7 +72,7 @@ class DevBuf {
   }
   void alloc(size_t bytes) {
     release();
-    if (bytes && direct_) VKV_HIP(hipMalloc(&p_, bytes));
+    if (bytes && direct_) p_ = DevPool::fresh(bytes);
     else if (bytes) p_ = DevPool::take(bytes, &cap_, &dev_);
     n_ = bytes;
   }

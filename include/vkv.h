@@ -700,9 +700,18 @@ int vkv_array_copy(const vkv_array *src, vkv_array *dst, void *stream);
  * buffer is kept, not freed, because a HIP graph captured earlier on that
  * stream still points at it, and growth during capture is refused (run the
  * call once before capturing).  vkv_workspace_release frees the stream's
- * workspace on the current device and every outgrown buffer (*bytes,
- * optional, receives the total); call it only when no captured graph that
- * used the stream will be replayed again. */
+ * workspace on the current device and every outgrown buffer; call it only
+ * when no captured graph that used the stream will be replayed again.
+ *
+ * Kept blocks.  Device blocks of dropped buffers (an updated, converted or
+ * freed cache, a freed pool) stay allocated for the library's next buffers:
+ * at most 1 GiB and 1024 blocks a device, blocks of up to 512 MiB, which the
+ * host program's own allocator cannot use meanwhile.  A block is used again
+ * only after the whole device has been waited for.  An allocation of the
+ * library that the device has no memory for gives them back and tries again;
+ * so does vkv_workspace_release, on any stream (one without a workspace too),
+ * for all kept blocks of the current device (safe beside other threads'
+ * calls on other streams).  *bytes (optional) receives the total of both. */
 int vkv_workspace_release(void *stream, int64_t *bytes);
 
 /* ------------------------------------------------------- dispatch options */

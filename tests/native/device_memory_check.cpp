@@ -50,6 +50,7 @@ struct DevPool {
 };
 float* attention_workspace(hipStream_t st, size_t floats);
 uint32_t* attention_counters(hipStream_t st, size_t n);
+size_t workspace_release(hipStream_t st);
 }  // namespace vkv
 
 #define CHECK(x)                                 \
@@ -79,6 +80,14 @@ int main() try {
   void* p = vkv::DevPool::take(60 * kMb - 512, &cap, &dev);
   vkv::DevPool::give(p, cap, dev);
   CHECK(vkv::attention_counters(nullptr, 50 * kMb / 4) && used() == 250 * kMb);
+  // a release counts the kept blocks beside the stream's scratch, with or
+  // without one
+  capacity = 400 * kMb;
+  keep();
+  CHECK(vkv::workspace_release(nullptr) == 378 * kMb && used() == 0);
+  keep();
+  CHECK(vkv::workspace_release(nullptr) == 128 * kMb && used() == 0);
+  CHECK(vkv::workspace_release(nullptr) == 0);
   std::printf("ok\n");
   return 0;
 } catch (const std::exception& e) {

@@ -2022,9 +2022,10 @@ void DevPool::give(void* p, size_t cap, int dev) {
     block_pool().give(p, cap, dev);
 }
 
-void DevPool::flush() {
+size_t DevPool::flush() {
   int dev = 0;
-  if (hipGetDevice(&dev) == hipSuccess) block_pool().flush(dev);
+  VKV_HIP(hipGetDevice(&dev));
+  return block_pool().flush(dev);
 }
 
 bool attention_scratch_ready(hipStream_t st, size_t floats, size_t counters) {
@@ -2074,11 +2075,11 @@ uint32_t* attention_counters(hipStream_t st, size_t n) {
 }
 
 size_t workspace_release(hipStream_t st) {
-  DevPool::flush();
+  size_t n = DevPool::flush();
   std::lock_guard<std::mutex> g(ws_mutex());
   auto it = ws_map().find(ws_key(st));
-  if (it == ws_map().end()) return 0;
-  size_t n = it->second.cur.size() + it->second.counters.size();
+  if (it == ws_map().end()) return n;
+  n += it->second.cur.size() + it->second.counters.size();
   for (auto& b : it->second.retired) n += b.size();
   ws_map().erase(it);  // hipFree waits for the device
   return n;

@@ -39,7 +39,7 @@ struct DevPool {
   static void* take(size_t bytes, size_t* cap, int* dev);
   static void* fresh(size_t bytes);
   static void give(void* p, size_t cap, int dev);
-  static void flush();  // frees every kept block of the current device
+  static size_t flush();  // frees every kept block of the current device, returns their bytes
 };
 
 // Owned device allocation.  A buffer can be dropped while work that reads it

@@ -377,8 +377,9 @@ def quantized_paged_attention(queries, view: PagedView, scale: float, mask=None,
 
 def workspace_release(stream=None) -> int:
     """Free the attention workspace of a stream, outgrown buffers included
-    (only once no captured graph that used the stream is replayed again);
-    returns the bytes released."""
+    (only once no captured graph that used the stream is replayed again), and
+    the current device's kept blocks of dropped buffers, whatever their
+    stream; returns the bytes of both."""
     n = C.c_int64()
     _chk(lib().vkv_workspace_release(stream_ptr(stream), C.byref(n)))
     return n.value

@@ -76,6 +76,14 @@ __device__ __forceinline__ float load_as(const void* p, int dt, int64_t i) {
   return dt == DT ? v : round_to<DT>(v);
 }
 
+// An attention sink as the running max that a row starts at (with sum 1): a
+// sink of -inf, or below the max of a row without one, starts there, so that
+// a first hidden score (-inf) less the max is -inf and not NaN; the first
+// visible key then scales the sum to 0.
+__device__ __forceinline__ float sink_start(float sink, float lowest) {
+  return sink < lowest ? lowest : sink;
+}
+
 // ---------------------------------------------------------------------------
 // Affine paged chunk format (block_size % 32 == 0, head_dim % 32 == 0).
 // One (block, kv head) chunk holds K codes, V codes, then the scale/bias

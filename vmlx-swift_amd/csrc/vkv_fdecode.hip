@@ -590,7 +590,7 @@ __global__ void __launch_bounds__(64 * kWaves16)
   // an attention sink is one more logit with a zero value row, counted once
   // per row: the running max starts at it with sum 1 (sdpa_vector.h:93-96)
   if (a.sinks && part == 0 && wv == 0 && mrow < nh) {
-    m_own = load_as<DT>(a.sinks, a.sinks_dtype, h0 + mrow);
+    m_own = sink_start(load_as<DT>(a.sinks, a.sinks_dtype, h0 + mrow), kLowest);
     l_own = kgrp == 0 ? 1.0f : 0.0f;
   }
   float o[REP][8];

@@ -840,7 +840,7 @@ __global__ void __launch_bounds__(256) attn_partial_kernel(AttnArgs a, int h_off
   // an attention sink (MLXFast semantics only) is one more logit with a
   // zero value row, counted once per row (sdpa_vector.h:93-96, :257-260)
   if (!QSEM && a.sinks && part == 0 && tid < REP) {
-    m_run = load_as<DT>(a.sinks, a.sinks_dtype, hk * rep_total + h_off + tid);
+    m_run = sink_start(load_as<DT>(a.sinks, a.sinks_dtype, hk * rep_total + h_off + tid), m_run);
     l_run = 1.0f;
   }
   __syncthreads();

@@ -441,7 +441,7 @@ prefill_kernel(const AttnArgs a, int rep) {
   // zero value row, counted once per row (sdpa_vector.h:93-96): the running
   // max (log2 units) starts at it with sum 1
   if (!QSEM && a.sinks && part == 0) {
-    m_run = load_as<DT>(a.sinks, a.sinks_dtype, qhead) * kLog2e;
+    m_run = sink_start(load_as<DT>(a.sinks, a.sinks_dtype, qhead) * kLog2e, m_run);
     l_run = kg == 0 ? 1.f : 0.f;  // the two lane halves' sums are added at the end
   }
 #pragma unroll

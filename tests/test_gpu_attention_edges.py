@@ -1,7 +1,8 @@
 """Attention sinks of -inf and of the type's lowest value (a logit that adds
 nothing) where the first keys a kernel takes are hidden: the running max has
 no finite value yet.  One-token decodes and prompt chunks, bool and additive
-masks, the float-decode, matrix-core and generic kernels, against the oracle."""
+masks, the float-decode, matrix-core and generic kernels, against the oracle.
+NaN keys in one-token decodes."""
 import numpy as np
 import pytest
 import torch
@@ -42,3 +43,21 @@ def test_sinks_that_add_nothing(additive, dtype, D, Hq, Hkv, L, T, generic, monk
     got = values(vkv.scaled_dot_product_attention(dev(q, dtype), dev(k, dtype), dev(v, dtype),
                                                   D ** -0.5, mask=mt, sinks=dev(sinks, dtype)), dtype)
     assert_within(got, ref, attn_tol(dtype, ref), "oracle")
+
+
+@pytest.mark.parametrize("dtype", [O.BF16, O.F16])
+@pytest.mark.parametrize("D,Hq,Hkv,T", [(256, 4, 2, 20), (128, 8, 2, 300), (64, 4, 4, 5000)])
+def test_a_nan_key_shows(dtype, D, Hq, Hkv, T):
+    """A NaN in one key makes its head's outputs NaN, not zeros, in launches
+    of one part and of several; the other heads stay as they are."""
+    rng = np.random.default_rng(D + T)
+    f = lambda a: O.to_f32(a, dtype)
+    q = rand_bits(rng, (1, Hq, 1, D), dtype)
+    k, v = (rand_bits(rng, (1, Hkv, T, D), dtype) for _ in range(2))
+    ref = O.sdpa(f(q), f(k), f(v), D ** -0.5, q_dtype=dtype)
+    kd = dev(k, dtype)
+    kd[0, 0, T // 2, 3] = float("nan")
+    got = values(vkv.scaled_dot_product_attention(dev(q, dtype), kd, dev(v, dtype), D ** -0.5), dtype)
+    rep = Hq // Hkv
+    assert np.isnan(got[:, :rep]).all()
+    assert_within(got[:, rep:], ref[:, rep:], attn_tol(dtype, ref[:, rep:]), "other heads")

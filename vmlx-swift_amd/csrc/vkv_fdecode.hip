@@ -731,9 +731,10 @@ __global__ void __launch_bounds__(64 * kWaves16)
       a1 = fmaf(f, mo_g[w][r][d + 1], a1);
     }
     if (a.n_parts == 1 || (merge_here && np == 1)) {
+      // (an empty row's sum is 0; a NaN one is NaN in the output)
       typename E::T* out = static_cast<typename E::T*>(a.out) + b * a.o_sb + h * a.o_sh + d;
-      out[0] = E::from_f32(den > 0.0f ? a0 / den : 0.0f);
-      out[1] = E::from_f32(den > 0.0f ? a1 / den : 0.0f);
+      out[0] = E::from_f32(den != 0.0f ? a0 / den : 0.0f);
+      out[1] = E::from_f32(den != 0.0f ? a1 / den : 0.0f);
     } else {
       const int64_t slot = (b * a.Hq + h) * a.n_parts + part;
       uint64_t* wo = reinterpret_cast<uint64_t*>(a.ws_o + slot * D + d);
@@ -791,8 +792,8 @@ __global__ void __launch_bounds__(64 * kWaves16)
       }
     }
     typename E::T* out = static_cast<typename E::T*>(a.out) + b * a.o_sb + h * a.o_sh + d;
-    out[0] = E::from_f32(den > 0.0f ? a0 / den : 0.0f);
-    out[1] = E::from_f32(den > 0.0f ? a1 / den : 0.0f);
+    out[0] = E::from_f32(den != 0.0f ? a0 / den : 0.0f);
+    out[1] = E::from_f32(den != 0.0f ? a1 / den : 0.0f);
   }
 }
 

@@ -176,11 +176,16 @@ void run_attention(int dtype, int bits, int group, bool qsem, AttnArgs& a, int64
     return;
   }
   // Quantized or paged K/V with a chunk of query tokens (uniform or ragged
-  // lengths): gather them to dense rows of the dtype (the dequantized values
-  // the reference's dequantize produces; a ragged row fills its own length),
-  // then the matrix-core multi-query kernel on the copy.  Fewer query tokens
-  // stay on the generic kernel, which keeps the dequantized values
-  // unrounded (fp32) as the quantized matmul of the oracle does.
+  // lengths): gather them to dense rows of the dtype (a ragged row fills its
+  // own length), then the matrix-core multi-query kernel on the copy.  A
+  // chunk of any mask attends quantized K/V dequantized and rounded to the
+  // dtype, as the reference's tiled quantized matmul reads them; fewer query
+  // tokens, and every call under the generic_attention option, stay on the
+  // generic kernel, which keeps the dequantized values in fp32 as the
+  // reference's vector kernels do.  Relative error against 64-bit attention of
+  // the rounded values 1.66e-3 in bf16 (f16 2.1e-4) here and 4.4e-3 to 4.5e-3
+  // (5.3e-4) on the generic kernel; against the unrounded values the other
+  // way round.
   if ((bits > 0 || a.kv.table) && a.L >= kGatherPrefillMinL && a.kv.T > 0 &&
       !option(VKV_OPTION_GENERIC_ATTENTION)) {
     AttnArgs d = a;
@@ -216,40 +221,40 @@ void run_attention(int dtype, int bits, int group, bool qsem, AttnArgs& a, int64
       const size_t floats = copy_floats + part_floats + prefill_mask_floats(d, batch);
       // (an array mask under a capture that may not allocate: the generic kernel)
       if (d.mask_mode != 2 || attention_scratch_ready(st, floats, 0)) {
-      float* ws = workspace(st, floats, noalloc);
-      uint8_t* kd = reinterpret_cast<uint8_t*>(ws);
-      uint8_t* vd = kd + wbytes;
-      const int64_t wph = wtok * a.D * es;  // copy bytes per (row, kv head)
-      d.kv.kc = Comp{kd, a.Hkv * wph, wph, a.D * es};
-      d.kv.vc = Comp{vd, a.Hkv * wph, wph, a.D * es};
-      if (d.n_parts > 1) {
-        d.ws_o = ws + copy_floats;
-        d.ws_ml = d.ws_o + per * a.Dv;
-      }
-      launch_prefill_mask(d, batch, ws + copy_floats + part_floats, st);
-      for (int p0 = 0; p0 < d.n_parts; p0 += ppw) {
-        GatherArgs g{};
-        g.kv = a.kv;
-        g.n_seqs = static_cast<int32_t>(batch);
-        g.H = a.Hkv;
-        g.t_begin = static_cast<int32_t>(static_cast<int64_t>(p0) * d.part_tokens);
-        // the copy's layout holds wtok tokens per (row, head); the gather
-        // fills each row's tokens of the window (fewer in the last one)
-        g.T = static_cast<int32_t>(wtok);
-        g.D = a.D;
-        g.bits = bits;
-        g.group = group;
-        g.dtype = dtype;
-        g.out = kd;
-        g.out_v = vd;
-        launch_gather(g, 0, st);
-        d.part0 = p0;
-        d.parts_run = std::min(ppw, d.n_parts - p0);
-        d.t_base = g.t_begin;
-        launch_prefill(dtype, qsem, d, batch, st, /*combine=*/false);
-      }
-      if (d.n_parts > 1) launch_attn_combine(dtype, d, rows, st);
-      return;
+        float* ws = workspace(st, floats, noalloc);
+        uint8_t* kd = reinterpret_cast<uint8_t*>(ws);
+        uint8_t* vd = kd + wbytes;
+        const int64_t wph = wtok * a.D * es;  // copy bytes per (row, kv head)
+        d.kv.kc = Comp{kd, a.Hkv * wph, wph, a.D * es};
+        d.kv.vc = Comp{vd, a.Hkv * wph, wph, a.D * es};
+        if (d.n_parts > 1) {
+          d.ws_o = ws + copy_floats;
+          d.ws_ml = d.ws_o + per * a.Dv;
+        }
+        launch_prefill_mask(d, batch, ws + copy_floats + part_floats, st);
+        for (int p0 = 0; p0 < d.n_parts; p0 += ppw) {
+          GatherArgs g{};
+          g.kv = a.kv;
+          g.n_seqs = static_cast<int32_t>(batch);
+          g.H = a.Hkv;
+          g.t_begin = static_cast<int32_t>(static_cast<int64_t>(p0) * d.part_tokens);
+          // the copy's layout holds wtok tokens per (row, head); the gather
+          // fills each row's tokens of the window (fewer in the last one)
+          g.T = static_cast<int32_t>(wtok);
+          g.D = a.D;
+          g.bits = bits;
+          g.group = group;
+          g.dtype = dtype;
+          g.out = kd;
+          g.out_v = vd;
+          launch_gather(g, 0, st);
+          d.part0 = p0;
+          d.parts_run = std::min(ppw, d.n_parts - p0);
+          d.t_base = g.t_begin;
+          launch_prefill(dtype, qsem, d, batch, st, /*combine=*/false);
+        }
+        if (d.n_parts > 1) launch_attn_combine(dtype, d, rows, st);
+        return;
       }
     }
   }

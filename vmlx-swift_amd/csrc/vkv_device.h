@@ -155,10 +155,6 @@ __device__ __forceinline__ float wave_max(float v, int width) {
   for (int o = width / 2; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, width));
   return v;
 }
-__device__ __forceinline__ float wave_min(float v, int width) {
-  for (int o = width / 2; o > 0; o >>= 1) v = fminf(v, __shfl_xor(v, o, width));
-  return v;
-}
 __device__ __forceinline__ float wave_sum(float v, int width) {
   for (int o = width / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, width);
   return v;

@@ -159,10 +159,10 @@ __device__ __forceinline__ void wave_lds_sync() {
 // come back through device-coherent loads; all 64 lanes take D / 64 dims of
 // a head each and issue every part's loads of the head together, one round
 // trip per head.
-template <int DT, int D, int REP>
+template <int D, int REP>
 __device__ __forceinline__ void fdecode_merge_rows(const AttnArgs& a, int64_t b, int h0, int nh,
                                                    int lane) {
-  using E = Elem<DT>;
+  using E = Elem<kF32>;
   constexpr int DPL = D / 64;  // dims per lane: 1, 2 or 4
   constexpr int kMaxP = 32;    // parts per round trip
   for (int r = 0; r < nh; r++) {
@@ -220,9 +220,9 @@ __device__ __forceinline__ void fdecode_merge_rows(const AttnArgs& a, int64_t b,
   }
 }
 
-template <int DT, int D, int REP>
+template <int D, int REP>
 __global__ void __launch_bounds__(64) fdecode_kernel(AttnArgs a, int rep_total) {
-  static_assert(DT == kF32, "16-bit K/V take fdecode16_kernel");
+  constexpr int DT = kF32;  // 16-bit K/V take fdecode16_kernel
   using E = Elem<DT>;
   constexpr int VEC = 16 / E::kBytes;  // elements per 16-byte load
   constexpr int KL = D / VEC;          // loads per key row
@@ -451,7 +451,7 @@ __global__ void __launch_bounds__(64) fdecode_kernel(AttnArgs a, int rep_total) 
   // the last part merges every part of the group's heads, then zeroes the
   // counter for the next launch
   if (lane == 0) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  fdecode_merge_rows<DT, D, REP>(a, b, h0, nh, lane);
+  fdecode_merge_rows<D, REP>(a, b, h0, nh, lane);
 }
 
 // ------------------------------------------------------ 16-bit K/V
@@ -809,7 +809,7 @@ void launch_r(const AttnArgs& a, int64_t rows, int rep, int n_hg, hipStream_t st
   const TimedLaunch tl = timing_prepare(kTimeFDecode);
   const dim3 grid(a.n_parts, a.Hkv * n_hg, static_cast<unsigned>(rows));
   if constexpr (DT == kF32) {
-    hipExtLaunchKernelGGL((fdecode_kernel<DT, D, R>), grid, dim3(64), 0, st, tl.start, tl.stop, 0, a,
+    hipExtLaunchKernelGGL((fdecode_kernel<D, R>), grid, dim3(64), 0, st, tl.start, tl.stop, 0, a,
                           rep);
   } else {
     auto run = [&](auto M_) {

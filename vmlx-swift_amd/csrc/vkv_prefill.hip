@@ -508,12 +508,13 @@ prefill_kernel(const AttnArgs a, int rep) {
     const int vpc = 2 * (a4 & 1) + (jj >> 1);  // piece within the 4-piece group
     const int vx = vswz<D>(e4);                // swizzle of rows 4 (a4 / 2) + e (+ 8 hf + 16 ks)
 
-    // HL: P carried as hi + lo (two operands of the dtype, ~16
-    // significant bits), so the weighted sum keeps fp32-like accuracy (on
-    // large value channels of quantized caches; under array masks, whose
-    // calls held the probabilities in fp32 on the generic kernel: error
-    // against 64 bits 1.7e-3 with it, 2.3e-3 with one bf16 operand);
-    // otherwise one operand
+    // HL: P carried as hi + lo (two operands of the dtype, ~16 significant
+    // bits in bf16), so the weighted sum keeps fp32-like accuracy (on large
+    // value channels of quantized caches; under array masks, whose calls held
+    // the probabilities in fp32 on the generic kernel: relative error against
+    // 64 bits 1.654e-3 to 1.663e-3 over chunks of 22-512 tokens in bf16, 2.07e-4
+    // in f16, the generic kernel's to five digits; 2.3e-3 with one bf16
+    // operand); otherwise one operand
     u32x4_t pb[2], pl[2];
     f32x16_t x;
     // the matrix phase: scores of the tile at LDS base kb (K rows) into x

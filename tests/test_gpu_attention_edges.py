@@ -2,7 +2,8 @@
 nothing) where the first keys a kernel takes are hidden: the running max has
 no finite value yet.  One-token decodes and prompt chunks, bool and additive
 masks, the float-decode, matrix-core and generic kernels, against the oracle.
-NaN keys in one-token decodes."""
+NaN keys in one-token decodes.  Short rows, whose heads are dealt to several
+workgroups, at the lines of that rule."""
 import numpy as np
 import pytest
 import torch
@@ -61,3 +62,41 @@ def test_a_nan_key_shows(dtype, D, Hq, Hkv, T):
     rep = Hq // Hkv
     assert np.isnan(got[:, :rep]).all()
     assert_within(got[:, rep:], ref[:, rep:], attn_tol(dtype, ref[:, rep:]), "other heads")
+
+
+@pytest.mark.parametrize("dtype,D", [(O.BF16, 128), (O.F16, 64), (O.BF16, 256)])
+@pytest.mark.parametrize("B,Hq,Hkv", [(1, 32, 8), (1, 24, 8), (2, 12, 1), (8, 16, 2), (5, 64, 8), (40, 8, 8)])
+def test_short_rows(B, Hq, Hkv, dtype, D):
+    """The edges of one part (32768 / D tokens), of the rows whose heads are
+    split (768 tokens) and of a wave's step, plain and masked."""
+    f = lambda a: O.to_f32(a, dtype)
+    for T in (1, 16, 17, 128, 129, 32768 // D, 32768 // D + 1, 768, 769):
+        rng = np.random.default_rng(B + Hq + D + T)
+        q = rand_bits(rng, (B, Hq, 1, D), dtype)
+        k, v = (rand_bits(rng, (B, Hkv, T, D), dtype) for _ in range(2))
+        m = rng.random((B, 1, 1, T)) < 0.7
+        for mask in (None, m):
+            ref = O.sdpa(f(q), f(k), f(v), D ** -0.5, mask=mask, q_dtype=dtype)
+            got = vkv.scaled_dot_product_attention(
+                dev(q, dtype), dev(k, dtype), dev(v, dtype), D ** -0.5,
+                mask=None if mask is None else torch.from_numpy(mask).cuda())
+            assert_within(values(got, dtype), ref, attn_tol(dtype, ref), f"T {T}")
+
+
+@pytest.mark.parametrize("Hq,Hkv,D", [(32, 8, 128), (64, 8, 128), (12, 1, 64), (16, 2, 256)])
+def test_a_step_writes_its_token_once_for_all_head_groups(Hq, Hkv, D):
+    """Decode steps through a cache: the token that the decode launch writes is
+    read by every head group of its kv head and is in the cache afterwards."""
+    torch.manual_seed(Hq + D)
+    T, c = 30, vkv.KVCacheSimple()
+    k, v = (torch.randn((2, Hkv, T + 4, D), device="cuda").bfloat16() for _ in range(2))
+    c.update(k[:, :, :T].contiguous(), v[:, :, :T].contiguous())
+    for t in range(T, T + 4):
+        q = torch.randn((2, Hq, 1, D), device="cuda").bfloat16()
+        out = vkv.attention_with_cache_update(q, k[:, :, t:t + 1].contiguous(),
+                                              v[:, :, t:t + 1].contiguous(), c, D ** -0.5)
+        n = lambda x: x.float().cpu().numpy()
+        ref = O.sdpa(n(q), n(k[:, :, :t + 1]), n(v[:, :, :t + 1]), D ** -0.5, q_dtype=O.BF16)
+        assert_within(n(out), ref, attn_tol(O.BF16, ref), f"step {t}")
+    for got, want in zip(c.state, (k, v)):
+        assert torch.equal(vkv.to_torch(got) if not torch.is_tensor(got) else got, want)

@@ -153,13 +153,16 @@ void run_attention(int dtype, int bits, int group, bool qsem, AttnArgs& a, int64
   }
   if (fdecode_supported(dtype, bits, qsem, a) && !option(VKV_OPTION_GENERIC_ATTENTION)) {
     const int waves = static_cast<int>(option(VKV_OPTION_FDECODE_WAVES));
-    a.n_parts = fdecode_parts(dtype, rows, a.Hq, a.Hkv, max_len, a.D, &a.part_tokens, waves);
+    const FdecodePlan plan = fdecode_plan(dtype, rows, a.Hq, a.Hkv, max_len, a.D, waves);
+    a.group_heads = plan.heads;
+    a.n_parts = plan.n_parts;
+    a.part_tokens = plan.part_tokens;
     const size_t per = static_cast<size_t>(rows) * a.Hq * a.n_parts;
-    const size_t counts = static_cast<size_t>(rows) * fdecode_counter_count(a.Hq, a.Hkv);
+    const size_t counts = static_cast<size_t>(rows) * fdecode_counter_count(a.Hq, a.Hkv, plan.heads);
     // merged inside the launch where that is the faster merge; the
     // no-allocation path has no counters
     const bool inside =
-        !noalloc && a.n_parts > 1 && fdecode_merge_here(dtype, a.n_parts, a.Dv, a.Hq, a.Hkv);
+        !noalloc && a.n_parts > 1 && fdecode_merge_here(dtype, a.n_parts, a.Dv, plan.heads);
     if (a.n_parts > 1 && dtype != VKV_F32 && !noalloc &&
         !attention_scratch_ready(st, per * (a.Dv + 2), counts)) {
       // a capture that may not allocate: one workgroup a row and head group,

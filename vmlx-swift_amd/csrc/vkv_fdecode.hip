@@ -460,6 +460,9 @@ constexpr int kWaves16 = 8;    // waves of a workgroup
 constexpr int kStep16 = 16;    // tokens of a wave's step
 constexpr float kTau = 8.0f;   // the running max lags a score by at most this
 constexpr float kLowest = -3.402823466e38f;
+constexpr int kCus = 256;            // compute units of the device
+constexpr int kOnePart = 32768;      // tokens x dims of a row that is one part
+constexpr int kShortRow = 768;       // tokens of a row whose heads may be split
 
 typedef __attribute__((address_space(4))) const int32_t c_i32_t;
 
@@ -797,9 +800,9 @@ __global__ void __launch_bounds__(64 * kWaves16)
   }
 }
 
-// Query heads a wave takes (its head group): all of a kv head's, up to 8,
-// so that each key row is read once for them.
-int fd_group_heads(int Hq, int Hkv) {
+// All of a kv head's query heads, up to 8, so that each key row is read once
+// for them; of the sizes 1, 2, 4 and 8 that the kernels are built for.
+int fd_most_heads(int Hq, int Hkv) {
   const int rep = Hq / Hkv;
   return rep <= 1 ? 1 : rep <= 2 ? 2 : rep <= 4 ? 4 : 8;
 }
@@ -826,8 +829,7 @@ void launch_r(const AttnArgs& a, int64_t rows, int rep, int n_hg, hipStream_t st
 
 template <int DT, int D>
 void launch_d(const AttnArgs& a, int64_t rows, hipStream_t st) {
-  const int rep = a.Hq / a.Hkv;
-  const int R = fd_group_heads(a.Hq, a.Hkv);
+  const int rep = a.Hq / a.Hkv, R = a.group_heads;
   const int n_hg = (rep + R - 1) / R;
   if (R == 1) launch_r<DT, D, 1>(a, rows, rep, n_hg, st);
   else if (R == 2) launch_r<DT, D, 2>(a, rows, rep, n_hg, st);
@@ -875,8 +877,9 @@ bool fdecode_supported(int dtype, int bits, bool qsem, const AttnArgs& a) {
          al(a.kv.vc.ptr, a.kv.vc.sb, a.kv.vc.sh, a.kv.vc.st);
 }
 
-int fdecode_parts(int dtype, int64_t rows, int Hq, int Hkv, int64_t T, int D, int32_t* part_tokens,
-                  int waves) {
+FdecodePlan fdecode_plan(int dtype, int64_t rows, int Hq, int Hkv, int64_t T, int D, int waves) {
+  FdecodePlan p;
+  p.heads = fd_most_heads(Hq, Hkv);
   int64_t parts, step;
   if (dtype == kF32) {
     // about `waves` (default 2048) one-wave workgroups
@@ -884,21 +887,49 @@ int fdecode_parts(int dtype, int64_t rows, int Hq, int Hkv, int64_t T, int D, in
     parts = (waves > 0 ? waves : 2048) / std::max<int64_t>(1, rows * Hkv);
     parts = std::min<int64_t>(parts, (T + step - 1) / step);
   } else {
-    // two workgroups a CU, each of at least one step a wave (8 x 6001 tokens:
-    // 256, 512, 1024, 2048 workgroups 39.3, 40.2, 44.7, 54.8 us; pages of 16
-    // rows to 4096 tokens 46.1, 47.5, 53.1, 60.7: a workgroup's fixed chain
-    // is ~5 us)
-    const int R = fd_group_heads(Hq, Hkv);
-    const int64_t groups = rows * Hkv * ((Hq / Hkv + R - 1) / R);
     step = kStep16;
-    parts = (waves > 0 ? waves / kWaves16 : 512) / std::max<int64_t>(1, groups);
-    parts = std::min<int64_t>(parts, (T + step * kWaves16 - 1) / (step * kWaves16));
+    constexpr int kRound = kStep16 * kWaves16;  // tokens of one step of every wave
+    auto groups = [&](int R) { return rows * Hkv * ((Hq / Hkv + R - 1) / R); };
+    if (waves > 0) {
+      parts = std::min<int64_t>(waves / kWaves16 / std::max<int64_t>(1, groups(p.heads)),
+                                (T + kRound - 1) / kRound);
+    } else {
+      // Rows up to 64 KB of keys are one part: the merge of parts through
+      // device memory costs ~2 us, more than a wave's second and third step
+      // (us of GPU a call in a graph, one part / parts of 128 tokens: 32/8
+      // heads x 128, 200 tokens 6.3 / 7.3, 300 6.7 / 7.4, 512 9.1 / 7.6; x 64,
+      // 512 tokens 6.9 / 6.9; 8 rows of 256 x 64 6.1 / 7.5).
+      const bool one = T * D <= kOnePart;
+      const int64_t most = one ? 1 : (T + kRound - 1) / kRound;
+      // Heads are dealt to more workgroups while that leaves the launch
+      // within a workgroup a CU: each then holds fewer accumulators and ends
+      // sooner, and the rows it reads again come from the L2 (64/8 heads x
+      // 128, in two or more heads a workgroup / the rule's: 100 tokens 7.3 / 4.5,
+      // 300 9.8 / 7.1, 512 9.9 / 7.6; 32/8 x 64, 100 tokens 5.2 / 3.9).  At
+      // 1500 tokens (32/8 x 64: 8.2 with four heads, 8.6 with two) and at 256
+      // dims (16/8 heads, 700 tokens 8.7 / 9.0) it does not pay.
+      if (T <= kShortRow && D <= 128)
+        for (int R = 1; R < p.heads; R *= 2)
+          if (groups(R) * most <= kCus) {
+            p.heads = R;
+            break;
+          }
+      // Two workgroups a CU, each of at least one step a wave: 1024 and 2048
+      // workgroups are slower, a workgroup's fixed chain being ~5 us.  256 are
+      // as fast or faster on long rows (us a call at 256, 512, 1024, 2048
+      // workgroups: 8 x 6001 tokens, 32/8 heads x 128, 35.8, 38.3, 43.4, 54.2; 8
+      // x 2000 of 64/8 heads 17.3, 23.6, 41.2, 41.2; pages of 16 rows to 4096
+      // tokens 39.3, 39.6, 44.4, 55.1); rows of very unequal length were not
+      // measured at 256.
+      parts = std::min<int64_t>(512 / std::max<int64_t>(1, groups(p.heads)), most);
+    }
   }
   parts = std::max<int64_t>(1, parts);
   int64_t pt = (T + parts - 1) / parts;
   pt = std::max<int64_t>(step, (pt + step - 1) / step * step);
-  *part_tokens = static_cast<int32_t>(pt);
-  return static_cast<int>(std::max<int64_t>(1, (T + pt - 1) / pt));
+  p.part_tokens = static_cast<int32_t>(pt);
+  p.n_parts = static_cast<int32_t>(std::max<int64_t>(1, (T + pt - 1) / pt));
+  return p;
 }
 
 void launch_fdecode(int dtype, const AttnArgs& a, int64_t rows, hipStream_t st) {
@@ -922,16 +953,15 @@ void launch_fdecode(int dtype, const AttnArgs& a, int64_t rows, hipStream_t st) 
   if (b.n_parts > 1 && !b.counters) launch_attn_combine(dtype, b, rows, st);
 }
 
-int fdecode_counter_count(int Hq, int Hkv) {
-  const int rep = Hq / Hkv, R = fd_group_heads(Hq, Hkv);
-  return Hkv * ((rep + R - 1) / R);
+int fdecode_counter_count(int Hq, int Hkv, int heads) {
+  return Hkv * ((Hq / Hkv + heads - 1) / heads);
 }
 
-bool fdecode_merge_here(int dtype, int n_parts, int Dv, int Hq, int Hkv) {
+bool fdecode_merge_here(int dtype, int n_parts, int Dv, int heads) {
   if (dtype != kF32) return true;  // the whole workgroup merges
   // partial floats the last part of a head group reads back
   constexpr int64_t kMaxMergeFloats = 12288;
-  return static_cast<int64_t>(n_parts) * Dv * fd_group_heads(Hq, Hkv) <= kMaxMergeFloats;
+  return static_cast<int64_t>(n_parts) * Dv * heads <= kMaxMergeFloats;
 }
 
 }  // namespace vkv

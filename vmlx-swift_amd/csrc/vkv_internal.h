@@ -122,6 +122,7 @@ struct AttnArgs {
   // group); non-null merges the split partials inside the decode launch
   // (the last part of a row merges, then zeroes its counter again)
   uint32_t* counters;
+  int32_t group_heads;  // float decode: query heads of a workgroup (1, 2, 4 or 8)
   // matrix-core prefill under a bool array mask: the mask as bits (row
   // b * mw_b + h * mw_h + l, mw_words words each), per (row, 256 keys) whether
   // any key is seen, and per (row block, 32-key tile) its class
@@ -226,13 +227,16 @@ void launch_prefill_mask(AttnArgs& a, int64_t batch, float* ws, hipStream_t st);
 // split (fdecode_waves > 0 overrides the waves aimed for), and the launch
 // (with the merge when a.n_parts > 1).
 bool fdecode_supported(int dtype, int bits, bool qsem, const AttnArgs& a);
-int fdecode_parts(int dtype, int64_t rows, int Hq, int Hkv, int64_t T, int D, int32_t* part_tokens,
-                  int waves);
+struct FdecodePlan {
+  int32_t heads;        // query heads of a workgroup (AttnArgs::group_heads)
+  int32_t n_parts, part_tokens;
+};
+FdecodePlan fdecode_plan(int dtype, int64_t rows, int Hq, int Hkv, int64_t T, int D, int waves);
 void launch_fdecode(int dtype, const AttnArgs& a, int64_t rows, hipStream_t st);
 // counters per batch row the float decode's in-launch merge uses, and
 // whether a launch merges inside or in attn_combine_kernel
-int fdecode_counter_count(int Hq, int Hkv);
-bool fdecode_merge_here(int dtype, int n_parts, int Dv, int Hq, int Hkv);
+int fdecode_counter_count(int Hq, int Hkv, int heads);
+bool fdecode_merge_here(int dtype, int n_parts, int Dv, int heads);
 // MFMA decode attention over paged affine bf16 KV (vkv_decode.hip).
 struct DecodeArgs {
   const uint16_t* q;         // [n_seqs][Hq][D] bf16 / f16

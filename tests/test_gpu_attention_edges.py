@@ -3,7 +3,8 @@ nothing) where the first keys a kernel takes are hidden: the running max has
 no finite value yet.  One-token decodes and prompt chunks, bool and additive
 masks, the float-decode, matrix-core and generic kernels, against the oracle.
 NaN keys in one-token decodes.  Short rows, whose heads are dealt to several
-workgroups, at the lines of that rule."""
+workgroups, and chunks of little work under a bool mask, at the lines of their
+rules."""
 import numpy as np
 import pytest
 import torch
@@ -100,3 +101,25 @@ def test_a_step_writes_its_token_once_for_all_head_groups(Hq, Hkv, D):
         assert_within(n(out), ref, attn_tol(O.BF16, ref), f"step {t}")
     for got, want in zip(c.state, (k, v)):
         assert torch.equal(vkv.to_torch(got) if not torch.is_tensor(got) else got, want)
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,L,T", [(8, 8, 128, 4, 1024), (16, 8, 256, 4, 1024),
+                                          (32, 8, 64, 2, 1024), (24, 8, 128, 3, 1024)])
+def test_little_masked_chunks_take_the_generic_kernel(Hq, Hkv, D, L, T, monkeypatch):
+    """The longest rows of chunks that the generic kernel takes, bit for bit;
+    with one key more they are packed, and agree with the oracle."""
+    rng = np.random.default_rng(D + L + T)
+    f = lambda a: O.to_f32(a, O.BF16)
+    for n in (T, T + 1):
+        q = rand_bits(rng, (1, Hq, L, D), O.BF16)
+        k, v = (rand_bits(rng, (1, Hkv, n, D), O.BF16) for _ in range(2))
+        m = rng.random((L, n)) < 0.6
+        run = lambda: values(vkv.scaled_dot_product_attention(
+            *(dev(x, O.BF16) for x in (q, k, v)), D ** -0.5, mask=torch.from_numpy(m).cuda()), O.BF16)
+        monkeypatch.setattr(OPTIONS, "generic_attention", 0)
+        got = run()
+        ref = O.sdpa(f(q), f(k), f(v), D ** -0.5, mask=m, q_dtype=O.BF16)
+        assert_within(got, ref, attn_tol(O.BF16, ref), f"T {n}")
+        monkeypatch.setattr(OPTIONS, "generic_attention", 1)
+        if n == T:
+            assert np.array_equal(got, run())

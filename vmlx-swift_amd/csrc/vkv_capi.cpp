@@ -77,6 +77,19 @@ int32_t choose_parts(int64_t rows_x_heads, int64_t max_len, int32_t* part_tokens
 }
 
 constexpr int kGatherPrefillMinL = 16;
+// Whether a chunk of rows = batch x L queries under a bool array mask, whose keys
+// would be split, is better done by the generic kernel than by the packing, the
+// parts and their merge: few (query, kv head, key) triples, each costing two
+// units for the row and one a query head, at most four heads, and no long chain
+// of keys (us of GPU a call, generic / packed; 8/8 heads x 128: 2 queries, 300
+// keys 12.0 / 16.6, 4, 1024 15.6 / 20.1, 8, 1024 22.6 / 20.2; 16/8 x 256: 4, 1024
+// 22.2 / 26.3, 16, 300 23.0 / 22.5; 32/8 x 128: 2, 1024 17.8 / 20.1, 8, 300 16.9 /
+// 17.5, 2, 1200 20.3 / 20.0, 2, 1900 24.9 / 19.9; 64/8 x 128: 2, 300 19.2 / 17.0).
+// One part of keys is always faster packed (32/8 x 128: 2, 64 13.4 / 9.5).
+bool little_masked_chunk(int64_t rows, int Hq, int Hkv, int64_t T) {
+  const int rep = Hq / Hkv;
+  return rep <= 4 && T <= 1024 && rows * Hkv * T * (2 + rep) <= 131072;
+}
 // Bytes of the K/V copy of one key window of a gathered chunk (the whole
 // context in one window up to this size).
 constexpr int64_t kGatherCopyBytes = int64_t{256} << 20;
@@ -269,7 +282,10 @@ void run_attention(int dtype, int bits, int group, bool qsem, AttnArgs& a, int64
     const size_t per = static_cast<size_t>(rows) * a.Hq * a.n_parts;
     const size_t part_floats = a.n_parts > 1 ? (per * (a.Dv + 2) + 63) / 64 * 64 : 0;
     const size_t mask_floats = prefill_mask_floats(a, batch);
-    if (a.mask_mode != 2 || attention_scratch_ready(st, part_floats + mask_floats, 0)) {
+    // (little work, or a captured stream without the scratch: the generic kernel)
+    const bool little =
+        a.mask_mode == 2 && a.n_parts > 1 && little_masked_chunk(rows, a.Hq, a.Hkv, a.kv.T);
+    if (a.mask_mode != 2 || (!little && attention_scratch_ready(st, part_floats + mask_floats, 0))) {
       if (part_floats + mask_floats) {
         float* ws = workspace(st, part_floats + mask_floats, noalloc);
         a.ws_o = ws;

@@ -4,7 +4,7 @@ no finite value yet.  One-token decodes and prompt chunks, bool and additive
 masks, the float-decode, matrix-core and generic kernels, against the oracle.
 NaN keys in one-token decodes.  Short rows, whose heads are dealt to several
 workgroups, and chunks of little work under a bool mask, at the lines of their
-rules."""
+rules.  The values that a masked chunk over a quantized cache attends."""
 import numpy as np
 import pytest
 import torch
@@ -123,3 +123,18 @@ def test_little_masked_chunks_take_the_generic_kernel(Hq, Hkv, D, L, T, monkeypa
         monkeypatch.setattr(OPTIONS, "generic_attention", 1)
         if n == T:
             assert np.array_equal(got, run())
+
+
+@pytest.mark.parametrize("bits,D", [(4, 128), (8, 64), (8, 256)])
+def test_masked_quantized_chunks_attend_what_causal_ones_do(bits, D):
+    """K and V dequantized and rounded to the dtype: the causal mask as an array
+    gives the causal mode's output (up to the order of the merge: one unit)."""
+    torch.manual_seed(bits + D)
+    B, Hq, Hkv, L, T = 2, 8, 4, 48, 300
+    q = torch.randn((B, Hq, L, D), device="cuda").bfloat16()
+    k, v = (vkv.quantized(torch.randn((B, Hkv, T, D), device="cuda").bfloat16(), 64, bits) for _ in range(2))
+    m = torch.ones((L, T), dtype=torch.bool, device="cuda").tril(T - L)
+    run = lambda mask: vkv.quantized_scaled_dot_product_attention(
+        q, k, v, D ** -0.5, mask=mask, group_size=64, bits=bits).float().cpu().numpy()
+    a, b = run(m), run("causal")
+    assert_within(a, b, 2.0 ** -8 * np.abs(b) + 1e-6, "causal")

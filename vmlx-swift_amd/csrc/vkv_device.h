@@ -174,8 +174,8 @@ __device__ __forceinline__ float wave_sum(float v, int width) {
 // The 8 divisions by one scale are products with its correctly rounded
 // reciprocal and two correction steps: the first makes the quotient
 // faithful, the second then correctly rounded (P. Markstein, IBM J. Res.
-// Dev. 34, 1990), so the codes are the division's (no difference in 2.2e9
-// random and near-tie cases).  The theorem leaves out a divisor whose
+// Dev. 34, 1990), so the codes are the division's (tests: random, tie and
+// near-tie operands on the CPU; hard groups bit for bit on the device).  The theorem leaves out a divisor whose
 // mantissa is all ones, and the steps a scale so large or small that they
 // could overflow or lose bits: a wave holding such a group divides.
 // round(q) of q >= 0 is trunc(q + pred(1/2)); the bounds are applied before

@@ -511,8 +511,8 @@ __device__ void unpack_rows(const uint32_t* words, int64_t r0, int nr, int D, in
 
 // acc(r, j) = sum_i a(r, i) M(i, j) of a tile of 32 rows, on f32 matrix
 // cores: v_mfma_f32_16x16x4_f32 adds its four products in index order with a
-// fused multiply-add each (checked bit for bit against fmaf chains, normal
-// and denormal), so a chain of D / 4 of them is the f32 chain in i order that
+// fused multiply-add each (the codec tests hold the signs and decoded values
+// to the CPU's fmaf chains bit for bit), so a chain of D / 4 of them is the f32 chain in i order that
 // the codec fixes, at twice the rate of unpacked vector FMAs and beside them.
 // Wave w takes columns [w D / 4, (w + 1) D / 4): CT tiles of 16 columns x 2 of
 // 16 rows.  A operand of step s: lane (r, g) holds a(r, 4 s + g); B: M(4 s +

@@ -532,8 +532,9 @@ __global__ void __launch_bounds__(64 * kWaves16)
     return nsteps > 0 ? table[page(t)] : 0;
   };
   u32x4_t kw[KS], vw[NV];
-  // non-temporal where one workgroup reads a row (at REP = 8 further head
-  // groups may): 8 x 6001 bf16 tokens 40.2 -> 37.6 us
+  // non-temporal where one workgroup reads a long row (at REP = 8 further head
+  // groups may; below, only those of short rows): 8 x 6001 bf16 tokens 40.2 ->
+  // 37.6 us
   constexpr int kNt = REP < 8 ? 2 : 0;
   // K (or V) rows of step i, as a buffer whose end is the last row's
   auto rows_of = [&](const uint8_t* base, const Comp& c, int st, int i, int blk) __attribute__((always_inline)) {
